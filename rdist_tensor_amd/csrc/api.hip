@@ -999,7 +999,10 @@ double als_fit_impl(ex_als* a) {
                f->sigma.as<double>(), R, d + 1, fpart);
     double h[2];
     d2h(st, h, d, sizeof(h));
-    return 1.0 - std::sqrt(h[0] + h[1]) / a->t->norm;
+    // |X - Xh|^2 by expansion: where the model reproduces X it is rounding
+    // noise of either sign, and a negative one counts as zero (NaN stays)
+    const double res2 = h[0] + h[1];
+    return 1.0 - std::sqrt(res2 < 0.0 ? 0.0 : res2) / a->t->norm;
 }
 
 // Keys of device sample tuples for `mode`, checked distinct (the sampled
@@ -1492,7 +1495,7 @@ int ex_sampler_create(ex_ctx* ctx, ex_factors* f, int kind, int precision, uint6
             }
             s->grams.ensure((size_t)N * R * R * 8);
             s->M.ensure((size_t)(N + 2) * R * R * 8);
-            s->lam.ensure((size_t)(N + 1) * R * 8);
+            s->lam.ensure((size_t)(N + 1) * R * 8 + kMaxModes * 4);   // eigenvalues, then a word per slot
             with_slack(s->eig, (size_t)N * s->ge.node_count * S * 8);
             if (precision == EX_MIXED) with_slack(s->eig32, (size_t)N * s->ge.node_count * tri_stride32(R) * 4);
             s->pinvp.ensure((size_t)tri_pad64(R) * 8);

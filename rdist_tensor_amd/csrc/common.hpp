@@ -194,6 +194,7 @@ void level_sums(hipStream_t s, const TreeGeom& g, int S, T* nodes);
 // the root node (packed upper, the Gram of the whole factor) as a full R x R FP64 matrix
 template <typename T>
 void unpack_root(hipStream_t s, const T* nodes, int R, double* G);
+// lam: (N + 1) R eigenvalues, then kMaxModes 32-bit words of scratch.
 void sts_compute_m(hipStream_t s, int N, int j, int R, const double* grams, double* M, double* lam);
 void eig_tree_build(hipStream_t s, int N, int j, int R, const double* M, const double* grams, double* eig_nodes);
 void eig_tree_build32(hipStream_t s, int N, int j, int R, const double* M, const double* grams, float* eig_nodes);

@@ -5,6 +5,7 @@
 // common.h:696-746 (parallel_dsymm, compute_DAGAT), distmat.hpp:85-151.
 #include "common.hpp"
 #include "jacobi_block.hpp"
+#include "wave_psd.hpp"
 #include "device.hpp"
 #include "dsymm.hpp"
 
@@ -118,112 +119,241 @@ __global__ __launch_bounds__(kJacobiThreads) void eigh_kernel(const double* __re
     if (threadIdx.x < R) lam[blockIdx.x * R + sh.j.rank[threadIdx.x]] = sh.A[tri_index(R, threadIdx.x, threadIdx.x)];
 }
 
-template <int NBL, int NV>
+// compute_pinv_square: eigenvalues at or below tol (relative: tol x the largest
+// diagonal entry) dropped.  Where the first wavefront's Gauss-Jordan inverse
+// shows that none is and that the matrix is well conditioned
+// (WavePsd::well_posed) it is the result: n pivots instead of the
+// eigendecomposition's eight sweeps of n - 1 rounds, and nearer the 64-bit value
+// (R = 32 Grams: 7e-16 against 8e-15 relative).  Otherwise the two-sided Jacobi.
+template <int NMAX, int NBL, int NV>
 __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __restrict__ Min, int R, double tol,
                                                         double* __restrict__ out, const int* __restrict__ only_if,
                                                         int relative) {
     if (only_if && *only_if == 0) return;   // the same for the whole block
-    __shared__ EighShared sh;
+    typedef WavePsd<NMAX> W;
+    __shared__ EighSharedT<NMAX> sh;
+    __shared__ double col[NMAX], tol_sh;
+    __shared__ int done;
     const int64_t R2 = (int64_t)R * R;
-    load_upper(Min + blockIdx.x * R2, R, sh.A);
-    if (relative) {
-        // tolerance relative to the largest diagonal entry (read before the
-        // rotations change the diagonal)
-        __shared__ double dmax;
-        __syncthreads();
+    const double* M = Min + blockIdx.x * R2;
+    if (threadIdx.x < 64) {
+        double x[W::RPL], dmax, kappa;
+        W::load(M, R, x);
+        const double tr = W::trace(M, R, dmax);
+        if (relative) tol *= dmax;
+        bool ok = W::inverse(col, x, R);
+        ok = W::well_posed(x, tr, tol, kappa) && ok;
+        if (ok) W::store(out + blockIdx.x * R2, R, x);
         if (threadIdx.x == 0) {
-            double m = 0.0;
-            for (int a = 0; a < R; a++) m = fmax(m, sh.A[tri_index(R, a, a)]);
-            dmax = m;
+            done = ok ? 1 : 0;
+            tol_sh = tol;
         }
-        __syncthreads();
-        tol *= dmax;
     }
+    __syncthreads();
+    if (done) return;
+    load_upper(M, R, sh.A);
     jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
-    pinv_from_jacobi(sh, R, tol, out + blockIdx.x * R2);
+    pinv_from_jacobi(sh, R, tol_sh, out + blockIdx.x * R2);
 }
 
 // ---------------------------------------------------------------- STS computeM
-// sts_cp.hpp:80-188 for target mode j, one workgroup.  grams: N x R x R
-// (full symmetric), M: (N+2) x R x R, lam: (N+1) x R.
-template <int NBL, int NV>
-__global__ __launch_bounds__(kJacobiThreads) void sts_compute_m_kernel(int N, int j, int R, const double* __restrict__ grams,
-                                                                 double* __restrict__ M, double* __restrict__ lam) {
-#pragma clang fp contract(off)
-    __shared__ EighShared sh;
-    __shared__ int ord[kMaxRank];
-    const int R2 = R * R;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    for (int i = tid; i < R2; i += nt) M[N * R2 + i] = 1.0;
-    __syncthreads();
-    int last = N;
-    for (int k = N - 1; k >= 0; k--) {
+// sts_cp.hpp:80-188 for target mode j.  grams: N x R x R (full symmetric), M:
+// (N+2) x R x R, lam: (N+1) x R.  Slot 0 is the pseudo-inverse of the Hadamard
+// product H of the other modes' Grams (eigenvalues at or below 1e-8 dropped),
+// slot N the rows u / sqrt(lam) of H's eigenvectors, slot k the rows
+// sqrt(lam) u of those of A_k = (later Grams) (.) slot 0.  The reference solves
+// slot N, then slot 0, then each k in turn; here every slot has a workgroup of
+// its own.
+//
+// The draws pick an eigenvector by its mass, so they depend on the vectors and
+// not only on the matrix.  Where H's (or A_k's) eigenvalues are apart, the
+// vectors are determined to rounding and the one-sided Jacobi's serve as well;
+// slot 0 is then the Gauss-Jordan inverse, where that shows that no eigenvalue is
+// dropped, so that one eigendecomposition is the longest chain.  Where two are
+// closer than kGap of the largest (kappa: slot 0 carries H's condition number
+// into A_k), the vectors of two solvers differ by more than about 5 eps / kGap =
+// 1e-9 (a draw in 1e4 calls of J = 65536 would move), and the oracle's two-sided
+// Jacobi runs, operation for operation: mostly before the first updates, when
+// every Gram is near the identity.
+constexpr double kGap = 1e-6;
+
+// The two-sided chain, in the oracle's order: H's eigenvectors, W = V
+// diag(lam^-1/2) with columns reversed (sh.w.L, row-major), slot 0 = W W^T (its
+// upper triangle packed), and for slot k the eigenvectors of later (.) slot 0.
+// sh.e.A holds H's upper triangle, sh.later the later Grams'.
+__device__ __forceinline__ int compute_m_slot(int N, int j, int block) {
+    // workgroup 0: slot N; workgroup q: the q-th k of N-1 .. 1 (k != j)
+    for (int k = N - 1, q = 0; k > 0 && block > 0; k--) {
         if (k == j) continue;
-        for (int i = tid; i < R2; i += nt) M[k * R2 + i] = grams[k * R2 + i] * M[last * R2 + i];
-        __syncthreads();
-        last = k;
+        if (++q == block) return k;
     }
-    if (j == 0) {
-        for (int i = tid; i < R2; i += nt) M[i] = M[R2 + i];
-        __syncthreads();
+    return N;
+}
+
+// One wavefront per slot; status[workgroup] = 1 where it wrote its slot.
+template <int NMAX>
+__global__ __launch_bounds__(64) void sts_compute_m_kernel(int N, int j, int R, const double* __restrict__ grams,
+                                                           double* __restrict__ M, double* __restrict__ lam,
+                                                           int* __restrict__ status) {
+    typedef WavePsd<NMAX> W;
+    __shared__ WavePsdShared<NMAX> sh;
+    const int R2 = R * R, tid = threadIdx.x;
+    const int slot = compute_m_slot(N, j, blockIdx.x);
+    const int lj = tid % NMAX, g = tid / NMAX;
+    double a[W::RPL], x[W::RPL], later[W::RPL];
+    double tr = 0.0, lo = 1e300, hi = 0.0, off2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < W::RPL; r++) {
+        const int i = g * W::RPL + r;
+        const bool in = i < R && lj < R;
+        const int o = in ? (i <= lj ? i * R + lj : lj * R + i) : 0;
+        double h = 1.0, lt = 0.0;
+        for (int k = N - 1; k >= 0; k--) {
+            if (k == j) continue;
+            h *= grams[k * R2 + o];
+            if (k == slot) lt = h;
+        }
+        a[r] = in ? h : 0.0;
+        later[r] = in ? lt : 0.0;
+        x[r] = a[r];
+        if (in && i == lj) {
+            tr += h;
+            lo = fmin(lo, h);
+            hi = fmax(hi, h);
+        } else if (in) {
+            off2 = fma(h, h, off2);
+        }
     }
-    for (int i = tid; i < R2; i += nt) M[(N + 1) * R2 + i] = M[i];
+    if (blockIdx.x == 0) W::store(M + (N + 1) * R2, R, a);
+    for (int off = 32; off >= 1; off >>= 1) {
+        tr += __shfl_xor(tr, off, 64);
+        off2 += __shfl_xor(off2, off, 64);
+        lo = fmin(lo, __shfl_xor(lo, off, 64));
+        hi = fmax(hi, __shfl_xor(hi, off, 64));
+    }
+    // R eigenvalues in an interval of this width, about R^2 / 4 to a close
+    // pair: near the identity nothing is tried
+    auto spread = [&](double l, double h, double o2, double gap) {
+        return R < 2 || 4.0 * (h - l + 2.0 * sqrt(o2)) > gap * R * R * h;
+    };
+    bool fast = spread(lo, hi, off2, kGap);
+    double kappa, gap = kGap;
+    if (fast) {
+        fast = W::inverse(sh.col, x, R);
+        fast = W::well_posed(x, tr, 1e-8, kappa) && fast;
+    }
+    if (fast && slot != N) {
+        gap *= fmax(1.0, 1e-2 * kappa);
+        lo = 1e300;
+        hi = off2 = 0.0;
+#pragma unroll
+        for (int r = 0; r < W::RPL; r++) {
+            a[r] = later[r] * x[r];
+            const int i = g * W::RPL + r;
+            if (i < R && lj < R && i == lj) {
+                lo = fmin(lo, a[r]);
+                hi = fmax(hi, a[r]);
+            } else {
+                off2 = fma(a[r], a[r], off2);
+            }
+        }
+        for (int off = 32; off >= 1; off >>= 1) {
+            off2 += __shfl_xor(off2, off, 64);
+            lo = fmin(lo, __shfl_xor(lo, off, 64));
+            hi = fmax(hi, __shfl_xor(hi, off, 64));
+        }
+        fast = spread(lo, hi, off2, gap);
+    }
+    if (fast) {
+        if (slot == N) W::store(M, R, x);
+        fast = W::cholesky(sh, a, R);
+        if (fast) {
+            W::onesided(sh, R);
+            fast = !W::close_pair(sh, R, gap);
+        }
+    }
+    if (tid == 0) status[blockIdx.x] = fast ? 1 : 0;
+    if (!fast) return;
+    // rows ascending by eigenvalue (slot N: descending, scaled by 1 / sqrt(lam))
+    const int ne = R + (R & 1);
+    for (int o = tid; o < ne * R; o += 64) {
+        const int c = o / R, u = o % R, at = sh.pos[c];
+        if (at < 0) continue;
+        const double lv = sh.lam[c], v = sh.L[c * NMAX + u];
+        if (slot == N) M[(int64_t)N * R2 + (R - 1 - at) * R + u] = lv > 1e-8 ? v / lv : 0.0;
+        else M[(int64_t)slot * R2 + at * R + u] = v;
+        if (u == 0) lam[(slot == N ? 0 : slot) * R + at] = lv;
+    }
+}
+
+// The slots that the kernel above left: the two-sided chain in the oracle's
+// order.  H's eigenvectors, W = V diag(lam^-1/2) with columns reversed, slot 0 =
+// W W^T, and for slot k the eigenvectors of A_k.
+template <int NBL, int NV>
+__global__ __launch_bounds__(kJacobiThreads) void sts_compute_m_exact(int N, int j, int R, const double* __restrict__ grams,
+                                                                      double* __restrict__ M, double* __restrict__ lam,
+                                                                      const int* __restrict__ status) {
+#pragma clang fp contract(off)
+    if (status[blockIdx.x] != 0) return;   // the same for the whole workgroup
+    constexpr int NMAX = NBL == 1 ? 32 : 64;
+    __shared__ EighSharedT<NMAX> sh;
+    __shared__ double Wm[NMAX * NMAX], later[NMAX * (NMAX + 1) / 2], s0[NMAX * (NMAX + 1) / 2];
+    __shared__ int ord[NMAX];
+    const int R2 = R * R, tid = threadIdx.x, nt = blockDim.x;
+    const int slot = compute_m_slot(N, j, blockIdx.x);
+    for (int o = tid; o < R2; o += nt) {
+        const int p = o / R, q = o % R;
+        if (p > q) continue;
+        double h = 1.0, lt = 0.0;
+        for (int k = N - 1; k >= 0; k--) {
+            if (k == j) continue;
+            h *= grams[k * R2 + o];
+            if (k == slot) lt = h;
+        }
+        sh.A[tri_index(R, p, q)] = h;
+        later[tri_index(R, p, q)] = lt;
+    }
     __syncthreads();
-    // eigendecomposition of the Hadamard product; slot N = V diag(lam^-1/2), columns reversed
-    load_upper(M, R, sh.A);
     jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
     if (tid < R) ord[sh.j.rank[tid]] = tid;
     __syncthreads();
-    if (tid < R) lam[sh.j.rank[tid]] = sh.A[tri_index(R, tid, tid)];
     for (int o = tid; o < R2; o += nt) {
-        int u = o / R, vs = o % R;          // vs = sorted column
-        int v = ord[vs];
-        double lv = sh.A[tri_index(R, v, v)];
-        M[N * R2 + u * R + R - 1 - vs] = lv > 1e-8 ? sh.V[u * R + v] / sqrt(lv) : 0.0;
+        const int u = o / R, vs = o % R;          // vs = sorted column
+        const int v = ord[vs];
+        const double lv = sh.A[tri_index(R, v, v)];
+        Wm[u * R + R - 1 - vs] = lv > 1e-8 ? sh.V[u * R + v] / sqrt(lv) : 0.0;
     }
+    if (slot == N && tid < R) lam[sh.j.rank[tid]] = sh.A[tri_index(R, tid, tid)];
     __syncthreads();
-    // slot 0 = W W^T (upper computed, mirrored)
     for (int o = tid; o < R2; o += nt) {
-        int a = o / R, b = o % R;
-        if (a > b) continue;
+        const int p = o / R, q = o % R;
+        if (p > q) continue;
         double acc = 0.0;
-        for (int c = 0; c < R; c++) acc += M[N * R2 + a * R + c] * M[N * R2 + b * R + c];
-        M[a * R + b] = acc;
-        M[b * R + a] = acc;
+        for (int c = 0; c < R; c++) acc += Wm[p * R + c] * Wm[q * R + c];
+        s0[tri_index(R, p, q)] = acc;
     }
     __syncthreads();
-    for (int k = N - 1; k > 0; k--) {
-        if (k == j) continue;
-        for (int i = tid; i < R2; i += nt) M[k * R2 + i] *= M[i];
-    }
-    __syncthreads();
-    for (int k = N; k > 0; k--) {
-        if (k == j) continue;
-        if (k < N) {
-            load_upper(M + k * R2, R, sh.A);
-            jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
-            if (tid < R) ord[sh.j.rank[tid]] = tid;
-            __syncthreads();
-            if (tid < R) lam[k * R + sh.j.rank[tid]] = sh.A[tri_index(R, tid, tid)];
-            // scaled eigenvectors, already transposed: row vs = sqrt(lam) * eigenvector
-            for (int o = tid; o < R2; o += nt) {
-                int vs = o / R, u = o % R;
-                int v = ord[vs];
-                double lv = sh.A[tri_index(R, v, v)];
-                M[k * R2 + vs * R + u] = sh.V[u * R + v] * sqrt(lv > 0.0 ? lv : 0.0);
-            }
-            __syncthreads();
-        } else {
-            // transpose slot N in place
-            for (int o = tid; o < R2; o += nt) {
-                int a = o / R, b = o % R;
-                if (a >= b) continue;
-                double x = M[N * R2 + a * R + b], y = M[N * R2 + b * R + a];
-                M[N * R2 + a * R + b] = y;
-                M[N * R2 + b * R + a] = x;
-            }
-            __syncthreads();
+    if (slot == N) {
+        for (int o = tid; o < R2; o += nt) {
+            const int p = o / R, q = o % R;
+            M[(int64_t)N * R2 + o] = Wm[q * R + p];
+            M[o] = s0[sym_index(R, p, q)];
         }
+        return;
+    }
+    for (int e = tid; e < tri_size(R); e += nt) sh.A[e] = later[e] * s0[e];
+    __syncthreads();
+    jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
+    if (tid < R) {
+        ord[sh.j.rank[tid]] = tid;
+        lam[slot * R + sh.j.rank[tid]] = sh.A[tri_index(R, tid, tid)];
+    }
+    __syncthreads();
+    for (int o = tid; o < R2; o += nt) {
+        const int vs = o / R, u = o % R;
+        const int v = ord[vs];
+        const double lv = sh.A[tri_index(R, v, v)];
+        M[(int64_t)slot * R2 + vs * R + u] = sh.V[u * R + v] * sqrt(lv > 0.0 ? lv : 0.0);
     }
 }
 
@@ -517,9 +647,17 @@ void eigh(hipStream_t s, const double* A, int R, double* lam, double* V, int nco
     EX_HIP(hipGetLastError());
 }
 
+// The wavefront solves, sized to the rank: columns padded to 16, 32 or 64.
+#define PSD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                                     \
+    do {                                                                                                              \
+        if ((R) <= 16) hipLaunchKernelGGL((KERNEL<16, 1, 2>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);     \
+        else if ((R) <= 32) hipLaunchKernelGGL((KERNEL<32, 1, 2>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__); \
+        else hipLaunchKernelGGL((KERNEL<64, 3, 8>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);               \
+    } while (0)
+
 void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int ncopies, const int* only_if,
           bool relative) {
-    JACOBI_DISPATCH(R, pinv_kernel, dim3(ncopies), s, M, R, tol, out, only_if, relative ? 1 : 0);
+    PSD_DISPATCH(R, pinv_kernel, dim3(ncopies), s, M, R, tol, out, only_if, relative ? 1 : 0);
     EX_HIP(hipGetLastError());
 }
 
@@ -583,7 +721,14 @@ void plain_sum(hipStream_t s, const double* v, int64_t n, double* out, DevBuf& p
 }
 
 void sts_compute_m(hipStream_t s, int N, int j, int R, const double* grams, double* M, double* lam) {
-    JACOBI_DISPATCH(R, sts_compute_m_kernel, dim3(1), s, N, j, R, grams, M, lam);
+    // one workgroup per slot: N and every k in 1 .. N-1, k != j
+    int jobs = 1;
+    for (int k = 1; k < N; k++) jobs += k != j ? 1 : 0;
+    int* status = reinterpret_cast<int*>(lam + (int64_t)(N + 1) * R);
+    if (R <= 16) hipLaunchKernelGGL(sts_compute_m_kernel<16>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
+    else if (R <= 32) hipLaunchKernelGGL(sts_compute_m_kernel<32>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
+    else hipLaunchKernelGGL(sts_compute_m_kernel<64>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
+    JACOBI_DISPATCH(R, sts_compute_m_exact, dim3(jobs), s, N, j, R, grams, M, lam, status);
     EX_HIP(hipGetLastError());
 }
 
