@@ -274,7 +274,7 @@ struct Span {
 // with the tensor so that a call enqueued on a caller's stream allocates
 // nothing once they are large enough).
 struct AdjScratch {
-    DevBuf kd, sd, wd, dg, dm, dD, table, work, cnt;
+    DevBuf kd, sd, wd, dg, dm, dD, table, work, cnt, units;
     DevBuf tmp[4];
 };
 
@@ -1057,7 +1057,7 @@ void smttkrp_backward_on(ex_tensor* t, hipStream_t st, int mode, int64_t Ju, con
     double* gp[kMaxModes] = {};
     for (int k2 = 0; k2 < t->N; k2++) gp[k2] = k2 == mode ? nullptr : grads[k2];
     k::smttkrp_adjoint(st, t->lk[mode], a.kd.as<uint64_t>(), samples, weights, Ju, t->N, mode, R, factors, G, gp,
-                       a.dD.as<double>());
+                       a.dD.as<double>(), a.units, a.cnt.as<uint64_t>());
     for (int k2 = 0; k2 < t->N; k2++)
         if (gp[k2]) k::poison_unless(st, a.cnt.as<uint64_t>(), Ju, gp[k2], t->dims[k2] * R);
 }

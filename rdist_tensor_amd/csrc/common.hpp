@@ -137,7 +137,7 @@ struct ModeLookup {
     DevBuf cpos;    // u32[nnz]: design row of the hit at a row-order position (valid where its bit is set)
     DevBuf marks;   // u8, whole 4096-position chunks: 1 at this step's hit positions (zero between steps)
     DevBuf cpart;   // u64 per-workgroup counter partials of the passes
-    // bucketed path (built on first use): key-order target row and value of each nonzero
+    // bucketed path and adjoint (built on first use): key-order target row and value of each nonzero
     DevBuf krow;    // u32[nnz]
     DevBuf kval;    // f64[nnz]
     DevBuf kval32;  // f32[nnz]
@@ -265,9 +265,11 @@ void exact_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const V* const* U
                   V* Y, int64_t I_j, DevBuf* tmp, uint64_t* counts = nullptr);
 // Adjoint of the sampled MTTKRP: dD = per-sample fiber sums of x * G[row]
 // (Ju x R, written), then grads[k] (k != j, non-null) += dD * dDesign/dU_k.
-void smttkrp_adjoint(hipStream_t s, const ModeLookup& L, const uint64_t* kd, const uint32_t* sd, const double* wd,
+// work: the units of long fibers; *distinct: the number of distinct keys in kd
+// (the gradients are not formed unless it is Ju).
+void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uint32_t* sd, const double* wd,
                      int64_t Ju, int N, int j, int R, const double* const* U, const double* G,
-                     double* const* grads, double* dD);
+                     double* const* grads, double* dD, DevBuf& work, const uint64_t* distinct);
 // out[0..n) = NaN unless *count == want: a device-side argument check whose
 // failure the caller sees in the output, with nothing waited for.
 void poison_unless(hipStream_t s, const uint64_t* count, int64_t want, double* out, int64_t n);

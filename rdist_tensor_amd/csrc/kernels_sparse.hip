@@ -1886,32 +1886,199 @@ void design(hipStream_t s, const uint32_t* sd, const double* wd, int64_t Ju, int
     EX_HIP(hipGetLastError());
 }
 
+// Lanes per hit of the grouped row sums: a power of two covering R columns
+// at group_vw values per lane.
+template <typename V>
+int group_lanes(int R) {
+    const int need = (R + group_vw<V>() - 1) / group_vw<V>();
+    int G = 2;
+    while (G < need) G *= 2;
+    return G;
+}
+
+// f(std::integral_constant<int, G>) for the runtime lane count G.
+template <typename F>
+void with_group(int G, F f) {
+    switch (G) {
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 8: f(std::integral_constant<int, 8>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        default: f(std::integral_constant<int, 32>{}); break;
+    }
+}
+
+// Key-order copies of a mode's target rows and values (L.krow, L.kval or
+// L.kval32), built on first use.
+template <typename V>
+void key_order(hipStream_t s, ModeLookup& L, const V* vals) {
+    DevBuf& kv = sizeof(V) == 4 ? L.kval32 : L.kval;
+    const bool rows = !L.krow.p;
+    const size_t n = (size_t)(L.nnz > 0 ? L.nnz : 1);
+    if (rows) L.krow.ensure(n * 4);
+    kv.ensure(n * sizeof(V));
+    if (L.nnz == 0) return;
+    hipLaunchKernelGGL(bk_keyorder<V>, dim3(grid_for(L.nnz, kThreads, 16384)), dim3(kThreads), 0, s,
+                       L.kpos.as<uint32_t>(), L.rrow.as<uint32_t>(), vals, L.nnz,
+                       rows ? L.krow.as<uint32_t>() : nullptr, kv.as<V>());
+}
+
 // ---------------------------------------------------------------- adjoint
 // dD[c] = sum over the nonzeros (row i, value x) of sample c's fiber of
-// x * G[i]: the transpose of the sampled MTTKRP, one wavefront per sample
-// (lane r < R sums column r over the fiber's nonzeros in key order).
+// x * G[i]: the transpose of the sampled MTTKRP.  The nonzeros are read in key
+// order (L.krow, L.kval), where a fiber's are contiguous, and the rows of G
+// gathered by GL lanes each, two columns a lane, 64 / GL nonzeros side by side
+// and kAdjBatch of each group in flight.
+//
+// Leverage samples fall on long fibers (Zipf(1.1), 2e7 nonzeros: 4e4 and more
+// in the longest), and one wavefront walking such a fiber set the time of the
+// whole launch.  A fiber of at most kAdjUnit nonzeros is summed by its sample's
+// wavefront; a longer one is cut into units of kAdjUnit, which fiber_units sums
+// (one wavefront a unit) and fiber_total adds in order, so the result does not
+// depend on the order in which the units were listed.  J = 65536, R = 32: 35.2
+// ms in one launch before, 0.24 ms in these (0.155 + 0.075 + 0.01).
+constexpr int kAdjUnit = 512;
+constexpr int kAdjBatch = 4;
+
+struct AdjUnits {
+    unsigned int* count;   // [0] units, [1] cut fibers (zero before and after a call)
+    uint2* unit;           // (first key-order position, its nonzeros) of each unit
+    uint4* cut;            // (sample, first unit, units) of each cut fiber
+    double* part;          // units x R
+};
+
+// acc[v] = sum over key-order positions [k0, k1) of kval * G[krow][2 sub + v],
+// complete in every lane group.
+template <int GL>
+__device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ krow, const double* __restrict__ kval,
+                                          uint32_t k0, uint32_t k1, const double* __restrict__ G, int R, bool vec,
+                                          int lane, double (&acc)[2]) {
+    constexpr int S = 64 / GL;
+    typedef double VT __attribute__((ext_vector_type(2)));
+    const int g = lane / GL, col = 2 * (lane % GL);
+    const int c0 = col < R ? col : 0, c1 = col + 1 < R ? col + 1 : 0;
+    acc[0] = acc[1] = 0.0;
+    for (uint32_t k = k0; k < k1; k += kAdjBatch * S) {
+        uint32_t row[kAdjBatch];
+        double x[kAdjBatch], d[kAdjBatch][2];
+#pragma unroll
+        for (int b = 0; b < kAdjBatch; b++) {
+            const uint32_t i = k + b * S + g;
+            const uint32_t at = i < k1 ? i : k1 - 1;
+            row[b] = krow[at];
+            const double v = kval[at];
+            x[b] = i < k1 ? v : 0.0;
+        }
+#pragma unroll
+        for (int b = 0; b < kAdjBatch; b++) {
+            const double* r = G + (int64_t)row[b] * R;
+            if (vec) {
+                const VT v = *reinterpret_cast<const VT*>(r + c0);
+                d[b][0] = v[0];
+                d[b][1] = v[1];
+            } else {
+                d[b][0] = r[c0];
+                d[b][1] = r[c1];
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kAdjBatch; b++) {
+            // (a position past the end adds nothing, whatever the row holds)
+            const bool in = k + b * S + g < k1;
+            acc[0] += in ? x[b] * d[b][0] : 0.0;
+            acc[1] += in ? x[b] * d[b][1] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int o = GL; o < 64; o <<= 1) {
+        acc[0] += __shfl_xor(acc[0], o, 64);
+        acc[1] += __shfl_xor(acc[1], o, 64);
+    }
+}
+
+template <int GL>
+__device__ __forceinline__ void adj_store(double* __restrict__ out, int R, int lane, const double (&acc)[2]) {
+    const int col = 2 * lane;
+    if (lane < GL && col < R) out[col] = acc[0];
+    if (lane < GL && col + 1 < R) out[col + 1] = acc[1];
+}
+
+template <int GL>
 __global__ __launch_bounds__(kThreads) void fiber_adjoint(const uint64_t* __restrict__ kd, int64_t Ju,
                                                           const uint64_t* __restrict__ fkey, int64_t nfib,
                                                           const uint32_t* __restrict__ fptr,
-                                                          const uint32_t* __restrict__ kpos,
-                                                          const uint32_t* __restrict__ rrow,
-                                                          const double* __restrict__ rval,
-                                                          const double* __restrict__ G, int R,
-                                                          double* __restrict__ dD) {
+                                                          const uint32_t* __restrict__ krow,
+                                                          const double* __restrict__ kval,
+                                                          const double* __restrict__ G, int R, bool vec,
+                                                          double* __restrict__ dD, AdjUnits units,
+                                                          const uint64_t* __restrict__ distinct) {
+    // repeated samples: the caller's outputs become NaN, and kd holds fewer
+    // than Ju keys (the unit lists are sized for distinct fibers)
+    if ((int64_t)*distinct != Ju) return;
     const int lane = threadIdx.x % 64;
     for (int64_t c = blockIdx.x * (int64_t)(kThreads / 64) + threadIdx.x / 64; c < Ju;
          c += (int64_t)gridDim.x * (kThreads / 64)) {
         const int64_t f = wave_find_key(fkey, nfib, kd[c], lane);
-        double acc = 0.0;
-        if (f >= 0 && lane < R) {
-            const uint32_t k1 = fptr[f + 1];
-            for (uint32_t k = fptr[f]; k < k1; k++) {
-                const uint32_t p = kpos[k];
-                acc += rval[p] * G[(int64_t)rrow[p] * R + lane];
+        double acc[2] = {0.0, 0.0};
+        if (f >= 0) {
+            const uint32_t k0 = fptr[f], k1 = fptr[f + 1];
+            if (units.count && k1 - k0 > kAdjUnit) {
+                const uint32_t n = (k1 - k0 + kAdjUnit - 1) / kAdjUnit;
+                uint32_t u0 = 0;
+                if (lane == 0) {
+                    u0 = atomicAdd(units.count, n);
+                    units.cut[atomicAdd(units.count + 1, 1u)] = make_uint4((uint32_t)c, u0, n, 0u);
+                }
+                u0 = readlane_u32(u0, 0);
+                for (uint32_t q = lane; q < n; q += 64) {
+                    const uint32_t b = k0 + q * kAdjUnit;
+                    units.unit[u0 + q] = make_uint2(b, k1 - b < kAdjUnit ? k1 - b : kAdjUnit);
+                }
+                continue;   // fiber_total writes this sample's row
             }
+            fiber_sum<GL>(krow, kval, k0, k1, G, R, vec, lane, acc);
         }
-        if (lane < R) dD[c * R + lane] = acc;
+        adj_store<GL>(dD + c * R, R, lane, acc);
     }
+}
+
+template <int GL>
+__global__ __launch_bounds__(kThreads) void fiber_units(const uint32_t* __restrict__ krow,
+                                                        const double* __restrict__ kval,
+                                                        const double* __restrict__ G, int R, bool vec,
+                                                        AdjUnits units) {
+    const int lane = threadIdx.x % 64;
+    const uint32_t n = units.count[0];
+    for (uint32_t u = blockIdx.x * (kThreads / 64) + threadIdx.x / 64; u < n; u += gridDim.x * (kThreads / 64)) {
+        const uint2 w = units.unit[u];
+        double acc[2];
+        fiber_sum<GL>(krow, kval, w.x, w.x + w.y, G, R, vec, lane, acc);
+        adj_store<GL>(units.part + (int64_t)u * R, R, lane, acc);
+    }
+}
+
+// One wavefront per cut fiber, lane r on column r: its units in order.
+__global__ __launch_bounds__(kThreads) void fiber_total(AdjUnits units, int R, double* __restrict__ dD) {
+    const int lane = threadIdx.x % 64;
+    const int col = lane < R ? lane : 0;
+    const uint32_t n = units.count[1];
+    for (uint32_t q = blockIdx.x * (kThreads / 64) + threadIdx.x / 64; q < n; q += gridDim.x * (kThreads / 64)) {
+        const uint4 w = units.cut[q];
+        double acc = 0.0;
+        for (uint32_t u = 0; u < w.z; u += 8) {
+            double v[8];
+#pragma unroll
+            for (int b = 0; b < 8; b++) v[b] = units.part[(int64_t)(w.y + (u + b < w.z ? u + b : w.z - 1)) * R + col];
+#pragma unroll
+            for (int b = 0; b < 8; b++)
+                if (u + b < w.z) acc += v[b];
+        }
+        if (lane < R) dD[(int64_t)w.x * R + lane] = acc;
+    }
+}
+
+__global__ void adj_clear(unsigned int* count) {
+    if (threadIdx.x < 2) count[threadIdx.x] = 0u;
 }
 
 struct GradArgs {
@@ -1951,13 +2118,39 @@ void poison_unless(hipStream_t s, const uint64_t* count, int64_t want, double* o
     EX_HIP(hipGetLastError());
 }
 
-void smttkrp_adjoint(hipStream_t s, const ModeLookup& L, const uint64_t* kd, const uint32_t* sd, const double* wd,
+void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uint32_t* sd, const double* wd,
                      int64_t Ju, int N, int j, int R, const double* const* U, const double* G,
-                     double* const* grads, double* dD) {
+                     double* const* grads, double* dD, DevBuf& work, const uint64_t* distinct) {
     if (Ju == 0) return;
-    hipLaunchKernelGGL(fiber_adjoint, dim3(grid_for(Ju, kThreads / 64, 16384)), dim3(kThreads), 0, s, kd, Ju,
-                       L.fkey.as<uint64_t>(), L.nfib, L.fptr.as<uint32_t>(), L.kpos.as<uint32_t>(),
-                       L.rrow.as<uint32_t>(), L.rval.as<double>(), G, R, dD);
+    if (!L.kval.p) key_order<double>(s, L, L.rval.as<double>());
+    // units of cut fibers: at most one per kAdjUnit hits and one more per cut
+    // fiber, each of which has more than kAdjUnit of the hits
+    AdjUnits units{};
+    if (L.maxfib > kAdjUnit) {
+        const double hb = (double)Ju * (double)L.maxfib;
+        const int64_t Hb = hb < (double)L.nnz ? (int64_t)hb : L.nnz;
+        const int64_t nu = 2 * (Hb / kAdjUnit) + 2, nc = Hb / kAdjUnit + 1;
+        size_t o = 0;
+        auto take = [&](size_t bytes) { size_t r = o; o = (o + bytes + 255) & ~(size_t)255; return r; };
+        const size_t o_c = take(8), o_u = take((size_t)nu * 8), o_l = take((size_t)nc * 16),
+                     o_p = take((size_t)nu * R * 8);
+        work.ensure(o);
+        char* b = work.as<char>();
+        units = AdjUnits{(unsigned int*)(b + o_c), (uint2*)(b + o_u), (uint4*)(b + o_l), (double*)(b + o_p)};
+        hipLaunchKernelGGL(adj_clear, dim3(1), dim3(64), 0, s, units.count);
+    }
+    const bool vec = R % 2 == 0 && ((uintptr_t)G % 16) == 0;
+    const dim3 block(kThreads);
+    with_group(group_lanes<double>(R), [&](auto gc) {
+        constexpr int GL = decltype(gc)::value;
+        hipLaunchKernelGGL(fiber_adjoint<GL>, dim3(grid_for(Ju, kThreads / 64, 16384)), block, 0, s, kd, Ju,
+                           L.fkey.as<uint64_t>(), L.nfib, L.fptr.as<uint32_t>(), L.krow.as<uint32_t>(),
+                           L.kval.as<double>(), G, R, vec, dD, units, distinct);
+        if (units.count)
+            hipLaunchKernelGGL(fiber_units<GL>, dim3((unsigned)(8 * num_cus(s))), block, 0, s, L.krow.as<uint32_t>(),
+                               L.kval.as<double>(), G, R, vec, units);
+    });
+    if (units.count) hipLaunchKernelGGL(fiber_total, dim3((unsigned)num_cus(s)), block, 0, s, units, R, dD);
     DesignArgs a;
     GradArgs g;
     for (int k = 0; k < N; k++) {
@@ -2019,16 +2212,6 @@ void carry_reduce(hipStream_t s, DevBuf* tmp, int64_t n1, int R, V* Y, const uin
     }
 }
 
-// Lanes per hit of the grouped row sums: a power of two covering R columns
-// at group_vw values per lane.
-template <typename V>
-int group_lanes(int R) {
-    const int need = (R + group_vw<V>() - 1) / group_vw<V>();
-    int G = 2;
-    while (G < need) G *= 2;
-    return G;
-}
-
 // Lanes per hit of the sampled-MTTKRP row pass: group_lanes, doubled (at
 // most 32) when the autotuner chose the wider variant.
 template <typename V>
@@ -2036,18 +2219,6 @@ int scan_lanes(int R) {
     int G = group_lanes<V>(R);
     if (tune_value(sizeof(V) == 8 ? kTuneScanF64 : kTuneScanF32) == 1 && G < 32) G *= 2;
     return G;
-}
-
-// f(std::integral_constant<int, G>) for the runtime lane count G.
-template <typename F>
-void with_group(int G, F f) {
-    switch (G) {
-        case 2: f(std::integral_constant<int, 2>{}); break;
-        case 4: f(std::integral_constant<int, 4>{}); break;
-        case 8: f(std::integral_constant<int, 8>{}); break;
-        case 16: f(std::integral_constant<int, 16>{}); break;
-        default: f(std::integral_constant<int, 32>{}); break;
-    }
 }
 
 // Per-workgroup counter partials of a pass over `blocks` workgroups (null
@@ -2066,15 +2237,7 @@ void sampled_mttkrp_buckets(hipStream_t s, ModeLookup& L, const V* vals, const u
     const int64_t nnz = L.nnz;
     EX_CHECK(nnz < ((int64_t)1 << 31), 4, "the bucketed sampled MTTKRP needs fewer than 2^31 nonzeros");
     DevBuf& kv = sizeof(V) == 4 ? L.kval32 : L.kval;
-    if (!kv.p) {
-        // key-order target rows and values, on first use
-        const bool rows = !L.krow.p;
-        if (rows) L.krow.ensure((size_t)nnz * 4);
-        kv.ensure((size_t)nnz * sizeof(V));
-        hipLaunchKernelGGL(bk_keyorder<V>, dim3(grid_for(nnz, kThreads, 16384)), dim3(kThreads), 0, s,
-                           L.kpos.as<uint32_t>(), L.rrow.as<uint32_t>(), vals, nnz,
-                           rows ? L.krow.as<uint32_t>() : nullptr, kv.as<V>());
-    }
+    if (!kv.p) key_order<V>(s, L, vals);
     int bsh = 13;
     while (((nnz - 1) >> bsh) + 1 > kBkMaxBuckets) bsh++;
     const int NB = (int)(((nnz - 1) >> bsh) + 1);
