@@ -285,7 +285,7 @@ struct ex_tensor {
     int64_t nnz = 0;
     DevBuf coords;  // u32 nnz x N
     DevBuf vals;    // f64 nnz
-    double norm = 0.0;
+    double norm = 0.0, norm2 = 0.0;   // |X|, |X|^2
     bool built = false;
     ModeLookup lk[kMaxModes];
     DevBuf tmp[4];
@@ -393,6 +393,7 @@ struct ex_als {
     bool exact = false, grams_valid = false;
     DevBuf grams;
     DevBuf sd, wd, kd, dg, dm, G, Gi, pivflag, GY, Ms, Y, scal;
+    DevBuf fit_grams, fit_part;
     DevBuf dht, dhw;   // hashed deduplication: table (zero between steps), per-sample slots
     DevBuf tmp[4];
     DevBuf part;
@@ -981,28 +982,29 @@ void exact_step_impl(ex_als* a, int j) {
     if (a->ev_pending.size() >= 6 * 64) als_resolve_regions(a);
 }
 
+// 1 - |X - Xh| / |X| by |X|^2 + |Xh|^2 - 2 <X, Xh>.
 double als_fit_impl(ex_als* a) {
     ex_factors* f = a->f;
+    ex_tensor* t = a->t;
     hipStream_t st = a->ctx->c.stream;
     const int N = f->N, R = f->R;
     a->scal.ensure(64);
-    a->G.ensure((size_t)N * R * R * 8 > (size_t)R * R * 8 ? (size_t)N * R * R * 8 : (size_t)R * R * 8);
-    DevBuf grams;
-    grams.ensure((size_t)N * R * R * 8);
+    a->fit_grams.ensure((size_t)N * R * R * 8);
     f->sync64_all();
     for (int k2 = 0; k2 < N; k2++)
-        k::gram(st, f->U[k2].as<double>(), f->dims[k2], R, grams.as<double>() + (int64_t)k2 * R * R, a->part);
+        k::gram(st, f->U[k2].as<double>(), f->dims[k2], R, a->fit_grams.as<double>() + (int64_t)k2 * R * R, a->part);
     double* d = a->scal.as<double>();
-    k::chain_had_norm(st, grams.as<double>(), N, R, f->sigma.as<double>(), d);
-    DevBuf fpart;
-    k::fit_bmb(st, a->t->coords.as<uint32_t>(), a->t->vals.as<double>(), a->t->nnz, N, f->ptrs,
-               f->sigma.as<double>(), R, d + 1, fpart);
+    k::chain_had_norm(st, a->fit_grams.as<double>(), N, R, f->sigma.as<double>(), d);
+    // in the row order of mode 0 the last mode's rows are the scattered ones,
+    // in the last mode's order the one before it: the smaller factor of the two
+    const int by = t->dims[N - 1] <= t->dims[N - 2] ? 0 : N - 1;
+    k::fit_dot(st, t->lk[by], f->ptrs, t->dims, f->sigma.as<double>(), R, d + 1, a->fit_part);
     double h[2];
     d2h(st, h, d, sizeof(h));
-    // |X - Xh|^2 by expansion: where the model reproduces X it is rounding
-    // noise of either sign, and a negative one counts as zero (NaN stays)
-    const double res2 = h[0] + h[1];
-    return 1.0 - std::sqrt(res2 < 0.0 ? 0.0 : res2) / a->t->norm;
+    // where the model reproduces X this is rounding noise of either sign, and
+    // a negative one counts as zero (NaN stays)
+    const double res2 = t->norm2 + h[0] - 2.0 * h[1];
+    return 1.0 - std::sqrt(res2 < 0.0 ? 0.0 : res2) / t->norm;
 }
 
 // Keys of device sample tuples for `mode`, checked distinct (the sampled
@@ -1216,6 +1218,7 @@ int ex_tensor_create(ex_ctx* ctx, int N, const int64_t* dims, int64_t nnz, const
         k::sumsq(st, t->vals.as<double>(), nnz, out1.as<double>(), part);
         double ss = 0;
         d2h(st, &ss, out1.p, 8);
+        t->norm2 = ss;
         t->norm = std::sqrt(ss);
         *out = t.release();
     });

@@ -273,8 +273,9 @@ void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uin
 // out[0..n) = NaN unless *count == want: a device-side argument check whose
 // failure the caller sees in the output, with nothing waited for.
 void poison_unless(hipStream_t s, const uint64_t* count, int64_t want, double* out, int64_t n);
-void fit_bmb(hipStream_t s, const uint32_t* coords, const double* vals, int64_t nnz, int N, const double* const* U,
-             const double* sigma, int R, double* out, DevBuf& part);
+// *out = <X, Xh> over the lookup's nonzeros (FP64 factors).
+void fit_dot(hipStream_t s, const ModeLookup& L, const double* const* U, const int64_t* dims, const double* sigma,
+             int R, double* out, DevBuf& part);
 // final stages shared with the mixed-precision kernels
 void gram_final_launch(hipStream_t s, const double* part, int nb, int R, double* G);
 void col_sumsq_final_launch(hipStream_t s, const double* part, int nb, int R, double* sigma);
