@@ -371,7 +371,9 @@ struct ex_sampler {
     // u64: STS-CP draws given weight 0 since creation (mixed path: a
     // rounding residue routed the draw into a leaf of zero mass)
     DevBuf dropped;
-    DevBuf first_cdf;   // mixed: prefix sums of the first non-target mode's leaf masses
+    // mixed: prefix sums of the first non-target mode's leaf masses; FP64: its
+    // node masses and draws
+    DevBuf first_cdf;
     // set when a batch advanced the factors: every mode's state is rebuilt
     // before the next draw or score read
     bool refresh = false;
@@ -549,16 +551,24 @@ void sampler_draw_impl(ex_sampler* s, int64_t J, int j, uint64_t sweep, const do
         Span sd(s->ctx, "sts_draw");
         // mixed: the first non-target mode's draws search prefix sums of its
         // leaf masses (its running product is 1, so R queries cover them all)
+        const int k0 = j == 0 ? 1 : 0;
         const double* first_cdf = nullptr;
         if (mixed && tune_value(kTuneFirstF32) == 0) {
-            const int k0 = j == 0 ? 1 : 0;
             const size_t L0 = s->g[k0].leaf_count;
             s->first_cdf.ensure((size_t)R * (L0 + (L0 + 31) / 32) * 8);
             k::sts_first_cdf(st, m[k0], R, s->first_cdf.as<double>());
             first_cdf = s->first_cdf.as<double>();
         }
+        // FP64: its draws from tabulated masses where that is faster
+        const k::StsFirstDraw* first_draw = nullptr;
+        if (!mixed && k::sts_first_pays(m[k0], R, J)) {
+            s->first_cdf.ensure(k::sts_first_bytes(m[k0], R, J));
+            const k::StsFirstArgs fa{m[k0].g, m[k0].ge, j, k0, J, s->seed, sweep, s->sweep_dev, draws_row_dev,
+                                     draws_eig_dev};
+            first_draw = k::sts_first_draw(st, m[k0], R, fa, s->first_cdf.p);
+        }
         k::sts_draw(st, N, j, R, J, m, s->pinvp.as<double>(), s->seed, sweep, draws_row_dev, draws_eig_dev, samples,
-                    weights, mixed ? 4 : 8, s->sweep_dev, s->dropped.as<unsigned long long>(), first_cdf);
+                    weights, mixed ? 4 : 8, s->sweep_dev, s->dropped.as<unsigned long long>(), first_cdf, first_draw);
         sd.end();
     }
 }
@@ -781,7 +791,7 @@ std::vector<const void*> graph_fingerprint(const ex_als* a) {
         add(*b);
     for (const DevBuf& b : a->tmp) add(b);
     for (const DevBuf* b : {&s->sums, &s->gtmp, &s->gpinv, &s->grams, &s->M, &s->lam, &s->eig, &s->eig32, &s->pinvp,
-                            &s->part, &s->samples, &s->weights, &s->draws_row, &s->draws_eig, &s->pivflag})
+                            &s->part, &s->samples, &s->weights, &s->draws_row, &s->draws_eig, &s->pivflag, &s->first_cdf})
         add(*b);
     for (int k2 = 0; k2 < kMaxModes; k2++) {
         add(s->scores[k2]);
@@ -1501,7 +1511,7 @@ int ex_sampler_create(ex_ctx* ctx, ex_factors* f, int kind, int precision, uint6
             s->lam.ensure((size_t)(N + 1) * R * 8 + kMaxModes * 4);   // eigenvalues, then a word per slot
             with_slack(s->eig, (size_t)N * s->ge.node_count * S * 8);
             if (precision == EX_MIXED) with_slack(s->eig32, (size_t)N * s->ge.node_count * tri_stride32(R) * 4);
-            s->pinvp.ensure((size_t)tri_pad64(R) * 8);
+            s->pinvp.ensure((size_t)tri_pad256(R) * 8);
         }
         for (int k2 = 0; k2 < N; k2++) sampler_update_impl(s.get(), k2);
         EX_HIP(hipStreamSynchronize(ctx->c.stream));

@@ -79,9 +79,9 @@ __host__ __device__ inline int tri_stride32(int R) { return (tri_size(R) + 31) &
 // reads all NV W-wide vectors of a node's G lanes (up to 17 KB) without a
 // bound check, so the reads past the last node land here.
 constexpr size_t kNodeSlackBytes = 32768;
-// Packed size rounded up to a multiple of 64 (a weight table read G lanes at a
-// time, G <= 64, with no bound check).
-__host__ __device__ inline int tri_pad64(int R) { return (tri_size(R) + 63) & ~63; }
+// Packed size rounded up to a multiple of 256 (a weight table read by G lanes,
+// G <= 64, up to four entries each, with no bound check).
+__host__ __device__ inline int tri_pad256(int R) { return (tri_size(R) + 255) & ~255; }
 
 // Heap-ordered segment tree over ceil(n/F) leaves (PartitionTree geometry,
 // partition_tree.hpp:82-115).
@@ -206,15 +206,38 @@ struct StsModeArgs {
     TreeGeom g;
     TreeGeom ge;
 };
+// The first non-target mode's draw of one sample: the position in the leaf as a
+// fraction of its mass, the eigen component, the leaf.
+struct StsFirstDraw {
+    double frac;
+    uint32_t component, leaf;
+};
+struct StsFirstArgs {
+    TreeGeom g, ge;        // the mode's row tree, the eigen trees
+    int j, k;              // target mode, the mode drawn
+    int64_t J;
+    uint64_t seed, sweep;
+    const uint64_t* sweep_dev;
+    const double* draws_row;
+    const double* draws_eig;
+};
+// FP64: the first non-target mode's draws from tabulated node masses, in work
+// (sts_first_bytes, 16-byte aligned); sts_first_pays: whether that is the
+// faster way to J of them.
+bool sts_first_pays(const StsModeArgs& m, int R, int64_t J);
+size_t sts_first_bytes(const StsModeArgs& m, int R, int64_t J);
+const StsFirstDraw* sts_first_draw(hipStream_t s, const StsModeArgs& m, int R, const StsFirstArgs& a, void* work);
 // node_bytes = 8: FP64 rows and row-tree nodes; 4: FP32 (the mixed path).
 // first_cdf (FP32 only): the prefix sums of sts_first_cdf for the first
 // non-target mode, whose draws then search them instead of descending the
-// trees (nullptr: every mode descends).
+// trees (nullptr: every mode descends).  first_draw (FP64 only): that mode's
+// draws, already made.
 void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* modes,
               const double* pinv_packed, uint64_t seed, uint64_t sweep,
               const double* draws_row, const double* draws_eig, uint32_t* samples, double* weights,
               int node_bytes = 8, const uint64_t* sweep_dev = nullptr,
-              unsigned long long* dropped = nullptr, const double* first_cdf = nullptr);
+              unsigned long long* dropped = nullptr, const double* first_cdf = nullptr,
+              const StsFirstDraw* first_draw = nullptr);
 // The first non-target mode's draw distribution in closed form: with the
 // running product h = 1 the row query is an eigen row w_v, so the leaf
 // masses m_v(l) = w_v^T G_l w_v (FP32 row-tree leaf Grams) give, per
@@ -223,8 +246,8 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
 // totals, cdf[R L + v NT + q]; the last is v's total.  R <= 64; cdf holds
 // R (L + NT) doubles.
 void sts_first_cdf(hipStream_t s, const StsModeArgs& m, int R, double* cdf);
-// packed[e] = (1 on the diagonal, 2 off it) x M[a][b] for the packed upper
-// element e = (a, b), zeros up to tri_pad64(R) entries (the draw's weight table).
+// packed[e] = M[a][b] for the packed upper element e = (a, b), zeros up to
+// tri_pad256(R) entries (the draw's weight table).
 void pack_upper(hipStream_t s, const double* M, int R, double* packed);
 // sparse
 void keys_from_coords(hipStream_t s, const uint32_t* coords, int64_t n, const KeyLayout& kl, uint64_t* keys,

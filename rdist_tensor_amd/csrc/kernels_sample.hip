@@ -8,6 +8,7 @@
 // discrete_distribution (random.tcc:2655-2712).
 #include "common.hpp"
 #include "device.hpp"
+#include "wave_psd.hpp"
 
 namespace exafac {
 namespace {
@@ -147,8 +148,8 @@ struct StsArgs {
     k::StsModeArgs m[kMaxModes];
     int N, j, R;
     int64_t J;
-    const double* pinvp;    // M[0] = pinv of the Hadamard product, packed upper with off-diagonal
-                            // entries doubled and zeros up to tri_pad64(R) entries (FP64)
+    const double* pinvp;    // M[0] = pinv of the Hadamard product, packed upper with zeros up to
+                            // tri_pad256(R) entries (FP64)
     uint64_t seed, sweep;
     const uint64_t* sweep_dev;   // when set, the sweep number is read here (graph replays)
     const double* draws_row;
@@ -158,6 +159,7 @@ struct StsArgs {
     unsigned long long* dropped;   // when set, draws given weight 0 are counted here
     int vec_leaf;           // leaf rows read as W-wide vectors (R % W == 0, aligned factors)
     const double* first_cdf;   // FP32: prefix sums for the first non-target mode (sts_first_cdf), or null
+    const k::StsFirstDraw* first_draw;   // FP64: the first non-target mode's draws (sts_first_draw), or null
 };
 
 // Lane exchange inside rows of 16 lanes through DPP (CTRL: quad_perm,
@@ -174,6 +176,17 @@ __device__ __forceinline__ double dpp_x(double v) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
+// v + the value of lane ^ 16 (or ^ 32), the same bits in both: the halves are
+// swapped between two copies of v.
+__device__ __forceinline__ float add_xor16(float v) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float add_xor32(float v) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
 // Sum over aligned groups of G lanes (8, 16, 32 or 64).  Each step adds the
 // same two operands on both partner lanes, so every lane of a group ends
 // with the same bits.
@@ -183,8 +196,40 @@ __device__ __forceinline__ V group_total(V v) {
     v += dpp_x<0x4E>(v);    // quad_perm [2,3,0,1]
     v += dpp_x<0x141>(v);   // row_half_mirror: quad 0 <-> quad 1 of each half row
     if (G >= 16) v += dpp_x<0x140>(v);   // row_mirror: half rows swapped
-    if (G >= 32) v += __shfl_xor(v, 16, 64);
-    if (G >= 64) v += __shfl_xor(v, 32, 64);
+    if (G >= 32) v = add_xor16(v);
+    if (G >= 64) v = add_xor32(v);
+    return v;
+}
+
+// Inclusive prefix sum over aligned groups of G lanes, l = lane in the group.
+template <int CTRL>
+__device__ __forceinline__ double dpp_shr(double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int G>
+__device__ __forceinline__ double group_scan(double v, int l) {
+    const int r = l & 15;
+    double y = dpp_shr<0x111>(v);   // row_shr:1, :2, :4, :8
+    v += r >= 1 ? y : 0.0;
+    y = dpp_shr<0x112>(v);
+    v += (G == 8 ? l & 7 : r) >= 2 ? y : 0.0;
+    y = dpp_shr<0x114>(v);
+    v += (G == 8 ? l & 7 : r) >= 4 ? y : 0.0;
+    if (G >= 16) {
+        y = dpp_shr<0x118>(v);
+        v += r >= 8 ? y : 0.0;
+    }
+    if (G >= 32) {
+        y = __shfl(v, (int)(threadIdx.x & 32) | 15, 64);   // the lower 16 lanes' total
+        v += (l & 16) ? y : 0.0;
+    }
+    if (G >= 64) {
+        y = __shfl(v, 31, 64);
+        v += (l & 32) ? y : 0.0;
+    }
     return v;
 }
 
@@ -199,15 +244,19 @@ template <> struct Vec<double> {
 };
 
 // LDS of one draw block: the packed-upper (a, b) table, and per sample the
-// running Hadamard product h, the current query and the leaf's q^2, in rows
-// of RP >= RMAX elements.  With RP = RMAX + 1 the groups of a wavefront,
-// which read the same element of their own rows together, fall on different
-// banks; with RP = RMAX (a power of two) every other group shares banks.
+// running Hadamard product h, the current query and the leaf's q^2.  A query
+// row holds x, then 2 x, then a zero: the table has the byte offsets of x_a and of
+// x_b (a == b) or 2 x_b (a < b), and of the zero past the triangle, so that an
+// entry of the weighted outer product is two reads and one product.  Rows of
+// odd length, so that the groups of a wavefront, which read the same element of
+// their own rows together, fall on different banks; h and q2 rows of RP
+// elements, RMAX + 1 or (a power of two, every other group sharing banks) RMAX.
 template <typename TN, int SLOTS, int RMAX, int RP>
 struct DrawShared {
-    uint16_t pairs[(RMAX * (RMAX + 1) / 2 + 63) & ~63];   // (0, 0) past the triangle
+    static constexpr int RX = 2 * RMAX + 1;
+    alignas(16) uint32_t pairs[(RMAX * (RMAX + 1) / 2 + 255) & ~255];
     TN h[SLOTS][RP];
-    TN x[SLOTS][RP];
+    TN x[SLOTS][RX];
     double q2[SLOTS][RP];
 };
 
@@ -225,25 +274,23 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+template <typename TN>
+__device__ __forceinline__ TN row_at(const TN* x, uint32_t off) {
+    return *reinterpret_cast<const TN*>(reinterpret_cast<const char*>(x) + off);
+}
+
 // xx[e] = w_e x_a x_b for the lane's packed elements e = (t G + l) W + i,
-// w = 1 on the diagonal and 2 off it, 0 past the triangle.
+// w = 1 on the diagonal and 2 off it, 0 past the triangle (x: a query row).
 template <typename TN, int G, int NV>
-__device__ __forceinline__ void outer_g(const uint16_t* pairs, const TN* x, int P, int l,
-                                        TN (&xx)[NV * Vec<TN>::W]) {
+__device__ __forceinline__ void outer_g(const uint32_t* pairs, const TN* x, int l, TN (&xx)[NV * Vec<TN>::W]) {
     constexpr int W = Vec<TN>::W;
+    typedef uint32_t PT __attribute__((ext_vector_type(W)));
 #pragma unroll
-    for (int t = 0; t < NV; t++)
+    for (int t = 0; t < NV; t++) {
+        const PT pr = *reinterpret_cast<const PT*>(pairs + (t * G + l) * W);
 #pragma unroll
-        for (int i = 0; i < W; i++) {
-            const int e = (t * G + l) * W + i;
-            TN v = 0;
-            if (e < P) {
-                const uint32_t pr = pairs[e];
-                const int a = pr & 0xFF, b = pr >> 8;
-                v = (a == b ? (TN)1 : (TN)2) * (x[a] * x[b]);
-            }
-            xx[t * W + i] = v;
-        }
+        for (int i = 0; i < W; i++) xx[t * W + i] = row_at(x, pr[i] & 0xFFFFu) * row_at(x, pr[i] >> 16);
+    }
 }
 
 // x^T G x of one packed node for the group's query: vector loads of W
@@ -295,15 +342,14 @@ __device__ __forceinline__ V sub_total(V v, int SG) {
     return v;
 }
 
-// Passes over a leaf whose loads are issued together (fewer in FP64, where
-// more would cost occupancy).
-template <typename TN>
-constexpr int leaf_batch() { return sizeof(TN) == 4 ? 8 : 2; }
+// Passes over a leaf whose loads are issued together (the query's products are
+// not live here, so their registers serve).
+constexpr int kLeafBatch = 8;
 
 // q2[r] = (U_blk[r] . x)^2 for r < F (0 for r >= rows) of the leaf block blk
 // (F rows of R, row-major).  SG lanes per row (the power of two covering its
 // VL-wide vectors, at most G), G / SG rows per pass; the loads of
-// leaf_batch passes are in flight together.  VL = W needs R % W == 0 and a
+// kLeafBatch passes are in flight together.  VL = W needs R % W == 0 and a
 // W-aligned factor; VL = 1 reads single elements.
 template <typename TN, int G, int VL>
 __device__ __forceinline__ void leaf_q2(const TN* __restrict__ blk, int rows, int F, int R, const TN* x,
@@ -313,7 +359,6 @@ __device__ __forceinline__ void leaf_q2(const TN* __restrict__ blk, int rows, in
     while (SG < nvec && SG < G) SG *= 2;
     const int RPS = G / SG, sr = l / SG, sl = l % SG;
     const int nu = (nvec + SG - 1) / SG;
-    constexpr int kLeafBatch = leaf_batch<TN>();
     for (int r0 = 0; r0 < F; r0 += RPS * kLeafBatch) {
         TN part[kLeafBatch];
 #pragma unroll
@@ -356,9 +401,8 @@ __device__ __forceinline__ void leaf_q2(const TN* __restrict__ blk, int rows, in
 }
 
 // Position in the leaf of a draw at fraction frac of its mass: the first r
-// < F - 1 with frac < (q2[0] + ... + q2[r]) / (q2[0] + ... + q2[F-1]), else
-// F - 1.  Every lane of the group forms the same sequential FP64 prefix and
-// keeps the entries r = k G + l.
+// < F - 1 with frac (q2[0] + ... + q2[F-1]) < q2[0] + ... + q2[r], else F - 1.
+// FP64 prefix sums across the group, G entries at a time.
 template <int G, int RMAX>
 __device__ __forceinline__ int leaf_pick(const double* q2, int F, double frac, int l, int grp, double& total) {
     constexpr int KMAX = (RMAX + G - 1) / G;
@@ -366,22 +410,17 @@ __device__ __forceinline__ int leaf_pick(const double* q2, int F, double frac, i
     double run = 0.0;
 #pragma unroll
     for (int k = 0; k < KMAX; k++) {
-        mine[k] = 0.0;
-#pragma unroll
-        for (int i = 0; i < G; i++) {
-            const int r = k * G + i;
-            if (r < F) {
-                run += q2[r];
-                if (i == l) mine[k] = run;
-            }
-        }
+        const int r = k * G + l;
+        mine[k] = run + group_scan<G>(r < F ? q2[r] : 0.0, l);
+        run = __shfl(mine[k], grp * G + G - 1, 64);
     }
     total = run;
+    const double t = frac * run;
     const uint64_t gmask = G == 64 ? ~0ull : ((1ull << G) - 1);
 #pragma unroll
     for (int k = 0; k < KMAX; k++) {
         const int r = k * G + l;
-        const bool cond = r < F - 1 && frac < mine[k] / run;
+        const bool cond = r < F - 1 && t < mine[k];
         const uint64_t bits = (__ballot(cond) >> (grp * G)) & gmask;
         if (bits) return k * G + __ffsll((unsigned long long)bits) - 1;
     }
@@ -420,34 +459,32 @@ __device__ __forceinline__ double quad_node(const TN* __restrict__ gnodes, const
     return quad_g<TN, G, NV, BATCH>(gnodes + c * S, xx, P, l);
 }
 
-// Root-to-leaf descent of one heap tree (partition_tree.hpp:226-307): masses
-// and cutoffs in FP64, left if u <= low + m_left / m_root.
+// Root-to-leaf descent of one heap tree (partition_tree.hpp:226-307): left if
+// u <= low + m_left / m_root, in units of mass, t = u m_root against low + m_left,
+// so that no level divides.  FP64 throughout; a root without mass leads right
+// at every level, as its quotients (NaN) would.  frac: the draw's position
+// between the leaf's ends.
 template <typename TN, int G, int NV, bool BATCH>
 __device__ __forceinline__ int64_t descend_g(const TN* __restrict__ nodes, const TN* snodes, int nst,
                                              const TreeGeom& g, int S, int P, const TN (&xx)[NV * Vec<TN>::W], int l,
-                                             double u, double& low, double& high) {
+                                             double u, double& frac) {
     const double m = quad_node<TN, G, NV, BATCH>(nodes, snodes, nst, 0, S, xx, P, l);
+    const double t = m > 0.0 ? u * m : __longlong_as_double(0x7ff0000000000000ll);
     int64_t c = 0;
-    low = 0.0;
-    high = 1.0;
-    for (uint32_t lvl = 0; lvl < g.lfill_level; lvl++) {
-        const double mL = quad_node<TN, G, NV, BATCH>(nodes, snodes, nst, 2 * c + 1, S, xx, P, l);
-        const double cutoff = low + mL / m;
-        if (u <= cutoff) { c = 2 * c + 1; high = cutoff; }
+    double low = 0.0, high = m;
+    for (uint32_t lvl = 0; lvl <= g.lfill_level; lvl++) {
+        if (lvl == g.lfill_level && g.is_leaf(c)) break;
+        const double cutoff = low + quad_node<TN, G, NV, BATCH>(nodes, snodes, nst, 2 * c + 1, S, xx, P, l);
+        if (t <= cutoff) { c = 2 * c + 1; high = cutoff; }
         else { c = 2 * c + 2; low = cutoff; }
     }
-    if (!g.is_leaf(c)) {
-        const double mL = quad_node<TN, G, NV, BATCH>(nodes, snodes, nst, 2 * c + 1, S, xx, P, l);
-        const double cutoff = low + mL / m;
-        if (u <= cutoff) { c = 2 * c + 1; high = cutoff; }
-        else { c = 2 * c + 2; low = cutoff; }
-    }
+    frac = (t - low) / (high - low);
     return c;
 }
 
-// xs[b] = h[b] w[b] (FP64 product, rounded to TN) for the lane's entries b =
+// The query row of x = h w (FP64 product, rounded to TN), the lane's entries b =
 // l + q G < R; every load of w is issued before the first product.
-template <typename TN, int G, int KB>
+template <typename TN, int G, int KB, int RMAX>
 __device__ __forceinline__ void query_of(TN* xs, const TN* hs, const double* __restrict__ w, int R, int l) {
     double wv[KB];
 #pragma unroll
@@ -458,7 +495,25 @@ __device__ __forceinline__ void query_of(TN* xs, const TN* hs, const double* __r
 #pragma unroll
     for (int q = 0; q < KB; q++) {
         const int b = l + q * G;
-        if (b < R) xs[b] = (TN)((double)hs[b] * wv[q]);
+        if (b < R) {
+            const TN x = (TN)((double)hs[b] * wv[q]);
+            xs[b] = x;
+            xs[RMAX + b] = x + x;
+        }
+    }
+}
+
+// The query row of h itself.
+template <typename TN, int G, int KB, int RMAX>
+__device__ __forceinline__ void query_h(TN* xs, const TN* hs, int R, int l) {
+#pragma unroll
+    for (int q = 0; q < KB; q++) {
+        const int b = l + q * G;
+        if (b < R) {
+            const TN x = hs[b];
+            xs[b] = x;
+            xs[RMAX + b] = x + x;
+        }
     }
 }
 
@@ -547,11 +602,17 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
     const int R = a.R, N = a.N, j = a.j;
     const int P = tri_size(R);
     const int S = sizeof(TN) == 8 ? tri_stride(R) : tri_stride32(R);
-    for (int e = threadIdx.x; e < tri_pad64(R); e += blockDim.x) {
-        int ea = 0, eb = 0;
-        if (e < P) tri_ab_direct(R, e, ea, eb);
-        sh.pairs[e] = (uint16_t)(ea | (eb << 8));
+    constexpr uint32_t kZero = 2 * RMAX * sizeof(TN);
+    for (int e = threadIdx.x; e < (int)(sizeof(sh.pairs) / 4); e += blockDim.x) {
+        uint32_t pr = kZero | (kZero << 16);
+        if (e < P) {
+            int ea, eb;
+            tri_ab_direct(R, e, ea, eb);
+            pr = (uint32_t)(ea * sizeof(TN)) | ((uint32_t)((ea == eb ? eb : RMAX + eb) * sizeof(TN)) << 16);
+        }
+        sh.pairs[e] = pr;
     }
+    for (int i = threadIdx.x; i < C::SLOTS; i += blockDim.x) sh.x[i][2 * RMAX] = (TN)0;
     for (int i = threadIdx.x; i < kStageAll; i += blockDim.x) stage_all[i] = (TN)0;
     // the first non-target mode: prefix sums instead of descents when given
     const int k0 = j == 0 ? 1 : 0;
@@ -576,6 +637,15 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
     double* q2 = sh.q2[slot];
     for (int b = l; b < R; b += G) hs[b] = (TN)1;
     wave_lds_sync();
+    // the sample's uniforms, one per lane (mode l / 2; eigen draw, then row
+    // draw) where the group has the lanes for it
+    const bool spread = G >= 2 * N;
+    auto uniform_of = [&](int k, int kind) -> double {
+        if (kind == 1) return a.draws_eig ? a.draws_eig[(int64_t)k * a.J + s] : uniform01(a.seed, stream_id(sweep, j, k, 1), s);
+        return a.draws_row ? a.draws_row[(int64_t)k * a.J + s] : uniform01(a.seed, stream_id(sweep, j, k, 2), s);
+    };
+    double u_lane = 0.0;
+    if (spread && active) u_lane = uniform_of(l < 2 * N ? l >> 1 : 0, 1 + (l & 1));
     TN xx[NV * W];
     uint32_t eig_idx = 0;
     bool dropped = false;
@@ -585,11 +655,14 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
         const TN* rows_k = static_cast<const TN*>(md.rows);
         const TN* eig_k = static_cast<const TN*>(md.eig);
         const TN* nodes_k = static_cast<const TN*>(md.nodes);
-        const bool by_cdf = a.first_cdf != nullptr && k == k0;   // the same in every thread
+        // the first mode's component and leaf from its prefix sums (FP32) or
+        // from its own kernel (FP64); the same in every thread
+        const bool by_cdf = sizeof(TN) == 4 && a.first_cdf != nullptr && k == k0;
+        const bool drawn = sizeof(TN) == 8 && a.first_draw != nullptr && k == k0;
         // stage the top levels of both trees (S is a multiple of W)
         const int ne = (int)md.ge.node_count < NST ? (int)md.ge.node_count : NST;
         const int nr = (int)md.g.node_count < NST ? (int)md.g.node_count : NST;
-        if (!by_cdf) {
+        if (!by_cdf && !drawn) {
             __syncthreads();
             if (NST > 0) {
                 const int ve = ne * S / W, vr = nr * S / W;
@@ -601,13 +674,25 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
             __syncthreads();
         }
         if (!active) continue;
-        const double ue = a.draws_eig ? a.draws_eig[(int64_t)k * a.J + s]
-                                      : uniform01(a.seed, stream_id(sweep, j, k, 1), s);
-        const double ur = a.draws_row ? a.draws_row[(int64_t)k * a.J + s]
-                                      : uniform01(a.seed, stream_id(sweep, j, k, 2), s);
+        double ue = 0.0, ur = 0.0;
+        if (spread) {
+            ue = __shfl(u_lane, grp * G + 2 * k, 64);
+            ur = __shfl(u_lane, grp * G + 2 * k + 1, 64);
+        } else if (!drawn) {
+            ue = uniform_of(k, 1);
+            ur = uniform_of(k, 2);
+        }
         int64_t v, leaf;
         double frac;
-        if (by_cdf) {
+        if (drawn) {
+            const k::StsFirstDraw fd = a.first_draw[s];
+            v = fd.component;
+            leaf = fd.leaf;
+            frac = fd.frac;
+            eig_idx = (uint32_t)v;
+            query_of<TN, G, KB, RMAX>(xs, hs, md.w + v * R, R, l);
+            wave_lds_sync();
+        } else if (by_cdf) {
             // component v with probability proportional to its total, then
             // the leaf at ur x total: the tile from the tiles' cumulative
             // totals, the leaf from the tile's own prefix sums
@@ -624,22 +709,24 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
             const double lo = jj > 0 ? lpt[jj - 1] : 0.0;
             frac = (t - base - lo) / (lpt[jj] - lo);
             eig_idx = (uint32_t)v;
-            query_of<TN, G, KB>(xs, hs, md.w + v * R, R, l);
+            query_of<TN, G, KB, RMAX>(xs, hs, md.w + v * R, R, l);
             wave_lds_sync();
         } else {
             // eigen tree: query h, F = 1
-            outer_g<TN, G, NV>(sh.pairs, hs, P, l, xx);
-            double low, high;
-            int64_t c = descend_g<TN, G, NV, C::BATCH>(eig_k, stage[0], ne, md.ge, S, P, xx, l, ue, low, high);
+            query_h<TN, G, KB, RMAX>(xs, hs, R, l);
+            wave_lds_sync();
+            outer_g<TN, G, NV>(sh.pairs, xs, l, xx);
+            double ignore;
+            int64_t c = descend_g<TN, G, NV, C::BATCH>(eig_k, stage[0], ne, md.ge, S, P, xx, l, ue, ignore);
             v = md.ge.leaf_idx(c);
             eig_idx = (uint32_t)v;
-            query_of<TN, G, KB>(xs, hs, md.w + v * R, R, l);
+            wave_lds_sync();
+            query_of<TN, G, KB, RMAX>(xs, hs, md.w + v * R, R, l);
             wave_lds_sync();
             // row tree: query sh = h * w_v, F = R
-            outer_g<TN, G, NV>(sh.pairs, xs, P, l, xx);
-            c = descend_g<TN, G, NV, C::BATCH>(nodes_k, stage[1], nr, md.g, S, P, xx, l, ur, low, high);
+            outer_g<TN, G, NV>(sh.pairs, xs, l, xx);
+            c = descend_g<TN, G, NV, C::BATCH>(nodes_k, stage[1], nr, md.g, S, P, xx, l, ur, frac);
             leaf = md.g.leaf_idx(c);
-            frac = (ur - low) / (high - low);
         }
         const int F = (int)md.g.F;
         const int rows = (int)((md.g.n - leaf * F) < F ? (md.g.n - leaf * F) : F);
@@ -662,16 +749,22 @@ __global__ __launch_bounds__(NT) void sts_draw_kernel(StsArgs a) {
         if (l == 0) a.samples[s * N + k] = (uint32_t)row;
     }
     if (!active) return;
-    // weight = R / (J * h^T pinv h), FP64
-    // (the table's diagonal factors are folded in and its padding is zero,
-    // so the G-strided terms need no bound check)
+    // weight = R / (J * h^T pinv h), FP64 (zeros past the triangle in the
+    // table and in the pseudo-inverse, so the vectors need no bound)
+    query_h<TN, G, KB, RMAX>(xs, hs, R, l);
+    wave_lds_sync();
     double q = 0.0;
-    const int ksteps = (P + G - 1) / G;
-#pragma unroll 8
-    for (int t = 0; t < ksteps; t++) {
-        const int e = t * G + l;
-        const uint32_t pr = sh.pairs[e];
-        q += a.pinvp[e] * ((double)hs[pr & 0xFF] * (double)hs[pr >> 8]);
+    const int vsteps = (P + G * W - 1) / (G * W);
+    typedef uint32_t PT __attribute__((ext_vector_type(W)));
+    typedef double DT __attribute__((ext_vector_type(W)));
+#pragma unroll 4
+    for (int t = 0; t < vsteps; t++) {
+        const int e = (t * G + l) * W;
+        const PT pr = *reinterpret_cast<const PT*>(sh.pairs + e);
+        const DT m = *reinterpret_cast<const DT*>(a.pinvp + e);
+#pragma unroll
+        for (int i = 0; i < W; i++)
+            q += m[i] * ((double)row_at(xs, pr[i] & 0xFFFFu) * (double)row_at(xs, pr[i] >> 16));
     }
     q = group_total<G>(q);
     if (l == 0) {
@@ -803,6 +896,161 @@ __global__ __launch_bounds__(1024) void first_scan_kernel(double* __restrict__ t
     }
 }
 
+// ---------------------------------------------------------------- first mode, FP64
+// A draw's running product is 1 in its first non-target mode, so every sample
+// asks that mode's trees the same R + 1 questions: the eigen tree's masses for
+// the query 1, and the row tree's for the R rows w_v.  Where many samples
+// descend the tree, all masses of all nodes are formed first, one FP64 matrix
+// product that reads each node once (mass[v NC + c] = sum_e A[v][e] G_c[e],
+// A[v][e] = (a == b ? 1 : 2) w_v[a] w_v[b] for the packed element e = (a, b)),
+// and a sample's descent reads one number per level instead of a node of
+// R (R + 1) / 2.  The comparisons are the descent's own.
+
+// A in the order the matrix instructions take it: step t of K block b, lane i +
+// 16 h supplies A[16 vt + i][32 b + 8 h + t] (so that a lane's node elements are
+// eight consecutive ones), at frag[((vt KB + b) 8 + t) 64 + lane]; and, by
+// workgroup `blocks` + c, the eigen node c's mass for the query 1.
+__global__ __launch_bounds__(kThreads) void first64_weights(const double* __restrict__ w, int R, int KB, int VT,
+                                                            int blocks, double* __restrict__ frag,
+                                                            const double* __restrict__ eig, int S,
+                                                            double* __restrict__ emass) {
+    const int P = tri_size(R);
+    if ((int)blockIdx.x < blocks) {
+        const int o = blockIdx.x * kThreads + threadIdx.x;
+        if (o >= VT * KB * 512) return;
+        const int lane = o % 64, t = (o / 64) % 8, b = (o / 512) % KB, vt = o / (512 * KB);
+        const int v = 16 * vt + lane % 16, e = 32 * b + 8 * (lane / 16) + t;
+        double x = 0.0;
+        if (e < P && v < R) {
+            int ea, eb;
+            tri_ab_direct(R, e, ea, eb);
+            x = (ea == eb ? 1.0 : 2.0) * (w[v * R + ea] * w[v * R + eb]);
+        }
+        frag[o] = x;
+        return;
+    }
+    __shared__ double red[kWaves];
+    const int c = blockIdx.x - blocks;
+    double acc = 0.0;
+    for (int e = threadIdx.x; e < P; e += kThreads) {
+        int ea, eb;
+        tri_ab_direct(R, e, ea, eb);
+        acc += (ea == eb ? 1.0 : 2.0) * eig[(int64_t)c * S + e];
+    }
+    acc = wave_sum(acc);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) emass[c] = red[0] + red[1] + red[2] + red[3];
+}
+
+// Masses of 32 nodes per workgroup, all components, on v_mfma_f64_16x16x4
+// (lane l: A[l % 16][l / 16], B[l / 16][l % 16], C[4 i + l / 16][l % 16]).  The
+// four wavefronts take the K blocks in turn, so that a small tree's launch is
+// not one long chain, and their products are added in wavefront order.
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+template <int VT>
+__global__ __launch_bounds__(kThreads) void first64_mass(const double* __restrict__ nodes, int64_t NC, int R, int S,
+                                                         int KB, const double* __restrict__ frag,
+                                                         double* __restrict__ mass) {
+    __shared__ double part[kWaves - 1][VT][2][4][64];
+    const int lane = threadIdx.x % 64, wv = threadIdx.x / 64, i = lane % 16, h = lane / 16;
+    const int64_t c0 = (int64_t)blockIdx.x * 32;
+    const int P = tri_size(R);
+    const double* p[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) p[q] = nodes + (c0 + 16 * q + i < NC ? c0 + 16 * q + i : NC - 1) * S + 8 * h;
+    f64x4 acc[VT][2];
+#pragma unroll
+    for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) acc[vt][q] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int b = wv; b < KB; b += kWaves) {
+        f64x2 x[2][4];
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) x[q][u] = *reinterpret_cast<const f64x2*>(p[q] + 32 * b + 2 * u);
+        double A[VT][8];
+#pragma unroll
+        for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+            for (int t = 0; t < 8; t++) A[vt][t] = frag[((vt * KB + b) * 8 + t) * 64 + lane];
+        if (b == KB - 1)   // past the triangle: the next node's elements, or the slack
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int z = 0; z < 2; z++)
+                        if (32 * b + 8 * h + 2 * u + z >= P) x[q][u][z] = 0.0;
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+#pragma unroll
+            for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    acc[vt][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[vt][t], x[q][t / 2][t % 2], acc[vt][q], 0, 0, 0);
+    }
+    if (wv > 0)
+#pragma unroll
+        for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) part[wv - 1][vt][q][r][lane] = acc[vt][q][r];
+    __syncthreads();
+    if (wv != 0) return;
+#pragma unroll
+    for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                double m = acc[vt][q][r];
+#pragma unroll
+                for (int w2 = 0; w2 < kWaves - 1; w2++) m += part[w2][vt][q][r][lane];
+                const int v = 16 * vt + 4 * r + h;
+                const int64_t c = c0 + 16 * q + i;
+                if (v < R && c < NC) mass[(int64_t)v * NC + c] = m;
+            }
+}
+
+// The descent of descend_g by tabulated masses.
+__device__ __forceinline__ int64_t descend_masses(const double* mass, const TreeGeom& g, double u, double& frac) {
+    const double m = mass[0];
+    const double t = m > 0.0 ? u * m : __longlong_as_double(0x7ff0000000000000ll);
+    int64_t c = 0;
+    double low = 0.0, high = m;
+    for (uint32_t lvl = 0; lvl <= g.lfill_level; lvl++) {
+        if (lvl == g.lfill_level && g.is_leaf(c)) break;
+        const double cutoff = low + mass[2 * c + 1];
+        if (t <= cutoff) { c = 2 * c + 1; high = cutoff; }
+        else { c = 2 * c + 2; low = cutoff; }
+    }
+    frac = (t - low) / (high - low);
+    return c;
+}
+
+__global__ __launch_bounds__(kThreads) void first64_descend(k::StsFirstArgs a, const double* __restrict__ emass,
+                                                            const double* __restrict__ mass,
+                                                            k::StsFirstDraw* __restrict__ out) {
+    __shared__ double em[2 * kMaxRank];
+    for (int c = threadIdx.x; c < (int)a.ge.node_count; c += kThreads) em[c] = emass[c];
+    __syncthreads();
+    const int64_t s = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (s >= a.J) return;
+    const uint64_t sweep = a.sweep_dev ? *a.sweep_dev : a.sweep;
+    const double ue = a.draws_eig ? a.draws_eig[(int64_t)a.k * a.J + s]
+                                  : uniform01(a.seed, stream_id(sweep, a.j, a.k, 1), s);
+    const double ur = a.draws_row ? a.draws_row[(int64_t)a.k * a.J + s]
+                                  : uniform01(a.seed, stream_id(sweep, a.j, a.k, 2), s);
+    double frac;
+    const int64_t v = a.ge.leaf_idx(descend_masses(em, a.ge, ue, frac));
+    const int64_t leaf = a.g.leaf_idx(descend_masses(mass + v * (int64_t)a.g.node_count, a.g, ur, frac));
+    out[s] = k::StsFirstDraw{frac, (uint32_t)v, (uint32_t)leaf};
+}
+
 // ---------------------------------------------------------------- CP-ARLS-LEV
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kThreads * kScanItems;
@@ -913,6 +1161,50 @@ __global__ __launch_bounds__(kThreads) void arls_draw_kernel(ArlsArgs a) {
 
 namespace k {
 
+// Doubles of the tables of sts_first_draw: A, the eigen masses, the masses; the
+// draws follow (16 bytes each).
+static int64_t first_tables(const StsModeArgs& m, int R) {
+    const int64_t KB = (tri_size(R) + 31) / 32, VT = (R + 15) / 16;
+    return VT * KB * 512 + 2 * kMaxRank + (int64_t)R * m.g.node_count;
+}
+
+// The tables cost three launches and one pass over the tree, the descents a node
+// per level and sample.  Measured (two modes of 3e5 rows, a draw with descents
+// only against one with the first mode tabulated): R = 32, J = 65536 648 -> 476
+// us, 16384 182 -> 168, 4096 65 -> 83; R = 64 3190 -> 1941, 785 -> 614, 202 ->
+// 257; R = 16, J = 65536 182 -> 151.
+bool sts_first_pays(const StsModeArgs& m, int R, int64_t J) {
+    return J >= (R <= 16 ? 24576 : 16384) && J * (int64_t)(m.g.lfill_level + 1) >= 4 * (int64_t)m.g.node_count;
+}
+
+size_t sts_first_bytes(const StsModeArgs& m, int R, int64_t J) {
+    return (size_t)first_tables(m, R) * 8 + (size_t)J * sizeof(StsFirstDraw);
+}
+
+const StsFirstDraw* sts_first_draw(hipStream_t s, const StsModeArgs& m, int R, const StsFirstArgs& a, void* work) {
+    const int S = tri_stride(R), KB = (tri_size(R) + 31) / 32, VT = (R + 15) / 16;
+    const int64_t NC = m.g.node_count;
+    double* frag = static_cast<double*>(work);
+    double* emass = frag + (int64_t)VT * KB * 512;
+    double* mass = emass + 2 * kMaxRank;
+    StsFirstDraw* out = reinterpret_cast<StsFirstDraw*>(frag + first_tables(m, R));
+    const int blocks = (VT * KB * 512 + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(first64_weights, dim3(blocks + m.ge.node_count), dim3(kThreads), 0, s, m.w, R, KB, VT, blocks,
+                       frag, static_cast<const double*>(m.eig), S, emass);
+    const dim3 grid((unsigned)((NC + 31) / 32));
+    const double* nodes = static_cast<const double*>(m.nodes);
+    switch (VT) {
+        case 1: hipLaunchKernelGGL(first64_mass<1>, grid, dim3(kThreads), 0, s, nodes, NC, R, S, KB, frag, mass); break;
+        case 2: hipLaunchKernelGGL(first64_mass<2>, grid, dim3(kThreads), 0, s, nodes, NC, R, S, KB, frag, mass); break;
+        case 3: hipLaunchKernelGGL(first64_mass<3>, grid, dim3(kThreads), 0, s, nodes, NC, R, S, KB, frag, mass); break;
+        default: hipLaunchKernelGGL(first64_mass<4>, grid, dim3(kThreads), 0, s, nodes, NC, R, S, KB, frag, mass); break;
+    }
+    hipLaunchKernelGGL(first64_descend, dim3((unsigned)((a.J + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, a,
+                       emass, mass, out);
+    EX_HIP(hipGetLastError());
+    return out;
+}
+
 void sts_first_cdf(hipStream_t s, const StsModeArgs& m, int R, double* cdf) {
     EX_CHECK(R >= 1 && R <= kMaxRank, 1, "rank out of range");
     const int64_t L = m.g.leaf_count, NT = (L + 31) / 32;
@@ -984,7 +1276,7 @@ void tree_build(hipStream_t s, const double* U, const TreeGeom& g, int R, double
 void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* modes, const double* pinv_packed,
               uint64_t seed, uint64_t sweep, const double* draws_row, const double* draws_eig, uint32_t* samples,
               double* weights, int node_bytes, const uint64_t* sweep_dev, unsigned long long* dropped,
-              const double* first_cdf) {
+              const double* first_cdf, const StsFirstDraw* first_draw) {
     EX_CHECK(node_bytes == 8 || node_bytes == 4, 1, "node precision must be FP64 or FP32");
     StsArgs a;
     for (int k = 0; k < N; k++) a.m[k] = modes[k];
@@ -995,6 +1287,7 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     a.samples = samples; a.weights = weights;
     a.dropped = dropped;
     a.first_cdf = node_bytes == 4 ? first_cdf : nullptr;
+    a.first_draw = node_bytes == 8 ? first_draw : nullptr;
     // vector reads of leaf rows: R a multiple of the vector width and every
     // drawn factor aligned to it
     const int vw = node_bytes == 8 ? 2 : 4;
@@ -1012,34 +1305,57 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     // NT threads per workgroup (1024: more samples share each staged copy of
     // the top levels; 512: registers for every node load of a level in
     // flight together).
+    bool deep = false;   // a tree of 2^7 leaves or more
+    for (int k = 0; k < N; k++) deep = deep || (k != j && modes[k].g.lfill_level >= 7);
     // Variant 0 of each rank class is the default; the others are the
     // alternatives the autotuner measures (tune_value).
     if (node_bytes == 8) {
+        // NV: no more vectors than the triangle fills (R = 25: 6, not 9)
         if (R <= 16) {
             switch (tune_value(kTuneDrawF64R16)) {
                 case 1: DRAW_LAUNCH(double, 8, 9, 1024); break;
                 case 2: DRAW_LAUNCH(double, 32, 3, 1024); break;
                 case 3: DRAW_LAUNCH(double, 8, 9, 512); break;
-                default: DRAW_LAUNCH(double, 16, 5, 1024); break;
+                default:
+                    // few samples: more lanes each, and small workgroups to
+                    // reach every CU (R = 16, J = 4096: 43 -> 22 us; J = 16384:
+                    // 45 against 57 the other way)
+                    if (J < 8192) DRAW_LAUNCH(double, 32, 3, 256);
+                    else DRAW_LAUNCH(double, 8, 9, 1024);
+                    break;
             }
         } else if (R <= 32) {
             switch (tune_value(kTuneDrawF64R32)) {
                 case 1: DRAW_LAUNCH(double, 16, 17, 1024); break;
                 case 2: DRAW_LAUNCH(double, 64, 5, 1024); break;
-                case 3: DRAW_LAUNCH(double, 32, 9, 256); break;
+                case 3: DRAW_LAUNCH(double, 32, 9, 1024); break;
                 case 4: DRAW_LAUNCH(double, 16, 17, 512); break;
                 case 5: DRAW_LAUNCH(double, 64, 5, 256); break;
-                default: DRAW_LAUNCH(double, 32, 9, 1024); break;
+                default:
+                    if (R <= 24) DRAW_LAUNCH(double, 32, 5, 256);
+                    else if (R <= 27) DRAW_LAUNCH(double, 32, 6, 256);
+                    else if (R <= 29) DRAW_LAUNCH(double, 32, 7, 256);
+                    else DRAW_LAUNCH(double, 32, 9, 256);
+                    break;
             }
+        } else if (R <= 35) {
+            DRAW_LAUNCH(double, 64, 5, 256);
+        } else if (R <= 41) {
+            DRAW_LAUNCH(double, 64, 7, 256);
         } else if (R <= 45) {
-            DRAW_LAUNCH(double, 64, 9, 1024);
+            DRAW_LAUNCH(double, 64, 9, 256);
+        } else if (R <= 54) {
+            DRAW_LAUNCH(double, 64, 12, 256);
         } else {
             DRAW_LAUNCH(double, 64, 17, 256);
         }
     } else {
         if (R <= 16) {
             switch (tune_value(kTuneDrawF32R16)) {
-                case 1: DRAW_LAUNCH(float, 8, 5, 1024); break;
+                case 1:
+                    if (J < 8192) DRAW_LAUNCH(float, 8, 5, 256);
+                    else DRAW_LAUNCH(float, 8, 5, 1024);
+                    break;
                 case 2: DRAW_LAUNCH(float, 32, 2, 1024); break;
                 case 3: DRAW_LAUNCH(float, 8, 5, 512); break;
                 default: DRAW_LAUNCH(float, 16, 3, 1024); break;
@@ -1055,10 +1371,20 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                 default: DRAW_LAUNCH(float, 8, 17, 1024); break;
             }
         } else if (R <= 45) {
-            DRAW_LAUNCH(float, 32, 9, 1024);
+            // (256 threads against 1024, R = 40, J = 65536: 514 against 678 us at
+            // 3e5 rows, 337 against 333 at 300)
+            DRAW_LAUNCH(float, 32, 9, 256);
         } else {
             switch (tune_value(kTuneDrawF32R64)) {
-                case 1: DRAW_LAUNCH(float, 32, 17, 1024); break;
+                case 1:
+                    // deep trees read most levels from L2 and beyond, where three
+                    // small workgroups per CU wait less than a large one; shallow
+                    // ones live on the levels that a large one stages (R = 64,
+                    // J = 65536: 975 against 1186 us at 3e5 rows, 622 against 529
+                    // at 300; J = 4096: 144 against 215)
+                    if (deep || J < 8192) DRAW_LAUNCH(float, 32, 17, 256);
+                    else DRAW_LAUNCH(float, 32, 17, 1024);
+                    break;
                 case 2: DRAW_LAUNCH(float, 32, 17, 512); break;
                 case 3: DRAW_LAUNCH(float, 64, 9, 256); break;
                 default: DRAW_LAUNCH(float, 64, 9, 1024); break;
