@@ -477,7 +477,10 @@ void sampler_update_mixed(ex_sampler* s, int j, int next, bool gram_done) {
     sp.end();
 }
 
-void sampler_update_impl(ex_sampler* s, int j, int next = -1, bool gram_done = false) {
+// for_batch: the state that a batch starts from, with the batch kernel's own
+// solver (the two-sided Jacobi): its sweeps run on factors of a few rows, where a
+// last-bit difference of the scores grows by orders of magnitude.
+void sampler_update_impl(ex_sampler* s, int j, int next = -1, bool gram_done = false, bool for_batch = false) {
     s->m_ready = -1;
     if (s->precision == EX_MIXED) return sampler_update_mixed(s, j, next, gram_done);
     ex_factors* f = s->f;
@@ -492,7 +495,7 @@ void sampler_update_impl(ex_sampler* s, int j, int next = -1, bool gram_done = f
         s->gtmp.ensure((size_t)R * R * 8);
         s->gpinv.ensure((size_t)R * R * 8);
         k::gram(st, U, I, R, s->gtmp.as<double>(), s->part);
-        k::pinv(st, s->gtmp.as<double>(), R, 1e-11, s->gpinv.as<double>());
+        k::pinv(st, s->gtmp.as<double>(), R, 1e-11, s->gpinv.as<double>(), 1, nullptr, false, for_batch);
         s->scores[j].ensure((size_t)I * 8);
         s->cdf[j].ensure((size_t)I * 8);
         k::dagat(st, U, I, R, s->gpinv.as<double>(), s->scores[j].as<double>());
@@ -1875,7 +1878,7 @@ int ex_batch_create(ex_als* const* als, int n, int64_t J, ex_batch** out) {
                 }
             }
             a->s->refresh = false;
-            for (int k2 = 0; k2 < a->f->N; k2++) sampler_update_impl(a->s, k2);
+            for (int k2 = 0; k2 < a->f->N; k2++) sampler_update_impl(a->s, k2, -1, false, true);
         }
         // descriptor slots: the most expensive tensors first (the queue hands
         // them out in slot order)

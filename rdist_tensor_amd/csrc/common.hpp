@@ -166,9 +166,10 @@ void gram_f32in(hipStream_t s, const float* A, int64_t m, int R, double* G, DevB
 void eigh(hipStream_t s, const double* A, int R, double* lam, double* V, int ncopies = 1);
 // only_if: when given, the launch does nothing unless *only_if != 0.
 // relative: eigenvalues <= tol * (largest diagonal entry of M) are dropped
-// instead of eigenvalues <= tol.
+// instead of eigenvalues <= tol.  two_sided: by the two-sided Jacobi whatever
+// the matrix.
 void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int ncopies = 1,
-          const int* only_if = nullptr, bool relative = false);
+          const int* only_if = nullptr, bool relative = false, bool two_sided = false);
 void dagat(hipStream_t s, const double* A, int64_t m, int R, const double* G, double* res);
 void dsymm(hipStream_t s, const double* G, const double* Y, int64_t m, int R, double* out);
 void col_sumsq(hipStream_t s, const double* U, int64_t m, int R, double* sigma, DevBuf& part);

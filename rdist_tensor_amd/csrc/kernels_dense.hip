@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kJacobiThreads) void eigh_kernel(const double* __re
 template <int NMAX, int NBL, int NV>
 __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __restrict__ Min, int R, double tol,
                                                         double* __restrict__ out, const int* __restrict__ only_if,
-                                                        int relative) {
+                                                        int relative, int two_sided) {
     if (only_if && *only_if == 0) return;   // the same for the whole block
     typedef WavePsd<NMAX> W;
     __shared__ EighSharedT<NMAX> sh;
@@ -141,8 +141,11 @@ __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __re
         W::load(M, R, x);
         const double tr = W::trace(M, R, dmax);
         if (relative) tol *= dmax;
-        bool ok = W::inverse(col, x, R);
-        ok = W::well_posed(x, tr, tol, kappa) && ok;
+        bool ok = false;
+        if (!two_sided) {
+            ok = W::inverse(col, x, R);
+            ok = W::well_posed(x, tr, tol, kappa) && ok;
+        }
         if (ok) W::store(out + blockIdx.x * R2, R, x);
         if (threadIdx.x == 0) {
             done = ok ? 1 : 0;
@@ -655,8 +658,8 @@ void eigh(hipStream_t s, const double* A, int R, double* lam, double* V, int nco
     } while (0)
 
 void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int ncopies, const int* only_if,
-          bool relative) {
-    PSD_DISPATCH(R, pinv_kernel, dim3(ncopies), s, M, R, tol, out, only_if, relative ? 1 : 0);
+          bool relative, bool two_sided) {
+    PSD_DISPATCH(R, pinv_kernel, dim3(ncopies), s, M, R, tol, out, only_if, relative ? 1 : 0, two_sided ? 1 : 0);
     EX_HIP(hipGetLastError());
 }
 
