@@ -398,7 +398,7 @@ __device__ void block_spd_pinv(const double* M, int R, double tol_rel, double* o
 __device__ void block_pinv_jacobi(const double* M, int R, double tol, double* out, const Lds& s) {
     EighSharedT<kBatchMaxRank>& sh = *reinterpret_cast<EighSharedT<kBatchMaxRank>*>(s.big + kOffSolve);
     load_upper(M, R, sh.A);
-    jacobi_block<1, 2>(sh.A, sh.A2, sh.V, R, sh.j);
+    jacobi_block<kBatchMaxRank>(sh.A, sh.A2, sh.V, R, sh.j);
     pinv_from_jacobi(sh, R, tol, out);
     __syncthreads();
 }

@@ -105,13 +105,13 @@ __global__ __launch_bounds__(kThreads) void gram_mfma64_partial(const TA* __rest
 }
 
 // Eigendecomposition of blockIdx.x-th matrix: lam ascending, V columns.
-template <int NBL, int NV>
+template <int NMAX>
 __global__ __launch_bounds__(kJacobiThreads) void eigh_kernel(const double* __restrict__ Min, int R,
                                                         double* __restrict__ lam, double* __restrict__ Vout) {
-    __shared__ EighShared sh;
+    __shared__ EighSharedT<NMAX> sh;
     const int64_t R2 = (int64_t)R * R;
     load_upper(Min + blockIdx.x * R2, R, sh.A);
-    jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
+    jacobi_block<NMAX>(sh.A, sh.A2, sh.V, R, sh.j);
     for (int o = threadIdx.x; o < R * R; o += blockDim.x) {
         int u = o / R, v = o % R;
         Vout[blockIdx.x * R2 + u * R + sh.j.rank[v]] = sh.V[u * R + v];
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kJacobiThreads) void eigh_kernel(const double* __re
 // (WavePsd::well_posed) it is the result: n pivots instead of the
 // eigendecomposition's eight sweeps of n - 1 rounds, and nearer the 64-bit value
 // (R = 32 Grams: 7e-16 against 8e-15 relative).  Otherwise the two-sided Jacobi.
-template <int NMAX, int NBL, int NV>
+template <int NMAX>
 __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __restrict__ Min, int R, double tol,
                                                         double* __restrict__ out, const int* __restrict__ only_if,
                                                         int relative, int two_sided) {
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __re
     __syncthreads();
     if (done) return;
     load_upper(M, R, sh.A);
-    jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
+    jacobi_block<NMAX>(sh.A, sh.A2, sh.V, R, sh.j);
     pinv_from_jacobi(sh, R, tol_sh, out + blockIdx.x * R2);
 }
 
@@ -180,10 +180,6 @@ __global__ __launch_bounds__(kJacobiThreads) void pinv_kernel(const double* __re
 // every Gram is near the identity.
 constexpr double kGap = 1e-6;
 
-// The two-sided chain, in the oracle's order: H's eigenvectors, W = V
-// diag(lam^-1/2) with columns reversed (sh.w.L, row-major), slot 0 = W W^T (its
-// upper triangle packed), and for slot k the eigenvectors of later (.) slot 0.
-// sh.e.A holds H's upper triangle, sh.later the later Grams'.
 __device__ __forceinline__ int compute_m_slot(int N, int j, int block) {
     // workgroup 0: slot N; workgroup q: the q-th k of N-1 .. 1 (k != j)
     for (int k = N - 1, q = 0; k > 0 && block > 0; k--) {
@@ -292,13 +288,12 @@ __global__ __launch_bounds__(64) void sts_compute_m_kernel(int N, int j, int R, 
 // The slots that the kernel above left: the two-sided chain in the oracle's
 // order.  H's eigenvectors, W = V diag(lam^-1/2) with columns reversed, slot 0 =
 // W W^T, and for slot k the eigenvectors of A_k.
-template <int NBL, int NV>
+template <int NMAX>
 __global__ __launch_bounds__(kJacobiThreads) void sts_compute_m_exact(int N, int j, int R, const double* __restrict__ grams,
                                                                       double* __restrict__ M, double* __restrict__ lam,
                                                                       const int* __restrict__ status) {
 #pragma clang fp contract(off)
     if (status[blockIdx.x] != 0) return;   // the same for the whole workgroup
-    constexpr int NMAX = NBL == 1 ? 32 : 64;
     __shared__ EighSharedT<NMAX> sh;
     __shared__ double Wm[NMAX * NMAX], later[NMAX * (NMAX + 1) / 2], s0[NMAX * (NMAX + 1) / 2];
     __shared__ int ord[NMAX];
@@ -317,7 +312,7 @@ __global__ __launch_bounds__(kJacobiThreads) void sts_compute_m_exact(int N, int
         later[tri_index(R, p, q)] = lt;
     }
     __syncthreads();
-    jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
+    jacobi_block<NMAX>(sh.A, sh.A2, sh.V, R, sh.j);
     if (tid < R) ord[sh.j.rank[tid]] = tid;
     __syncthreads();
     for (int o = tid; o < R2; o += nt) {
@@ -346,7 +341,7 @@ __global__ __launch_bounds__(kJacobiThreads) void sts_compute_m_exact(int N, int
     }
     for (int e = tid; e < tri_size(R); e += nt) sh.A[e] = later[e] * s0[e];
     __syncthreads();
-    jacobi_block<NBL, NV>(sh.A, sh.A2, sh.V, R, sh.j);
+    jacobi_block<NMAX>(sh.A, sh.A2, sh.V, R, sh.j);
     if (tid < R) {
         ord[sh.j.rank[tid]] = tid;
         lam[slot * R + sh.j.rank[tid]] = sh.A[tri_index(R, tid, tid)];
@@ -638,24 +633,18 @@ void col_sumsq_final_launch(hipStream_t s, const double* part, int nb, int R, do
 
 // Jacobi work per thread: (2x2 blocks, V rows) = (1, 2) for R <= 32, (3, 8)
 // for R <= 64.
-#define JACOBI_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                     \
-    do {                                                                                                  \
-        if ((R) <= 32) hipLaunchKernelGGL((KERNEL<1, 2>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERNEL<3, 8>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);        \
+// The R x R solves, sized to the rank: 16, 32 or 64.
+#define PSD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                                     \
+    do {                                                                                                              \
+        if ((R) <= 16) hipLaunchKernelGGL((KERNEL<16>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);     \
+        else if ((R) <= 32) hipLaunchKernelGGL((KERNEL<32>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__); \
+        else hipLaunchKernelGGL((KERNEL<64>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);               \
     } while (0)
 
 void eigh(hipStream_t s, const double* A, int R, double* lam, double* V, int ncopies) {
-    JACOBI_DISPATCH(R, eigh_kernel, dim3(ncopies), s, A, R, lam, V);
+    PSD_DISPATCH(R, eigh_kernel, dim3(ncopies), s, A, R, lam, V);
     EX_HIP(hipGetLastError());
 }
-
-// The wavefront solves, sized to the rank: columns padded to 16, 32 or 64.
-#define PSD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                                     \
-    do {                                                                                                              \
-        if ((R) <= 16) hipLaunchKernelGGL((KERNEL<16, 1, 2>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);     \
-        else if ((R) <= 32) hipLaunchKernelGGL((KERNEL<32, 1, 2>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERNEL<64, 3, 8>), GRID, dim3(kJacobiThreads), 0, STREAM, __VA_ARGS__);               \
-    } while (0)
 
 void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int ncopies, const int* only_if,
           bool relative, bool two_sided) {
@@ -730,7 +719,7 @@ void sts_compute_m(hipStream_t s, int N, int j, int R, const double* grams, doub
     if (R <= 16) hipLaunchKernelGGL(sts_compute_m_kernel<16>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
     else if (R <= 32) hipLaunchKernelGGL(sts_compute_m_kernel<32>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
     else hipLaunchKernelGGL(sts_compute_m_kernel<64>, dim3(jobs), dim3(64), 0, s, N, j, R, grams, M, lam, status);
-    JACOBI_DISPATCH(R, sts_compute_m_exact, dim3(jobs), s, N, j, R, grams, M, lam, status);
+    PSD_DISPATCH(R, sts_compute_m_exact, dim3(jobs), s, N, j, R, grams, M, lam, status);
     EX_HIP(hipGetLastError());
 }
 
