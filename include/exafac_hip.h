@@ -255,8 +255,9 @@ int ex_als_run_batch(ex_als* const* als, int n, int64_t rounds, int64_t J, doubl
  * M^T (Y^T Y) M, so results agree with ex_als_run's to rounding, not bitwise.
  * ex_batch_create rebuilds every optimizer's sampler state and copies it;
  * ex_batch_run runs `rounds` sweeps (draws keyed by sweeps 1..rounds, as
- * ex_als_run keys them), each one launch (or one graph replay after
- * ex_batch_use_graph(b, 1)); *seconds (optional) receives the wall time of
+ * ex_als_run keys them), each one launch (EX_MIXED) or a chain of launches that
+ * each run a phase of every tensor's mode step (EX_FP64), or one graph replay
+ * after ex_batch_use_graph(b, 1); *seconds (optional) receives the wall time of
  * the launches.  A factor written outside the batch after its creation makes
  * ex_batch_run fail with EX_ERR_STATE.  After a run the optimizers' own
  * sampler state is rebuilt before their next draw, so ex_als_run and fits

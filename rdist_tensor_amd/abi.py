@@ -449,7 +449,7 @@ class ALS(_Owned):
 
 
 class Batch(_Owned):
-    """CP-ARLS-LEV optimizers advanced together by one kernel launch per sweep
+    """CP-ARLS-LEV optimizers advanced together, each kernel launch for all of them
     (ex_batch_create): same device and precision, R <= 32, J <= 8192."""
     _destroy = "ex_batch_destroy"
 

@@ -1782,8 +1782,9 @@ int ex_als_run_batch(ex_als* const* als, int n, int64_t rounds, int64_t J, doubl
 }
 
 // ---------------------------------------------------------------- batched sweeps
-// Many CP-ARLS-LEV decompositions advanced by one kernel launch per sweep
-// (kernels_batch.hip): the descriptors, the per-tensor leverage state and
+// Many CP-ARLS-LEV decompositions advanced together (mixed precision: one launch
+// per sweep, kernels_batch.hip; FP64: ten per mode step, kernels_batch64.hip): the
+// descriptors, the per-tensor leverage state and
 // scratch live in one device arena; the launches run on the batch's own
 // stream, ordered after and before the optimizers' context streams.
 struct ex_batch {
@@ -1796,6 +1797,7 @@ struct ex_batch {
     int precision = 0;
     int64_t J = 0;
     int grid = 0;
+    BatchShape shape;
     DevBuf desc, ctl, arena;
     unsigned long long first_sweep = 1;  // host source of the sweep reset
     bool use_graph = false;
@@ -1898,9 +1900,10 @@ int ex_batch_create(ex_als* const* als, int n, int64_t J, ex_batch** out) {
         auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
         struct Plan {
             size_t samples, weights, sd, kd, wd, dg, dm, Yc, hu, hstamp, rstamp, cnt, ssum, stats;
+            size_t skey, ju, gpart, npart, gi, Uc;   // FP64
             size_t list[kMaxModes], csc[kMaxModes], ccdf[kMaxModes], rowptr[kMaxModes];
         };
-        std::vector<Plan> plan((size_t)n);
+        std::vector<Plan> plan((size_t)n, Plan{});
         size_t off = 0;
         auto take = [&](size_t bytes) {
             const size_t o = off;
@@ -1920,7 +1923,7 @@ int ex_batch_create(ex_als* const* als, int n, int64_t J, ex_batch** out) {
             P.kd = take((size_t)J * 8);
             P.wd = take((size_t)J * 8);
             P.dg = take((size_t)J * R * vb);
-            P.dm = take((size_t)J * R * vb);
+            if (mixed) P.dm = take((size_t)J * R * vb);
             P.Yc = take((size_t)Imax * R * vb);
             P.hu = take(nnz * 4);
             P.hstamp = take(nnz * 4);
@@ -1928,6 +1931,18 @@ int ex_batch_create(ex_als* const* als, int n, int64_t J, ex_batch** out) {
             P.cnt = take(kMaxModes * 4);
             P.ssum = take(kMaxModes * 8);
             P.stats = take(24);
+            if (!mixed) {
+                P.skey = take((size_t)J * 8);
+                P.ju = take(4);
+                P.gpart = take(kBatchGramPart * 8);
+                P.npart = take(kBatchNormPart * 8);
+                P.gi = take((size_t)R * R * 8);
+                P.Uc = take((size_t)Imax * R * 8);
+            }
+            b->shape.N_max = std::max(b->shape.N_max, N);
+            b->shape.R_min = std::min(b->shape.R_min, R);
+            b->shape.R_max = std::max(b->shape.R_max, R);
+            b->shape.I_max = std::max(b->shape.I_max, Imax);
             for (int k2 = 0; k2 < N; k2++) {
                 P.list[k2] = take((size_t)a->f->dims[k2] * 4);
                 P.csc[k2] = take((size_t)a->f->dims[k2] * 8);
@@ -1980,11 +1995,19 @@ int ex_batch_create(ex_als* const* als, int n, int64_t J, ex_batch** out) {
             T.kd = reinterpret_cast<uint64_t*>(base + P.kd);
             T.wd = reinterpret_cast<double*>(base + P.wd);
             T.dg = base + P.dg;
-            T.dm = base + P.dm;
+            if (mixed) T.dm = base + P.dm;
             T.Yc = base + P.Yc;
             T.hu = reinterpret_cast<uint32_t*>(base + P.hu);
             T.hstamp = reinterpret_cast<uint32_t*>(base + P.hstamp);
             T.rstamp = reinterpret_cast<uint32_t*>(base + P.rstamp);
+            if (!mixed) {
+                T.skey = reinterpret_cast<uint64_t*>(base + P.skey);
+                T.ju = reinterpret_cast<uint32_t*>(base + P.ju);
+                T.gpart = reinterpret_cast<double*>(base + P.gpart);
+                T.npart = reinterpret_cast<double*>(base + P.npart);
+                T.gi = reinterpret_cast<double*>(base + P.gi);
+                T.Uc = reinterpret_cast<double*>(base + P.Uc);
+            }
             b->stats_off[(size_t)t] = P.stats;
         }
         // the sampler state (every row listed) after the context streams' work
@@ -2039,12 +2062,15 @@ int ex_batch_run(ex_batch* b, int64_t rounds, double* seconds) {
         // sweeps are numbered from 1 in every run, as ex_als_run numbers them
         EX_HIP(hipMemcpyAsync(b->ctl.p, &b->first_sweep, sizeof(b->first_sweep), hipMemcpyHostToDevice,
                               b->stream));
-        const int vb = b->precision == EX_MIXED ? 4 : 8;
-        BatchTensor* desc = b->desc.as<BatchTensor>();
-        BatchCtl* ctl = b->ctl.as<BatchCtl>();
+        auto sweep = [&] {
+            BatchTensor* desc = b->desc.as<BatchTensor>();
+            BatchCtl* ctl = b->ctl.as<BatchCtl>();
+            if (b->precision == EX_MIXED) k::batch_sweep32(b->stream, desc, n, b->J, ctl, b->grid);
+            else k::batch_sweep64(b->stream, desc, n, b->J, ctl, b->shape);
+        };
         if (b->use_graph && !b->gexec && rounds > 0) {
             EX_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            k::batch_sweep(b->stream, desc, n, b->J, ctl, b->grid, vb);
+            sweep();
             EX_HIP(hipStreamEndCapture(b->stream, &b->graph));
             EX_HIP(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
         }
@@ -2052,7 +2078,7 @@ int ex_batch_run(ex_batch* b, int64_t rounds, double* seconds) {
         auto t0 = std::chrono::steady_clock::now();
         for (int64_t r = 0; r < rounds; r++) {
             if (b->gexec) EX_HIP(hipGraphLaunch(b->gexec, b->stream));
-            else k::batch_sweep(b->stream, desc, n, b->J, ctl, b->grid, vb);
+            else sweep();
         }
         EX_HIP(hipStreamSynchronize(b->stream));
         if (seconds) *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

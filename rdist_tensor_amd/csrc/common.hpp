@@ -370,8 +370,7 @@ int tune_value(int knob);
 void tune_select(int knob, int value);
 
 // ---------------------------------------------------------------- batched sweeps
-// Device descriptors of the batched CP-ARLS-LEV sweep (one workgroup runs
-// whole tensors).  V = float (mixed precision) or double (FP64) for factor
+// Device descriptors of the batched CP-ARLS-LEV sweep.  V = float (mixed precision) or double (FP64) for factor
 // rows, nonzero values, design rows and MTTKRP rows.
 constexpr int kBatchMaxRank = 32;
 constexpr int kBatchMaxJ = 8192;
@@ -408,30 +407,46 @@ struct BatchTensor {
     double* weights;          // J
     uint32_t* sd;             // J x N unique tuples, first-occurrence order
     uint64_t* kd;             // J their fiber keys
-    double* wd;               // J weight x multiplicity
+    double* wd;               // J weight x multiplicity (FP64: its square root)
     void* dg;                 // V[J x R] design rows (Gram)
-    void* dm;                 // V[J x R] design rows (MTTKRP)
+    void* dm;                 // V[J x R] design rows (MTTKRP; mixed only)
     void* Yc;                 // V[Imax x R] MTTKRP rows of the listed rows
     uint32_t* hu;             // nnz: design row of a hit position
     uint32_t* hstamp;         // nnz: step stamp of a hit position
     uint32_t* rstamp;         // Imax: step stamp of a hit row
+    // FP64 sweeps only (null otherwise)
+    uint64_t* skey;           // J: fiber keys of the samples
+    uint32_t* ju;             // number of unique samples
+    double* gpart;            // Gram sums of row groups (kBatchGramPart)
+    double* npart;            // kBatchNormPart: column-norm sums of row classes
+    double* gi;               // R x R pseudo-inverse
+    double* Uc;               // Imax x R: updated listed rows before normalisation
 };
+// 256 / ceil(R/2)^2 x 4 groups (at most 256) of R x R sums; 1024 / R classes of R
+constexpr int kBatchGramPart = 4096, kBatchNormPart = 1024;
 
-// Read by every workgroup at launch start; the last workgroup to finish
-// advances sweep and epoch and resets the queue.
+// Read by every workgroup of a sweep, whose end advances sweep and epoch (and,
+// on the mixed path, resets the queue).
 struct BatchCtl {
-    unsigned long long sweep;  // keys the draws of the launch
-    unsigned int epoch;        // launches since creation (step stamps)
+    unsigned long long sweep;  // keys the draws of the sweep
+    unsigned int epoch;        // sweeps since creation (step stamps)
     unsigned int next;         // tensor queue
     unsigned int done;         // finished workgroups
     unsigned int pad;
 };
 
+// Extremes over a batch, for the grids of the FP64 sweep.
+struct BatchShape {
+    int N_max = 0, R_min = kBatchMaxRank, R_max = 0;
+    int64_t I_max = 1;
+};
+
 namespace k {
 // list = iota and rowptr for every mode of every tensor
 void batch_init(hipStream_t s, const BatchTensor* ts, int n);
-// one sweep of every tensor (grid workgroups); vbytes 4 (mixed) or 8 (FP64)
-void batch_sweep(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, int grid, int vbytes);
+// one sweep of every tensor: mixed precision (grid workgroups), FP64
+void batch_sweep32(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, int grid);
+void batch_sweep64(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, const BatchShape& shape);
 }  // namespace k
 
 inline unsigned grid_for(int64_t work, int per_block, int64_t cap = 1 << 20) {

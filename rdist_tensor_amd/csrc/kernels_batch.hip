@@ -1,5 +1,5 @@
-// Batched CP-ARLS-LEV: one launch runs one ALS sweep of every tensor of a
-// batch.  A workgroup of 1024 threads takes whole tensors from a queue and
+// Batched CP-ARLS-LEV, mixed precision (FP64: kernels_batch64.hip): one launch
+// runs one ALS sweep of every tensor of a batch.  A workgroup of 1024 threads takes whole tensors from a queue and
 // runs each mode step of AccumulatorStationary::execute_ALS_step
 // (accumulator_stationary.hpp:139-295) with CP-ARLS-LEV as the sampler
 // (cp_arls_lev.hpp:25-163) as a chain of workgroup-level phases separated by
@@ -20,39 +20,25 @@
 //
 // LDS: a 96 KiB region shared by the phases (the deduplication table; Gram
 // staging, the R x R solver's scratch, Y^T Y) and three R x R matrices.
-#include "common.hpp"
-#include "device.hpp"
-#include "jacobi_block.hpp"
+#include "batch_block.hpp"
 #include "spd_block.hpp"
 
 namespace exafac {
 namespace {
 
-constexpr int kBT = 1024;                        // threads per workgroup
-constexpr int kWaves = kBT / 64;
-constexpr int kTableBits = 14;                   // deduplication slots: 2^14 >= 2 kBatchMaxJ
-constexpr int kMaxQ = kBatchMaxJ / kBT;          // samples per thread at the largest J
-constexpr int kLane = 8;                         // binary searches in flight per thread
-constexpr int kChunk = 8;                        // entries per thread of a scan pass
 constexpr int kBigBytes = 96 << 10;              // 96 KiB
-constexpr int kRR = kBatchMaxRank * kBatchMaxRank;
-static_assert(kBatchMaxJ * 2 <= (1 << kTableBits), "deduplication table load above 1/2");
-static_assert(kBatchMaxJ < (1 << 16), "table entries pack a 16-bit index and a 16-bit count");
 
 // offsets in the shared region (bytes) of the phases that run after the
 // deduplication
 constexpr int kGramRows = 256;                   // rows per staged Gram chunk
 constexpr int kOffStage = 0;                     // Gram staging: kGramRows x R doubles (64 KiB)
-constexpr int kOffPart = 64 << 10;               // column-norm partials (FP64 update): 1024 doubles
-constexpr int kOffSolve = 24 << 10;              // R x R solver scratch (SpdShared + perm, or EighShared)
+constexpr int kOffPart = 64 << 10;               // end of the staging area
+constexpr int kOffSolve = 24 << 10;              // R x R solver scratch (SpdShared + perm)
 constexpr int kOffGY = 80 << 10;                 // Y^T Y (R x R doubles)
 constexpr int kOffTmp = 88 << 10;                // R x R temporary
 static_assert(kOffSolve + (int)sizeof(SpdShared) + 128 <= kOffGY, "solver scratch overlaps Y^T Y");
-static_assert(kOffSolve + (int)sizeof(EighSharedT<kBatchMaxRank>) <= kOffGY, "solver scratch overlaps Y^T Y");
-static_assert(kBT >= kJacobiThreads, "the Jacobi solver needs kJacobiThreads threads");
 static_assert(kOffTmp + kRR * 8 <= kBigBytes, "shared region too small");
 static_assert(kOffStage + kGramRows * kBatchMaxRank * 8 <= kOffPart, "Gram staging overlaps its partials");
-static_assert(kOffPart + kRR * 8 <= kOffGY, "partials overlap Y^T Y");
 // block_gram's partials: 1024 / ceil(R/2)^2 groups of R^2 doubles, at most
 // 4 * R^2 * 8 (R even) or about that (R odd) -- within the staging area
 static_assert(4 * kRR * 8 <= kOffPart - kOffStage, "Gram partials do not fit the staging area");
@@ -67,89 +53,6 @@ struct Lds {
     uint32_t* wsu;  // kWaves
     double* wsd;    // kWaves
 };
-
-__device__ __forceinline__ uint64_t pack_key(const uint32_t* c, int N, const int* shift) {
-    uint64_t key = 0;
-    for (int k = 0; k < N; k++)
-        if (shift[k] >= 0) key |= (uint64_t)c[k] << shift[k];
-    return key;
-}
-
-__device__ __forceinline__ uint32_t table_slot(uint64_t key) {
-    return (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> (64 - kTableBits));
-}
-
-// Exclusive prefix over the workgroup (thread order) of one value per
-// thread; *total receives the sum.  Two barriers.
-__device__ uint32_t block_exscan_u32(uint32_t x, uint32_t* ws, uint32_t& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t inc = x;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(inc, d, 64);
-        if (lane >= d) inc += y;
-    }
-    if (lane == 63) ws[w] = inc;
-    __syncthreads();
-    uint32_t off = 0, tot = 0;
-#pragma unroll
-    for (int q = 0; q < kWaves; q++) {
-        const uint32_t v = ws[q];
-        off += q < w ? v : 0u;
-        tot += v;
-    }
-    __syncthreads();
-    total = tot;
-    return off + inc - x;
-}
-
-__device__ double block_exscan_f64(double x, double* ws, double& total) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const double inc = wave_inclusive_scan(x, lane);
-    if (lane == 63) ws[w] = inc;
-    __syncthreads();
-    double off = 0.0, tot = 0.0;
-#pragma unroll
-    for (int q = 0; q < kWaves; q++) {
-        const double v = ws[q];
-        if (q < w) off += v;
-        tot += v;
-    }
-    __syncthreads();
-    total = tot;
-    return off + (inc - x);
-}
-
-// Sum over the workgroup, waves added in order (every thread gets it).
-__device__ double block_sum_f64(double x, double* ws) {
-    const double s = wave_sum(x);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = s;
-    __syncthreads();
-    double tot = 0.0;
-#pragma unroll
-    for (int q = 0; q < kWaves; q++) tot += ws[q];
-    __syncthreads();
-    return tot;
-}
-
-// lower_bound of u in the ascending array a[0, n) for kLane searches at
-// once (every search takes ceil(log2 n) steps, their loads in flight
-// together).  Result n when every entry is below u.
-template <typename K>
-__device__ __forceinline__ void lower_bounds(const K* __restrict__ a, uint32_t n, const K (&u)[kLane],
-                                             uint32_t (&b)[kLane]) {
-#pragma unroll
-    for (int q = 0; q < kLane; q++) b[q] = 0;
-    if (n == 0) return;
-    for (uint32_t len = n; len > 1;) {
-        const uint32_t half = len >> 1;
-#pragma unroll
-        for (int q = 0; q < kLane; q++) b[q] += a[b[q] + half - 1] < u[q] ? half : 0u;
-        len -= half;
-    }
-#pragma unroll
-    for (int q = 0; q < kLane; q++) b[q] += a[b[q]] < u[q] ? 1u : 0u;
-}
 
 // ---------------------------------------------------------------- phases
 // Draws (cp_arls_lev.hpp:36-163 with the row CDFs of the other modes):
@@ -393,26 +296,6 @@ __device__ void block_spd_pinv(const double* M, int R, double tol_rel, double* o
     __syncthreads();
 }
 
-// compute_pinv_square (common.h:405-443) as the FP64 path computes it: cyclic
-// Jacobi eigendecomposition, eigenvalues <= tol (absolute) dropped.
-__device__ void block_pinv_jacobi(const double* M, int R, double tol, double* out, const Lds& s) {
-    EighSharedT<kBatchMaxRank>& sh = *reinterpret_cast<EighSharedT<kBatchMaxRank>*>(s.big + kOffSolve);
-    load_upper(M, R, sh.A);
-    jacobi_block<kBatchMaxRank>(sh.A, sh.A2, sh.V, R, sh.j);
-    pinv_from_jacobi(sh, R, tol, out);
-    __syncthreads();
-}
-
-// The R x R solves of a mode step: FP64 as the FP64 optimizer solves them
-// (Jacobi pseudo-inverse, absolute tolerance 1e-11), mixed as the mixed one
-// (Gauss-Jordan / pivoted-Cholesky pseudo-inverse, tolerance 1e-11 relative
-// to the largest diagonal entry).
-template <typename V>
-__device__ void block_solve(const double* M, int R, double* out, const Lds& s) {
-    if constexpr (sizeof(V) == 8) block_pinv_jacobi(M, R, 1e-11, out, s);
-    else block_spd_pinv(M, R, 1e-11, out, s);
-}
-
 // Sampled MTTKRP, part 1: find each unique sample's fiber (binary search of
 // its key in the sorted fiber keys) and stamp the fiber's nonzeros (row-order
 // positions: design row, step stamp) and their rows.  Returns the hits of
@@ -591,44 +474,6 @@ __device__ void update_phase(const BatchTensor& T, int j, uint32_t L, const Lds&
     __syncthreads();
 }
 
-// Factor update as the FP64 optimizer performs it (accumulator_stationary.hpp:
-// 280-289): U_j rows = Y Gi on the listed rows, sigma_c = their column norms,
-// U_j /= sigma; then the sampler's Gram U_j^T U_j over the listed rows (the
-// others are zero) into s.G.
-__device__ void update_fp64_phase(const BatchTensor& T, int j, uint32_t L, const Lds& s) {
-    const int R = T.R;
-    const int rows = kBT / R, rl = threadIdx.x / R, r = threadIdx.x - rl * R;
-    const double* Y = static_cast<const double*>(T.Yc);
-    double* U = static_cast<double*>(T.m[j].U);
-    const uint32_t* lst = T.m[j].list;
-    double* part = reinterpret_cast<double*>(s.big + kOffPart);
-    double ss = 0.0;
-    if (rl < rows)
-        for (uint32_t q = rl; q < L; q += rows) {
-            double acc = 0.0;
-            for (int b = 0; b < R; b++) acc += Y[(int64_t)q * R + b] * s.Gi[b * R + r];
-            U[(int64_t)lst[q] * R + r] = acc;
-            ss += acc * acc;
-        }
-    part[threadIdx.x] = ss;
-    __syncthreads();
-    if (threadIdx.x < R) {
-        double t = 0.0;
-        for (int g = 0; g < rows; g++) t += part[g * R + threadIdx.x];
-        const double sg = sqrt(t);
-        T.sigma[threadIdx.x] = sg;
-        s.sig[threadIdx.x] = sg;
-    }
-    __syncthreads();
-    if (rl < rows)
-        for (uint32_t q = rl; q < L; q += rows) {
-            double* u = U + (int64_t)lst[q] * R + r;
-            *u = *u / s.sig[r];
-        }
-    __syncthreads();
-    block_gram<double>(U, lst, L, R, s.G, s);
-}
-
 // Sampler update (cp_arls_lev.hpp:25-34): Gp = pinv(U_j^T U_j) (in s.Gi),
 // score of each listed row u^T Gp u (FP64 from V rows; the row's lanes hold
 // one entry each, t_c = sum_b u_b Gp[b][c] over broadcasts, then a butterfly
@@ -689,18 +534,14 @@ __device__ void mode_step(const BatchTensor& T, int j, int64_t J, uint64_t sweep
     const uint32_t Ju = dedup_phase(T, j, J, s);
     design_phase<V>(T, j, Ju);
     block_gram<V>(static_cast<const V*>(T.dg), nullptr, Ju, R, s.G, s);
-    block_solve<V>(s.G, R, s.Gi, s);
+    block_spd_pinv(s.G, R, 1e-11, s.Gi, s);
     const uint64_t hits = hits_phase(T, j, Ju, stamp);
     clear_rows_phase<V>(T, j);
     const uint32_t L = list_phase(T, j, stamp, s);
     y_phase<V>(T, j, L, stamp);
-    if constexpr (sizeof(V) == 8) {
-        update_fp64_phase(T, j, L, s);
-    } else {
-        block_gram<V>(static_cast<const V*>(T.Yc), nullptr, L, R, reinterpret_cast<double*>(s.big + kOffGY), s);
-        update_phase<V>(T, j, L, s);
-    }
-    block_solve<V>(s.G, R, s.Gi, s);
+    block_gram<V>(static_cast<const V*>(T.Yc), nullptr, L, R, reinterpret_cast<double*>(s.big + kOffGY), s);
+    update_phase<V>(T, j, L, s);
+    block_spd_pinv(s.G, R, 1e-11, s.Gi, s);
     scores_phase<V>(T, j, L, s);
     const double h = block_sum_f64((double)hits, s.wsd);
     if (threadIdx.x == 0) {
@@ -772,13 +613,10 @@ void batch_init(hipStream_t s, const BatchTensor* ts, int n) {
     EX_HIP(hipGetLastError());
 }
 
-void batch_sweep(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, int grid, int vbytes) {
+void batch_sweep32(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, int grid) {
     EX_CHECK(J >= 1 && J <= kBatchMaxJ, 1, "batched sweep: J out of range");
     EX_CHECK(grid >= 1, 1, "batched sweep: empty grid");
-    if (vbytes == 4)
-        hipLaunchKernelGGL(batch_sweep_kernel<float>, dim3((unsigned)grid), dim3(kBT), 0, s, ts, n, J, ctl);
-    else
-        hipLaunchKernelGGL(batch_sweep_kernel<double>, dim3((unsigned)grid), dim3(kBT), 0, s, ts, n, J, ctl);
+    hipLaunchKernelGGL(batch_sweep_kernel<float>, dim3((unsigned)grid), dim3(kBT), 0, s, ts, n, J, ctl);
     EX_HIP(hipGetLastError());
 }
 
