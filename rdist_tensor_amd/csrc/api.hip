@@ -761,8 +761,7 @@ void als_step_impl(ex_als* a, int j, int64_t J, uint64_t sweep) {
     } else {
         double* Uj = f->U[j].as<double>();
         k::dsymm(st, a->Gi.as<double>(), a->Y.as<double>(), Ij, R, Uj);
-        k::col_sumsq(st, Uj, Ij, R, f->sigma.as<double>(), a->part);
-        k::scale_cols(st, Uj, Ij, R, f->sigma.as<double>());
+        k::normalize_cols(st, Uj, Ij, R, f->sigma.as<double>(), a->part);
         f->wrote64(j);
     }
     s_fu.end();
@@ -980,8 +979,7 @@ void exact_step_impl(ex_als* a, int j) {
     } else {
         double* Uj = f->U[j].as<double>();
         k::dsymm(st, a->Gi.as<double>(), a->Y.as<double>(), Ij, R, Uj);
-        k::col_sumsq(st, Uj, Ij, R, f->sigma.as<double>(), a->part);
-        k::scale_cols(st, Uj, Ij, R, f->sigma.as<double>());
+        k::normalize_cols(st, Uj, Ij, R, f->sigma.as<double>(), a->part);
         f->wrote64(j);
     }
     s_fu.end();
@@ -1439,8 +1437,7 @@ int ex_factors_renormalize(ex_factors* f, int mode, double* sigma) {
         DevBuf sg;
         sg.ensure((size_t)f->R * 8);
         f->sync64(mode);
-        k::col_sumsq(st, f->U[mode].as<double>(), f->dims[mode], f->R, sg.as<double>(), f->part);
-        k::scale_cols(st, f->U[mode].as<double>(), f->dims[mode], f->R, sg.as<double>());
+        k::normalize_cols(st, f->U[mode].as<double>(), f->dims[mode], f->R, sg.as<double>(), f->part);
         f->wrote64(mode);
         if (sigma) d2h(st, sigma, sg.p, (size_t)f->R * 8);
         EX_HIP(hipStreamSynchronize(st));
@@ -1455,8 +1452,7 @@ int ex_factors_init_deterministic(ex_factors* f) {
         sg.ensure((size_t)f->R * 8);
         for (int k2 = 0; k2 < f->N; k2++) {
             k::cos_init(st, f->U[k2].as<double>(), f->dims[k2], f->R);
-            k::col_sumsq(st, f->U[k2].as<double>(), f->dims[k2], f->R, sg.as<double>(), f->part);
-            k::scale_cols(st, f->U[k2].as<double>(), f->dims[k2], f->R, sg.as<double>());
+            k::normalize_cols(st, f->U[k2].as<double>(), f->dims[k2], f->R, sg.as<double>(), f->part);
             f->wrote64(k2);
         }
         std::vector<double> ones(f->R, 1.0);

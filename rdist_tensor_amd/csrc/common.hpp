@@ -172,8 +172,8 @@ void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int nc
           const int* only_if = nullptr, bool relative = false, bool two_sided = false);
 void dagat(hipStream_t s, const double* A, int64_t m, int R, const double* G, double* res);
 void dsymm(hipStream_t s, const double* G, const double* Y, int64_t m, int R, double* out);
-void col_sumsq(hipStream_t s, const double* U, int64_t m, int R, double* sigma, DevBuf& part);
-void scale_cols(hipStream_t s, double* U, int64_t m, int R, const double* sigma);
+// sigma_c = the column norms of U, U /= sigma
+void normalize_cols(hipStream_t s, double* U, int64_t m, int R, double* sigma, DevBuf& part);
 void cos_init(hipStream_t s, double* U, int64_t m, int R);
 void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out);
 // out = elementwise product of grams[k] (k != exclude), k ascending
@@ -182,6 +182,7 @@ void chain_had(hipStream_t s, const double* grams, int N, int exclude, int R, do
 void preprocess(hipStream_t s, double* vals, int64_t nnz, int kind);
 void sumsq(hipStream_t s, const double* v, int64_t n, double* out, DevBuf& part);
 void plain_sum(hipStream_t s, const double* v, int64_t n, double* out, DevBuf& part);
+int plain_sum_blocks(int64_t n);   // pieces that it adds up in order
 // ARLS
 void arls_cdf(hipStream_t s, const double* scores, int64_t I, double* cdf, double* sum, DevBuf& part);
 void arls_draw(hipStream_t s, int N, int j, int64_t J, const double* const* cdfs, const double* const* scores,

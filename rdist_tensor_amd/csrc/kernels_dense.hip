@@ -406,25 +406,51 @@ __global__ __launch_bounds__(kThreads) void eig_tree_kernel(int N, int j, int R,
     for (int c = grp; c < nodes; c += ngrp) out[(int64_t)c * S + e] = (TO)(T[c * kEigCols + col] * g);
 }
 
-// ---------------------------------------------------------------- row-wise
-// res_i = a_i^T G a_i, G symmetric (full storage).  One thread per row.
-__global__ __launch_bounds__(kThreads) void dagat_kernel(const double* __restrict__ A, int64_t m, int R,
+// res_i = u_i^T G u_i: sum_c u_c (sum_b u_b G[b][c]), each sum in order, in FP64
+// (TA = float: rows of the mixed path, converted exactly).  One thread per row,
+// which holds it in registers and takes four columns of G at a time (LDS, every
+// lane the same address): four independent chains, and no load in the inner
+// loop but G's.  RMAX is R rounded up to 8, the columns past R are zero; rows of
+// short modes are spread over 64-thread workgroups.  2000 rows, R = 16: 36 ->
+// 5.7 us (one column at a time, the row read again for each).
+template <typename TA, int RMAX>
+__global__ __launch_bounds__(kThreads) void dagat_kernel(const TA* __restrict__ A, int64_t m, int R,
                                                          const double* __restrict__ G, double* __restrict__ res) {
-    __shared__ double g[kMaxRank * kMaxRank];
-    for (int e = threadIdx.x; e < R * R; e += blockDim.x) g[e] = G[e];
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double g[RMAX * RMAX];
+    for (int e = threadIdx.x; e < RMAX * RMAX; e += blockDim.x) {
+        const int b = e / RMAX, c = e % RMAX;
+        g[e] = b < R && c < R ? G[b * R + c] : 0.0;
+    }
     __syncthreads();
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const double* a = A + i * R;
+        const TA* a = A + i * R;
+        double u[RMAX];
+#pragma unroll
+        for (int b = 0; b < RMAX; b++) u[b] = (double)a[b < R ? b : 0];
+#pragma unroll
+        for (int b = 0; b < RMAX; b++) u[b] = b < R ? u[b] : 0.0;
         double r = 0.0;
-        for (int c = 0; c < R; c++) {
-            double t = 0.0;
-            for (int b = 0; b < R; b++) t += a[b] * g[b * R + c];
-            r += a[c] * t;
+        for (int c = 0; c < R; c += 4) {
+            double uc[4], t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < 4; q++) uc[q] = (double)a[c + q < R ? c + q : 0];
+#pragma unroll
+            for (int b = 0; b < RMAX; b++) {
+                const d2 x = *reinterpret_cast<const d2*>(g + b * RMAX + c);
+                const d2 y = *reinterpret_cast<const d2*>(g + b * RMAX + c + 2);
+                t[0] += u[b] * x[0];
+                t[1] += u[b] * x[1];
+                t[2] += u[b] * y[0];
+                t[3] += u[b] * y[1];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (c + q < R) r += uc[q] * t[q];
         }
         res[i] = r;
     }
 }
-
 
 // Column sums of squares, stage 1: part[block][c].
 __global__ __launch_bounds__(kThreads) void col_sumsq_partial(const double* __restrict__ U, int64_t m, int R,
@@ -437,8 +463,17 @@ __global__ __launch_bounds__(kThreads) void col_sumsq_partial(const double* __re
         const int64_t rows_per_block = (m + gridDim.x - 1) / gridDim.x;
         const int64_t r0 = blockIdx.x * rows_per_block;
         const int64_t r1 = r0 + rows_per_block < m ? r0 + rows_per_block : m;
-        for (int64_t i = r0 + rl; i < r1; i += lanes) {
-            double v = U[i * R + c];
+        // eight rows in flight, added in order (2000 rows, R = 16: 17 -> 6.5 us)
+        int64_t i = r0 + rl;
+        for (; i + 7 * lanes < r1; i += 8 * lanes) {
+            double v[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) v[q] = U[(i + q * lanes) * R + c];
+#pragma unroll
+            for (int q = 0; q < 8; q++) acc += v[q] * v[q];
+        }
+        for (; i < r1; i += lanes) {
+            const double v = U[i * R + c];
             acc += v * v;
         }
     }
@@ -464,11 +499,35 @@ __global__ __launch_bounds__(kThreads) void col_sumsq_final(const double* __rest
     if (lane == 0) sigma[c] = sqrt(s);
 }
 
+// U /= sigma by columns.  With few partials (part, at most kScaleParts of them)
+// every workgroup adds them up itself, as col_sumsq_final does, and the first one
+// writes sigma: a launch less, which is most of the time for short modes.
+constexpr int kScaleParts = 16;
 __global__ __launch_bounds__(kThreads) void scale_cols_kernel(double* __restrict__ U, int64_t m, int R,
-                                                              const double* __restrict__ sigma) {
+                                                              double* __restrict__ sigma,
+                                                              const double* __restrict__ part, int nparts) {
+    __shared__ double sg[kMaxRank];
+    if (threadIdx.x < R) {
+        double s;
+        if (part) {
+            double v[kScaleParts];   // the lanes of that kernel's butterfly; the others hold zero
+#pragma unroll
+            for (int p = 0; p < kScaleParts; p++) v[p] = p < nparts ? part[(int64_t)p * R + threadIdx.x] : 0.0;
+#pragma unroll
+            for (int off = kScaleParts / 2; off >= 1; off >>= 1)
+#pragma unroll
+                for (int p = 0; p < off; p++) v[p] += v[p + off];
+            s = sqrt(v[0]);
+            if (blockIdx.x == 0) sigma[threadIdx.x] = s;
+        } else {
+            s = sigma[threadIdx.x];
+        }
+        sg[threadIdx.x] = s;
+    }
+    __syncthreads();
     const RowMap rm(R);
     if (!rm.on()) return;
-    const double sc = sigma[rm.c];
+    const double sc = sg[rm.c];
     for (int64_t i = rm.first(); i < m; i += rm.step()) U[i * R + rm.c] = U[i * R + rm.c] / sc;
 }
 
@@ -631,8 +690,6 @@ void col_sumsq_final_launch(hipStream_t s, const double* part, int nb, int R, do
     EX_HIP(hipGetLastError());
 }
 
-// Jacobi work per thread: (2x2 blocks, V rows) = (1, 2) for R <= 32, (3, 8)
-// for R <= 64.
 // The R x R solves, sized to the rank: 16, 32 or 64.
 #define PSD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                                     \
     do {                                                                                                              \
@@ -652,25 +709,46 @@ void pinv(hipStream_t s, const double* M, int R, double tol, double* out, int nc
     EX_HIP(hipGetLastError());
 }
 
-void dagat(hipStream_t s, const double* A, int64_t m, int R, const double* G, double* res) {
-    hipLaunchKernelGGL(dagat_kernel, dim3(grid_for(m, kThreads, 4096)), dim3(kThreads), 0, s, A, m, R, G, res);
+template <typename TA>
+void dagat_rows(hipStream_t s, const TA* A, int64_t m, int R, const double* G, double* res) {
+    const int threads = m < 65536 ? 64 : kThreads;
+    const dim3 grid(grid_for(m, threads, 4096));
+#define DAGAT(K) \
+    case K: hipLaunchKernelGGL((dagat_kernel<TA, 8 * K>), grid, dim3(threads), 0, s, A, m, R, G, res); break
+    switch ((R + 7) / 8) {
+        DAGAT(1);
+        DAGAT(2);
+        DAGAT(3);
+        DAGAT(4);
+        DAGAT(5);
+        DAGAT(6);
+        DAGAT(7);
+        DAGAT(8);
+        default: EX_CHECK(false, 1, "rank out of range");
+    }
+#undef DAGAT
     EX_HIP(hipGetLastError());
+}
+
+void dagat(hipStream_t s, const double* A, int64_t m, int R, const double* G, double* res) {
+    dagat_rows<double>(s, A, m, R, G, res);
+}
+
+void dagat32(hipStream_t s, const float* A, int64_t m, int R, const double* G, double* res) {
+    dagat_rows<float>(s, A, m, R, G, res);
 }
 
 void dsymm(hipStream_t s, const double* G, const double* Y, int64_t m, int R, double* out) {
     dsymm_tile<double>(s, G, Y, m, R, out);
 }
 
-void col_sumsq(hipStream_t s, const double* U, int64_t m, int R, double* sigma, DevBuf& part) {
-    int nb = (int)grid_for(m, 1024, 1024);
+void normalize_cols(hipStream_t s, double* U, int64_t m, int R, double* sigma, DevBuf& part) {
+    const int nb = (int)grid_for(m, 1024, 1024);
     part.ensure((size_t)nb * R * sizeof(double));
     hipLaunchKernelGGL(col_sumsq_partial, dim3(nb), dim3(kThreads), 0, s, U, m, R, part.as<double>());
-    EX_HIP(hipGetLastError());
-    col_sumsq_final_launch(s, part.as<double>(), nb, R, sigma);
-}
-
-void scale_cols(hipStream_t s, double* U, int64_t m, int R, const double* sigma) {
-    hipLaunchKernelGGL(scale_cols_kernel, dim3(grid_for(m, kThreads / R, 8192)), dim3(kThreads), 0, s, U, m, R, sigma);
+    if (nb > kScaleParts) col_sumsq_final_launch(s, part.as<double>(), nb, R, sigma);
+    hipLaunchKernelGGL(scale_cols_kernel, dim3(grid_for(m, kThreads / R, 8192)), dim3(kThreads), 0, s, U, m, R, sigma,
+                       nb > kScaleParts ? nullptr : part.as<double>(), nb);
     EX_HIP(hipGetLastError());
 }
 
@@ -703,8 +781,10 @@ void sumsq(hipStream_t s, const double* v, int64_t n, double* out, DevBuf& part)
     EX_HIP(hipGetLastError());
 }
 
+int plain_sum_blocks(int64_t n) { return (int)grid_for(n, 4096, 1024); }
+
 void plain_sum(hipStream_t s, const double* v, int64_t n, double* out, DevBuf& part) {
-    int nb = (int)grid_for(n, 4096, 1024);
+    const int nb = plain_sum_blocks(n);
     part.ensure((size_t)nb * sizeof(double));
     hipLaunchKernelGGL(plainsum_partial, dim3(nb), dim3(kThreads), 0, s, v, n, part.as<double>());
     hipLaunchKernelGGL(sum_final, dim3(1), dim3(64), 0, s, part.as<double>(), nb, out);

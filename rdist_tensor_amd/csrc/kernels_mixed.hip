@@ -444,24 +444,6 @@ __global__ __launch_bounds__(kThreads) void scale_cols_f32(float* __restrict__ U
     for (int64_t i = rm.first(); i < m; i += rm.step()) U[i * R + rm.c] = (float)((double)U[i * R + rm.c] / sc);
 }
 
-// res_i = u_i^T G u_i with FP32 rows and an FP64 G, accumulated in FP64.
-__global__ __launch_bounds__(kThreads) void dagat_f32(const float* __restrict__ A, int64_t m, int R,
-                                                      const double* __restrict__ G, double* __restrict__ res) {
-    __shared__ double g[kMaxRank * kMaxRank];
-    for (int e = threadIdx.x; e < R * R; e += blockDim.x) g[e] = G[e];
-    __syncthreads();
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const float* a = A + i * R;
-        double r = 0.0;
-        for (int c = 0; c < R; c++) {
-            double t = 0.0;
-            for (int b = 0; b < R; b++) t += (double)a[b] * g[b * R + c];
-            r += (double)a[c] * t;
-        }
-        res[i] = r;
-    }
-}
-
 }  // namespace
 
 namespace k {
@@ -583,11 +565,6 @@ void renormalize32(hipStream_t s, float* U, int64_t m, int R, double* sigma, Dev
 void sigma_from_gram(hipStream_t s, const double* GY, const double* Gi, int R, double* sigma, float* Ms,
                      double* gu) {
     hipLaunchKernelGGL(sigma_from_gram_kernel, dim3(1), dim3(1024), 0, s, GY, Gi, R, sigma, Ms, gu);
-    EX_HIP(hipGetLastError());
-}
-
-void dagat32(hipStream_t s, const float* A, int64_t m, int R, const double* G, double* res) {
-    hipLaunchKernelGGL(dagat_f32, dim3(grid_for(m, kThreads, 4096)), dim3(kThreads), 0, s, A, m, R, G, res);
     EX_HIP(hipGetLastError());
 }
 

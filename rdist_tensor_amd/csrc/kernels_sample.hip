@@ -1055,6 +1055,34 @@ __global__ __launch_bounds__(kThreads) void first64_descend(k::StsFirstArgs a, c
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kThreads * kScanItems;
 
+// The chain run, run + x[0], run + x[0] + x[1], ... over the kThreads entries of x
+// (LDS) on one thread: its value past the last one, and with kWrite each entry
+// replaced by the value before it.  Sixteen loads in flight ahead of the adds (one
+// at a time, a load's latency per entry: 7 us a tile).
+template <bool kWrite>
+__device__ __forceinline__ double serial_chain(double* x, double run) {
+    constexpr int kAhead = 16;
+    double v[2][kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; q++) v[0][q] = x[q];
+    for (int i = 0; i < kThreads; i += 2 * kAhead) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int at = i + h * kAhead;
+            if (at + kAhead < kThreads)
+#pragma unroll
+                for (int q = 0; q < kAhead; q++) v[1 - h][q] = x[at + kAhead + q];
+#pragma unroll
+            for (int q = 0; q < kAhead; q++) {
+                const double t = v[h][q];
+                if (kWrite) x[at + q] = run;
+                run += t;
+            }
+        }
+    }
+    return run;
+}
+
 // p_i = s_i / sum; block partial sums of p (tile order).
 __global__ __launch_bounds__(kThreads) void cdf_tile_sums(const double* __restrict__ sc, int64_t I,
                                                           const double* __restrict__ sum, double* __restrict__ tsum) {
@@ -1068,11 +1096,7 @@ __global__ __launch_bounds__(kThreads) void cdf_tile_sums(const double* __restri
     }
     red[threadIdx.x] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int i = 0; i < kThreads; i++) t += red[i];
-        tsum[blockIdx.x] = t;
-    }
+    if (threadIdx.x == 0) tsum[blockIdx.x] = serial_chain<false>(red, 0.0);
 }
 
 // exclusive scan of tile sums (sequential, one thread)
@@ -1102,20 +1126,68 @@ __global__ __launch_bounds__(kThreads) void cdf_tile_apply(const double* __restr
     }
     pre[threadIdx.x] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = toff[blockIdx.x];
-        for (int i = 0; i < kThreads; i++) {
-            double t = pre[i];
-            pre[i] = run;
-            run += t;
-        }
-    }
+    if (threadIdx.x == 0) serial_chain<true>(pre, toff[blockIdx.x]);
     __syncthreads();
     const double off = pre[threadIdx.x];
     for (int i = 0; i < kScanItems; i++) {
         int64_t g = base + i;
         if (g < I) cdf[g] = (g == I - 1) ? 1.0 : off + loc[i];
     }
+}
+
+// The sum of the scores and their CDF on one workgroup, for at most kCdfTiles
+// tiles: what plain_sum and the three kernels above compute, in their order (the
+// sum in `sum_blocks` pieces).  2000 scores: 25 us in five launches, 7 us so.
+constexpr int kCdfTiles = 4;
+__global__ __launch_bounds__(kThreads* kCdfTiles) void cdf_small(const double* __restrict__ sc, int I, int sum_blocks,
+                                                                 double* __restrict__ sum, double* __restrict__ cdf) {
+    __shared__ double pre[kCdfTiles][kThreads];
+    __shared__ double tot[kCdfTiles];
+    const int tile = threadIdx.x / kThreads, t = threadIdx.x % kThreads;
+    const int base = tile * kScanTile + t * kScanItems;
+    double p[kScanItems];
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) p[i] = base + i < I ? sc[base + i] : 0.0;
+    {
+        const int per = (I + sum_blocks - 1) / sum_blocks;
+        const int lo = tile * per, hi = lo + per < I ? lo + per : I;
+        double acc = 0.0;
+        if (tile < sum_blocks)
+            for (int i = lo + t; i < hi; i += kThreads) acc += sc[i];
+        pre[tile][t] = acc;
+    }
+    __syncthreads();
+    for (int w = kThreads / 2; w > 0; w >>= 1) {
+        if (t < w) pre[tile][t] += pre[tile][t + w];
+        __syncthreads();
+    }
+    double S = 0.0;
+    for (int b = 0; b < sum_blocks; b++) S += pre[b][0];
+    __syncthreads();
+    if (threadIdx.x == 0) *sum = S;
+    double acc = 0.0;
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        acc += base + i < I ? p[i] / S : 0.0;
+        p[i] = acc;
+    }
+    pre[tile][t] = acc;
+    __syncthreads();
+    const int tiles = (I + kScanTile - 1) / kScanTile;
+    if (tiles > 1) {
+        if (t == 0) tot[tile] = serial_chain<false>(pre[tile], 0.0);
+        __syncthreads();
+    }
+    if (t == 0) {
+        double run = 0.0;
+        for (int b = 0; b < tile; b++) run += tot[b];
+        serial_chain<true>(pre[tile], run);
+    }
+    __syncthreads();
+    const double off = pre[tile][t];
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++)
+        if (base + i < I) cdf[base + i] = base + i == I - 1 ? 1.0 : off + p[i];
 }
 
 struct ArlsArgs {
@@ -1398,6 +1470,14 @@ void arls_cdf(hipStream_t s, const double* scores, int64_t I, double* cdf, doubl
     // sum of the scores (deterministic two-stage), then a tiled inclusive scan
     // of p = score / sum with the last entry set to 1
     const int64_t ntiles = (I + kScanTile - 1) / kScanTile;
+    if (I > 0 && ntiles <= kCdfTiles) {
+        const int sum_blocks = plain_sum_blocks(I);
+        EX_CHECK(sum_blocks <= kCdfTiles, 1, "cdf_small: more pieces than thread groups");
+        hipLaunchKernelGGL(cdf_small, dim3(1), dim3((unsigned)(kThreads * (ntiles > sum_blocks ? ntiles : sum_blocks))), 0,
+                           s, scores, (int)I, sum_blocks, sum, cdf);
+        EX_HIP(hipGetLastError());
+        return;
+    }
     plain_sum(s, scores, I, sum, part);
     DevBuf& tiles = part;  // plain_sum's partials are consumed before reuse
     tiles.ensure((size_t)(ntiles + 1) * sizeof(double));

@@ -423,12 +423,16 @@ __device__ __forceinline__ int64_t wave_find_key(const uint64_t* __restrict__ fk
     return hitmask ? lo + __ffsll((unsigned long long)hitmask) - 1 : -1;
 }
 
+// y (when given): y[0, ny) = 0 on the way, for the row pass that follows.
+template <typename V>
 __global__ __launch_bounds__(kThreads) void mark_fibers(const uint64_t* __restrict__ kd, int64_t Jb,
                                                         const uint64_t* __restrict__ Ju_dev,
                                                         const uint64_t* __restrict__ fkey, int64_t nfib,
                                                         uint64_t* __restrict__ cmap, uint32_t* __restrict__ filt,
-                                                        uint32_t* __restrict__ fsel) {
+                                                        uint32_t* __restrict__ fsel, V* __restrict__ y, int64_t ny) {
     const int64_t Ju = rows_of(Jb, Ju_dev);
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < ny; i += (int64_t)gridDim.x * blockDim.x)
+        y[i] = (V)0;
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < Ju; c += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t key = kd[c];
         // (a binary search measured faster here than 4-ary or wavefront-wide
@@ -450,13 +454,48 @@ __global__ __launch_bounds__(kThreads) void mark_fibers(const uint64_t* __restri
     }
 }
 
+// counts[0..1] += the per-workgroup partials of nb workgroups (one workgroup).
+__device__ __forceinline__ void add_counts(const unsigned long long* __restrict__ part, int nb,
+                                           uint64_t* __restrict__ counts) {
+    __shared__ unsigned long long red[2][kThreads];
+    unsigned long long h = 0, t = 0;
+    for (int b = threadIdx.x; b < nb; b += kThreads) {
+        h += part[2 * b];
+        t += part[2 * b + 1];
+    }
+    red[0][threadIdx.x] = h;
+    red[1][threadIdx.x] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kThreads; q++) {
+            h += red[0][q];
+            t += red[1][q];
+        }
+        counts[0] += h;
+        counts[1] += t;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void sum_counts(const unsigned long long* __restrict__ part, int nb,
+                                                       uint64_t* __restrict__ counts) {
+    add_counts(part, nb, counts);
+}
+
 // Every set bit belongs to this step's samples, so whole words are cleared;
-// the sampled fibers' map entries are reset too.
+// the sampled fibers' map entries are reset too.  With counts, one more workgroup
+// adds up the row pass's counters.
 __global__ __launch_bounds__(kThreads) void clear_fibers(const uint32_t* __restrict__ fsel, int64_t Jb,
                                                          const uint64_t* __restrict__ Ju_dev,
-                                                         uint32_t* __restrict__ filt, uint64_t* __restrict__ cmap) {
+                                                         uint32_t* __restrict__ filt, uint64_t* __restrict__ cmap,
+                                                         const unsigned long long* __restrict__ part, int nb,
+                                                         uint64_t* __restrict__ counts) {
     const int64_t Ju = rows_of(Jb, Ju_dev);
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < Ju; c += (int64_t)gridDim.x * blockDim.x) {
+    const unsigned blocks = gridDim.x - (counts ? 1 : 0);
+    if (blockIdx.x == blocks) {
+        add_counts(part, nb, counts);
+        return;
+    }
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < Ju; c += (int64_t)blocks * blockDim.x) {
         const uint32_t f = fsel[c];
         if (f != ~0u) {
             filt[filter_h1(f) >> 5] = 0u;
@@ -754,28 +793,6 @@ __device__ __forceinline__ void add_counts(unsigned long long whits, unsigned lo
         }
         part[2 * blockIdx.x] = h;
         part[2 * blockIdx.x + 1] = t;
-    }
-}
-
-// counts[0..1] += the per-workgroup partials of nb workgroups (one block).
-__global__ __launch_bounds__(kThreads) void sum_counts(const unsigned long long* __restrict__ part, int nb,
-                                                       uint64_t* __restrict__ counts) {
-    __shared__ unsigned long long red[2][kThreads];
-    unsigned long long h = 0, t = 0;
-    for (int b = threadIdx.x; b < nb; b += kThreads) {
-        h += part[2 * b];
-        t += part[2 * b + 1];
-    }
-    red[0][threadIdx.x] = h;
-    red[1][threadIdx.x] = t;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < kThreads; q++) {
-            h += red[0][q];
-            t += red[1][q];
-        }
-        counts[0] += h;
-        counts[1] += t;
     }
 }
 
@@ -2376,17 +2393,20 @@ template <typename V>
 void sampled_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const uint64_t* kd, int64_t Ju, const V* design,
                     int R, V* Y, int64_t I_j, DevBuf* tmp, uint64_t* counts, hipEvent_t* scan_events,
                     const uint64_t* Ju_dev, bool zero_y) {
-    if (zero_y)
+    // the row pass's first kernel clears Y itself
+    const bool any = Ju > 0 && L.nfib > 0 && L.nnz > 0;
+    const bool row_pass = any && L.mttkrp_path != 3 && !use_hit_list(L, Ju);
+    if (zero_y && !row_pass)
         hipLaunchKernelGGL(zero_fill<V>, dim3(grid_for(I_j * R, kThreads, 8192)), dim3(kThreads), 0, s, Y, I_j * R);
     if (scan_events) EX_HIP(hipEventRecord(scan_events[0], s));
-    if (Ju > 0 && L.nfib > 0 && L.nnz > 0) {
+    if (any) {
         const int64_t nch = (L.nnz + kScanChunk - 1) / kScanChunk;
         if (L.mttkrp_path == 3) {
             sampled_mttkrp_buckets<V>(s, L, vals, kd, Ju, design, R, Y, tmp, counts, Ju_dev);
             if (scan_events) EX_HIP(hipEventRecord(scan_events[1], s));
             return;
         }
-        if (use_hit_list(L, Ju)) {
+        if (!row_pass) {
             const int64_t nchb = (L.nnz + kMarkChunk - 1) / kMarkChunk;
             if (!L.marks.p) {
                 L.marks.ensure((size_t)nchb * kMarkChunk);
@@ -2454,8 +2474,10 @@ void sampled_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const uint64_t*
         V* vec;
         uint32_t *flag, *key;
         carry_views(tmp[2], 2 * nch, R, vec, flag, key);
-        hipLaunchKernelGGL(mark_fibers, dim3(grid_for(Ju, kThreads, 16384)), dim3(kThreads), 0, s, kd, Ju, Ju_dev,
-                           L.fkey.as<uint64_t>(), L.nfib, L.cmap.as<uint64_t>(), L.filt.as<uint32_t>(), fsel);
+        const int64_t ny = zero_y ? I_j * R : 0;
+        hipLaunchKernelGGL(mark_fibers<V>, dim3(std::max(grid_for(Ju, kThreads, 16384), grid_for(ny, 4 * kThreads, 4096))),
+                           dim3(kThreads), 0, s, kd, Ju, Ju_dev, L.fkey.as<uint64_t>(), L.nfib, L.cmap.as<uint64_t>(),
+                           L.filt.as<uint32_t>(), fsel, Y, ny);
         const dim3 scan_grid(grid_for(nch, kScanThreads / 64, num_cus(s)));   // one workgroup per CU (LDS)
         unsigned long long* part = count_parts(L, counts, scan_grid.x);
         with_group(scan_lanes<V>(R), [&](auto gc) {
@@ -2464,10 +2486,10 @@ void sampled_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const uint64_t*
                                L.cmap.as<uint64_t>(), L.filt.as<uint32_t>(), design, ExactSrc<V>{}, R, Y, vec, flag,
                                key, part);
         });
-        if (counts) hipLaunchKernelGGL(sum_counts, dim3(1), dim3(kThreads), 0, s, part, (int)scan_grid.x, counts);
         carry_reduce<V>(s, tmp, 2 * nch, R, Y);
-        hipLaunchKernelGGL(clear_fibers, dim3(grid_for(Ju, kThreads, 16384)), dim3(kThreads), 0, s, fsel, Ju, Ju_dev,
-                           L.filt.as<uint32_t>(), L.cmap.as<uint64_t>());
+        hipLaunchKernelGGL(clear_fibers, dim3(grid_for(Ju, kThreads, 16384) + (counts ? 1 : 0)), dim3(kThreads), 0, s,
+                           fsel, Ju, Ju_dev, L.filt.as<uint32_t>(), L.cmap.as<uint64_t>(), part, (int)scan_grid.x,
+                           counts);
     }
     if (scan_events) EX_HIP(hipEventRecord(scan_events[1], s));
     EX_HIP(hipGetLastError());
