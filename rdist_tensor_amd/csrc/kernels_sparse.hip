@@ -455,8 +455,8 @@ __global__ __launch_bounds__(kThreads) void mark_fibers(const uint64_t* __restri
 }
 
 // counts[0..1] += the per-workgroup partials of nb workgroups (one workgroup).
-__device__ __forceinline__ void add_counts(const unsigned long long* __restrict__ part, int nb,
-                                           uint64_t* __restrict__ counts) {
+__device__ __forceinline__ void total_counts(const unsigned long long* __restrict__ part, int nb,
+                                             uint64_t* __restrict__ counts) {
     __shared__ unsigned long long red[2][kThreads];
     unsigned long long h = 0, t = 0;
     for (int b = threadIdx.x; b < nb; b += kThreads) {
@@ -478,7 +478,7 @@ __device__ __forceinline__ void add_counts(const unsigned long long* __restrict_
 
 __global__ __launch_bounds__(kThreads) void sum_counts(const unsigned long long* __restrict__ part, int nb,
                                                        uint64_t* __restrict__ counts) {
-    add_counts(part, nb, counts);
+    total_counts(part, nb, counts);
 }
 
 // Every set bit belongs to this step's samples, so whole words are cleared;
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(kThreads) void clear_fibers(const uint32_t* __restr
     const int64_t Ju = rows_of(Jb, Ju_dev);
     const unsigned blocks = gridDim.x - (counts ? 1 : 0);
     if (blockIdx.x == blocks) {
-        add_counts(part, nb, counts);
+        total_counts(part, nb, counts);
         return;
     }
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < Ju; c += (int64_t)blocks * blockDim.x) {
@@ -767,10 +767,8 @@ __device__ __forceinline__ bool rows_vec(const V* p, int R) {
     return R % VW == 0 && ((uintptr_t)p % (sizeof(V) * VW)) == 0;
 }
 
-// Grouped steps whose loads are issued together (4: more cost registers;
-// the exact MTTKRP issues each mode's factor rows of all 4 at once).
-template <typename V, bool kExact>
-constexpr int step_batch() { return 4; }
+// Grouped steps whose loads are issued together (more cost registers).
+constexpr int kStepBatch = 4;
 
 // Sums each wavefront's hit and head counts per workgroup into
 // part[2 * blockIdx.x + {0, 1}] (no atomics: many workgroups adding to one
@@ -808,34 +806,214 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// kExact = false: sampled MTTKRP (hits are the nonzeros of sampled fibers,
-// rows from `design`).  kExact = true: exact MTTKRP from `ex`; the filter,
-// map and design arguments are unused.  Each chunk's hits are listed in LDS
-// in order, then summed G lanes per hit (GroupRows).
-template <typename V, bool kExact, int G>
+// Row sums over a chunk's hits (for the exact MTTKRP every position is one).  They
+// are cut into S = 64 / G runs of consecutive positions, G = ceil(R / VW)
+// lanes to a run (any G, not only powers of two), lane `sub` of a run holding
+// columns sub*VW .. sub*VW + VW - 1: a lane adds up its own columns over its run
+// with no exchange between lanes, writes the rows that begin and end inside the
+// run, and the runs' first and last rows are joined at the chunk's end, once.
+// (Taking S consecutive hits at a time, as GroupRows does, costs a segmented scan
+// over the wavefront for each S.  Exact, 3e6 nonzeros, R = 32, FP64: 206 -> 139
+// us; 1e7, R = 20, FP32: 419 -> 268; sampled, 2e7, R = 32, FP64: 222 -> 155; 5e7,
+// R = 32, FP32: 383 -> 266.)  Rows that cross a chunk's boundary go to the carry
+// list as there.  The joins are the scan of GroupRows over the runs, so up to S
+// hits are added in its order.
+//
+// AT is the type of the sums, kFused whether a product is rounded before it is
+// added.  FP32 sums of 3-256 hits are as close to the exact ones as before or
+// closer (rms 4e-8 -> 4e-8 at 20 positive terms, 9e-8 -> 5e-8 at 256); the exact
+// MTTKRP sums in FP64 (20 of the 268 us; its factors 2.0e-7 -> 1.7e-7 from those
+// in 64 bits).
+template <typename V, typename AT, int VW, int NB, bool kFused>
+struct RunRows {
+    int lane, R, G, S, g, sub;
+    bool on, vst;
+    V* Y;
+    V* carry;
+    uint32_t first_row, last_row;   // rows at the chunk's first and last positions
+    bool first_cont, continues;     // first row began before / last row runs past the chunk
+    int64_t w;
+    uint32_t heads = 0;   // rows that this lane's run (sub == 0) or lane 0 finished
+
+    __device__ void init(int lane_, int R_, int lanes, V* Y_, V* carry_) {
+        lane = lane_;
+        R = R_;
+        Y = Y_;
+        carry = carry_;
+        G = lanes;
+        S = 64 / G;
+        g = lane / G;
+        sub = lane - g * G;
+        on = g < S;
+        vst = R % VW == 0 && ((uintptr_t)Y % (sizeof(V) * VW)) == 0 && ((uintptr_t)carry % (sizeof(V) * VW)) == 0;
+    }
+    __device__ bool head_row(uint32_t r) const { return !(first_cont && r == first_row); }
+    __device__ void write(V* dst, const AT (&x)[VW]) const {
+        if (vst) {
+            typedef V VT __attribute__((ext_vector_type(VW)));
+            VT y;
+#pragma unroll
+            for (int v = 0; v < VW; v++) y[v] = (V)x[v];
+            if (sub * VW < R) *reinterpret_cast<VT*>(dst + sub * VW) = y;
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < VW; v++)
+            if (sub * VW + v < R) dst[sub * VW + v] = (V)x[v];
+    }
+    // row r's sum, written by the calling run's lanes: Y, or (false) carry slot 0
+    // for the row running in from the left
+    __device__ bool finish_row(uint32_t r, const AT (&x)[VW]) {
+        const bool head = head_row(r);
+        write(head ? Y + (int64_t)r * R : carry + (2 * w) * R, x);
+        if (head && sub == 0) heads++;
+        return head;
+    }
+    __device__ static AT mul(AT d, AT x) {
+#pragma clang fp contract(off)
+        return d * x;
+    }
+    // s + d x: one rounding (kFused), or the product's and the sum's
+    __device__ static AT mul_add(AT s, AT d, AT x) {
+        if constexpr (kFused) return s + d * x;
+        else return s + mul(d, x);
+    }
+    // hits 0 .. n - 1 (n >= 1) in row order: meta(k, row, handle, x),
+    // rows_of(handles, col0, d) the NB rows' values (columns past R are not used)
+    template <typename Meta, typename RowsOf>
+    __device__ void chunk(int n, Meta meta, RowsOf rows_of, uint32_t* cflag, uint32_t* ckey) {
+        const int q = (n + S - 1) / S;
+        const int k0 = on ? g * q : n, k1 = k0 + q < n ? k0 + q : n;
+        AT acc[VW], fsum[VW];
+        uint32_t cur = 0, frow = 0;
+        int segs = 0;   // rows of the run so far
+#pragma unroll
+        for (int v = 0; v < VW; v++) acc[v] = fsum[v] = (AT)0;
+        for (int t = 0; t < q; t += NB) {
+            uint32_t rr[NB];
+            V xx[NB];
+            uint64_t hh[NB];
+            V dd[NB][VW];
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const int k = k0 + t + b;
+                meta(k < k1 ? k : n - 1, rr[b], hh[b], xx[b]);
+            }
+            rows_of(hh, sub * VW, dd);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                const bool in = k0 + t + b < k1;
+                if (in && (segs == 0 || rr[b] != cur)) {
+                    if (segs == 1) {
+                        frow = cur;
+#pragma unroll
+                        for (int v = 0; v < VW; v++) fsum[v] = acc[v];
+                    } else if (segs > 1) {
+                        write(Y + (int64_t)cur * R, acc);
+                        heads += sub == 0 ? 1u : 0u;
+                    }
+                    segs++;
+                    cur = rr[b];
+#pragma unroll
+                    for (int v = 0; v < VW; v++) acc[v] = (AT)0;
+                }
+#pragma unroll
+                for (int v = 0; v < VW; v++) {
+                    const AT s = mul_add(acc[v], (AT)dd[b][v], (AT)xx[b]);
+                    acc[v] = in ? s : acc[v];
+                }
+            }
+        }
+        if (segs == 1) frow = cur;
+        // Join the runs.  acc becomes the sum of the run's last row up to and
+        // including this run: a segmented scan (a run of one row that is also the
+        // last row d runs before joins it; rows are sorted, so those between are
+        // of that row too).
+        for (int d = 1; d < S; d <<= 1) {
+            const int src = lane - d * G;
+            const uint32_t before = (uint32_t)__shfl((int)cur, src, 64);
+            AT po[VW];
+#pragma unroll
+            for (int v = 0; v < VW; v++) po[v] = __shfl(acc[v], src, 64);
+            if (g >= d && segs == 1 && before == frow) {
+#pragma unroll
+                for (int v = 0; v < VW; v++) acc[v] += po[v];
+            }
+        }
+        // each run writes the row that ended where it began, and its own first row
+        // if it holds more than one
+        uint32_t f0 = 0, f1 = 0;
+        const uint32_t pcur = (uint32_t)__shfl((int)cur, lane - G, 64);
+        AT pacc[VW];
+#pragma unroll
+        for (int v = 0; v < VW; v++) pacc[v] = __shfl(acc[v], lane - G, 64);
+        const bool joined = g > 0 && segs > 0 && pcur == frow;
+        const bool ends = g > 0 && segs > 0 && !joined;
+        bool odd = false;   // the row running in from the left
+        if (ends) odd = !finish_row(pcur, pacc);
+        if (segs > 1) {
+#pragma unroll
+            for (int v = 0; v < VW; v++) fsum[v] += joined ? pacc[v] : (AT)0;
+            odd |= !finish_row(frow, fsum);
+        }
+        // the last run's last row is open
+        const int last = ((n + q - 1) / q - 1) * G;
+        const uint32_t c = readlane_u32(cur, last);
+        AT a[VW];
+#pragma unroll
+        for (int v = 0; v < VW; v++) a[v] = __shfl(acc[v], last + sub, 64);
+        if (continues && c == last_row) {
+            const bool head = head_row(c);
+            if (g == 0) write(carry + (2 * w + (head ? 1 : 0)) * R, a);
+            if (head) {
+                f1 = 1;
+                heads += lane == 0 ? 1u : 0u;
+            } else {
+                f0 = 1;
+            }
+        } else if (g == 0) {
+            odd |= !finish_row(c, a);
+        }
+        if (__ballot(odd) != 0) f0 = 1;
+        close(f0, f1, cflag, ckey);
+    }
+    // (a chunk without hits leaves no partial)
+    __device__ void close(uint32_t f0, uint32_t f1, uint32_t* cflag, uint32_t* ckey) const {
+        if (lane == 0) {
+            cflag[2 * w] = f0;
+            cflag[2 * w + 1] = f1;
+            ckey[2 * w] = first_row;
+            ckey[2 * w + 1] = last_row;
+        }
+    }
+};
+
+// Sampled MTTKRP: the hits are the nonzeros of sampled fibers, their rows those
+// of `design`.  Each chunk's hits are listed in LDS in order, then summed run by run
+// (RunRows).
+template <typename V>
 __global__ __launch_bounds__(kScanThreads) void row_scan_reduce(const uint32_t* __restrict__ rrow,
                                                             const uint32_t* __restrict__ rfib,
                                                             const V* __restrict__ rval, int64_t nnz, int64_t nch,
                                                             const uint64_t* __restrict__ cmap,
                                                             const uint32_t* __restrict__ filt,
-                                                            const V* __restrict__ design, ExactSrc<V> ex, int R,
+                                                            const V* __restrict__ design, int R, int lanes,
                                                             V* __restrict__ Y, V* __restrict__ carry,
                                                             uint32_t* __restrict__ cflag, uint32_t* __restrict__ ckey,
                                                             unsigned long long* __restrict__ counts) {
     constexpr int NT = kScanThreads;
     constexpr int VW = group_vw<V>();
-    constexpr int S = 64 / G;
-    __shared__ uint32_t lfilt[kExact ? 1 : kFilterWords];
+    __shared__ uint32_t lfilt[kFilterWords];
     __shared__ uint32_t lrow[NT / 64][kScanChunk], lcol[NT / 64][kScanChunk];
     __shared__ V lval[NT / 64][kScanChunk];
-    if constexpr (!kExact) {
-        for (int i = threadIdx.x; i < kFilterWords; i += NT) lfilt[i] = filt[i];
-        __syncthreads();
-    }
+    for (int i = threadIdx.x; i < kFilterWords; i += NT) lfilt[i] = filt[i];
+    __syncthreads();
     const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
     constexpr int M = kScanChunk / 64;
-    unsigned long long whits = 0, wheads = 0;   // this wavefront's counts over its chunks
+    unsigned long long whits = 0;   // this wavefront's count over its chunks
     const int64_t step = (int64_t)gridDim.x * (NT / 64);
+    RunRows<V, V, VW, kStepBatch, sizeof(V) == 4> st;
+    st.init(lane, R, lanes, Y, carry);
     // rows and fiber numbers of the next chunk, with the rows just before
     // and after it, are loaded while the current chunk is processed
     uint32_t nrow[M], nfib[M], nprev = 0, nnext = 0;
@@ -851,57 +1029,23 @@ __global__ __launch_bounds__(kScanThreads) void row_scan_reduce(const uint32_t* 
         nprev = b2 > 0 ? rrow[b2 - 1] : 0u;
         nnext = e2 < nnz ? rrow[e2] : 0u;
     };
-    // design-row handle: the fiber key (exact) or the design row
-    auto pre_of = [ex](uint32_t c) -> uint64_t {
-        if constexpr (kExact) return ex.fkey[c];
-        else return (uint64_t)c;
-    };
-    auto rows_of = [ex, design, R](const auto& h, int col0, auto& d) {
-        constexpr int NB = sizeof(h) / sizeof(h[0]);
-        constexpr int VW = group_vw<V>();
-        if constexpr (kExact) {
-            // product of each fiber's factor rows in mode order; per mode the
-            // loads of all NB rows are issued before the first product
+    const bool vec = rows_vec<V, VW>(design, R);
+    auto rows_of = [&](const uint64_t (&h)[kStepBatch], int col0, V (&d)[kStepBatch][VW]) {
+        typedef V VT __attribute__((ext_vector_type(VW)));
 #pragma unroll
-            for (int b = 0; b < NB; b++)
+        for (int b = 0; b < kStepBatch; b++) {
+            const V* row = design + (int64_t)h[b] * R;
+            if (vec) {
+                const VT x = *reinterpret_cast<const VT*>(row + (col0 < R ? col0 : 0));
 #pragma unroll
-                for (int v = 0; v < VW; v++) d[b][v] = (V)1;
+                for (int v = 0; v < VW; v++) d[b][v] = x[v];
+            } else {
 #pragma unroll
-            for (int k = 0; k < kMaxModes; k++) {
-                if (k < ex.N && ex.shift[k] >= 0) {
-                    V u[NB][VW];
-                    int64_t off[NB];
-#pragma unroll
-                    for (int b = 0; b < NB; b++) off[b] = (int64_t)((h[b] >> ex.shift[k]) & ex.mask[k]) * R;
-                    if constexpr (sizeof(V) == 4) {
-                        rows_cols<V, VW, NB>(ex.U[k], off, col0, R, rows_vec<V, VW>(ex.U[k], R), u);
-                    } else {
-                        // FP64: element loads, column 0 in place of columns
-                        // >= R (zeroed at the end)
-#pragma unroll
-                        for (int b = 0; b < NB; b++)
-#pragma unroll
-                            for (int v = 0; v < VW; v++) u[b][v] = ex.U[k][off[b] + (col0 + v < R ? col0 + v : 0)];
-                    }
-#pragma unroll
-                    for (int b = 0; b < NB; b++)
-#pragma unroll
-                        for (int v = 0; v < VW; v++) d[b][v] *= u[b][v];
-                }
+                for (int v = 0; v < VW; v++) d[b][v] = row[col0 + v < R ? col0 + v : 0];
             }
-#pragma unroll
-            for (int b = 0; b < NB; b++)
-#pragma unroll
-                for (int v = 0; v < VW; v++)
-                    if (col0 + v >= R) d[b][v] = (V)0;
-        } else {
-            int64_t off[NB];
-#pragma unroll
-            for (int b = 0; b < NB; b++) off[b] = (int64_t)h[b] * R;
-            rows_cols<V, VW, NB>(design, off, col0, R, rows_vec<V, VW>(design, R), d);
         }
     };
-    auto meta = [&](int64_t k, uint32_t& r, uint32_t& c, V& x) {
+    auto meta = [&](int k, uint32_t& r, uint64_t& c, V& x) {
         r = lrow[wv][k];
         c = lcol[wv][k];
         x = lval[wv][k];
@@ -920,16 +1064,7 @@ __global__ __launch_bounds__(kScanThreads) void row_scan_reduce(const uint32_t* 
         }
         const uint32_t prev_row = nprev, next_row = nnext;
         if (w + step < nch) load_raw(w + step);
-        if constexpr (kExact) {
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                const int64_t i = b + 64 * m + lane;
-                hit[m] = i < e;
-                hc[m] = fr[m];
-                const V x = rval[hit[m] ? i : b];
-                hx[m] = hit[m] ? x : (V)0;
-            }
-        } else {
+        {
             // filter probes first, then every map entry and value of the
             // probe-positive nonzeros in one batch of independent loads
             bool pos[M];
@@ -963,8 +1098,7 @@ __global__ __launch_bounds__(kScanThreads) void row_scan_reduce(const uint32_t* 
                 hc[m] = (uint32_t)cm[m];
             }
         }
-        GroupRows<V, G, VW> st;
-        st.init(lane, R, w, Y, carry);
+        st.w = w;
         st.first_row = readlane_u32(hr[0], 0);
         const int last = (int)(e - 1 - b);
         st.last_row = st.first_row;
@@ -987,13 +1121,132 @@ __global__ __launch_bounds__(kScanThreads) void row_scan_reduce(const uint32_t* 
             nh += (uint32_t)__popcll(mask);
         }
         wave_lds_sync();
-        if (nh > 0) st.template run<step_batch<V, kExact>()>(0, nh, meta, pre_of, rows_of);
-        st.finish(cflag, ckey);
+        if (nh > 0) st.chunk((int)nh, meta, rows_of, cflag, ckey);
+        else st.close(0u, 0u, cflag, ckey);
         wave_lds_sync();
         whits += nh;
-        wheads += st.nheads;
     }
-    add_counts<NT>(whits, wheads, counts);
+    unsigned long long heads = st.heads;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) heads += __shfl_xor(heads, o, 64);
+    add_counts<NT>(whits, heads, counts);
+}
+
+// ---------------------------------------------------------------- exact MTTKRP
+constexpr int kExactThreads = 256;
+
+// One wavefront per chunk of kScanChunk nonzeros.  The next chunk's rows, values
+// and fiber keys (one gather per nonzero, kept in LDS for the lanes of a run) are
+// loaded beside the sums of this one.
+template <typename V>
+__global__ __launch_bounds__(kExactThreads, 4) void exact_rows(const uint32_t* __restrict__ rrow,
+                                                            const uint32_t* __restrict__ rfib,
+                                                            const V* __restrict__ rval, int64_t nnz, int64_t nch,
+                                                            ExactSrc<V> ex, int R, V* __restrict__ Y,
+                                                            V* __restrict__ carry, uint32_t* __restrict__ cflag,
+                                                            uint32_t* __restrict__ ckey,
+                                                            unsigned long long* __restrict__ counts) {
+    constexpr int VW = group_vw<V>(), M = kScanChunk / 64, NB = 4;
+    __shared__ uint64_t lkey[kExactThreads / 64][kScanChunk];
+    __shared__ uint32_t lrow[kExactThreads / 64][kScanChunk];
+    __shared__ V lval[kExactThreads / 64][kScanChunk];
+    const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+    const int64_t step = (int64_t)gridDim.x * (kExactThreads / 64);
+    uint32_t nrow[M], nfib[M], nprev = 0, nnext = 0;
+    V nval[M];
+    uint64_t nkey[M];
+    auto load_raw = [&](int64_t w2) {
+        const int64_t b2 = w2 * kScanChunk, e2 = b2 + kScanChunk;
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const int64_t i = b2 + 64 * m + lane < nnz ? b2 + 64 * m + lane : nnz - 1;
+            nrow[m] = rrow[i];
+            nfib[m] = rfib[i];
+            nval[m] = rval[i];
+        }
+        nprev = b2 > 0 ? rrow[b2 - 1] : 0u;
+        nnext = e2 < nnz ? rrow[e2] : 0u;
+    };
+    auto load_keys = [&] {
+#pragma unroll
+        for (int m = 0; m < M; m++) nkey[m] = ex.fkey[nfib[m]];
+    };
+    bool vec = true;
+    for (int k = 0; k < ex.N; k++) vec = vec && (ex.shift[k] < 0 || rows_vec<V, VW>(ex.U[k], R));
+    // product of each fiber's factor rows in mode order; per mode the loads of all
+    // NB rows are issued before the first product
+    auto rows_of = [&](const uint64_t (&h)[NB], int col0, V (&d)[NB][VW]) {
+        typedef V VT __attribute__((ext_vector_type(VW)));
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int v = 0; v < VW; v++) d[b][v] = (V)1;
+#pragma unroll
+        for (int k = 0; k < kMaxModes; k++) {
+            if (k < ex.N && ex.shift[k] >= 0) {
+                V u[NB][VW];
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const V* row = ex.U[k] + (int64_t)((h[b] >> ex.shift[k]) & ex.mask[k]) * R;
+                    if (vec) {
+                        const VT x = *reinterpret_cast<const VT*>(row + (col0 < R ? col0 : 0));
+#pragma unroll
+                        for (int v = 0; v < VW; v++) u[b][v] = x[v];
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < VW; v++) u[b][v] = row[col0 + v < R ? col0 + v : 0];
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int v = 0; v < VW; v++) d[b][v] *= u[b][v];
+            }
+        }
+    };
+    auto meta = [&](int k, uint32_t& r, uint64_t& h, V& x) {
+        r = lrow[wv][k];
+        h = lkey[wv][k];
+        x = lval[wv][k];
+    };
+    RunRows<V, double, VW, NB, true> st;
+    st.init(lane, R, (R + VW - 1) / VW, Y, carry);
+    unsigned long long whits = 0;
+    int64_t w = (int64_t)blockIdx.x * (kExactThreads / 64) + wv;
+    if (w < nch) {
+        load_raw(w);
+        load_keys();
+    }
+    for (; w < nch; w += step) {
+        const int64_t b = w * kScanChunk, e = b + kScanChunk < nnz ? b + kScanChunk : nnz;
+        const int n = (int)(e - b);
+        wave_lds_sync();
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            lrow[wv][64 * m + lane] = nrow[m];
+            lkey[wv][64 * m + lane] = nkey[m];
+            lval[wv][64 * m + lane] = nval[m];
+        }
+        st.w = w;
+        st.first_row = readlane_u32(nrow[0], 0);
+        st.last_row = st.first_row;
+#pragma unroll
+        for (int m = 0; m < M; m++)
+            if ((n - 1) / 64 == m) st.last_row = readlane_u32(nrow[m], (n - 1) % 64);
+        st.first_cont = b > 0 && nprev == st.first_row;
+        st.continues = e < nnz && nnext == st.last_row;
+        wave_lds_sync();
+        if (w + step < nch) {
+            load_raw(w + step);
+            load_keys();
+        }
+        st.chunk(n, meta, rows_of, cflag, ckey);
+        whits += (unsigned long long)n;
+    }
+    unsigned long long heads = st.heads;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) heads += __shfl_xor(heads, o, 64);
+    add_counts<kExactThreads>(whits, heads, counts);
 }
 
 // ---------------------------------------------------------------- hit list
@@ -1206,7 +1459,7 @@ __global__ __launch_bounds__(kBitThreads) void hit_scan_reduce(const uint32_t* _
         st.last_row = rrow[hits[e - 1]];
         st.first_cont = b > 0 && rrow[hits[b - 1]] == st.first_row;
         st.continues = e < H && rrow[hits[e]] == st.last_row;
-        st.template run<step_batch<V, false>()>(b, e, meta, pre_of, rows_of);
+        st.template run<kStepBatch>(b, e, meta, pre_of, rows_of);
         st.finish(cflag, ckey);
         whits += (unsigned long long)(e - b);
         wheads += st.nheads;
@@ -1499,7 +1752,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_reduce(const uint32_t* __restri
                 c = h.c;
                 x = h.x;
             };
-            if (nh > 0) st.template run<step_batch<V, false>()>(0, nh, meta, pre_of, rows_of);
+            if (nh > 0) st.template run<kStepBatch>(0, nh, meta, pre_of, rows_of);
             st.finish(cflag, ckey);
             whits += nh;
             wheads += st.nheads;
@@ -2294,13 +2547,13 @@ void carry_reduce(hipStream_t s, DevBuf* tmp, int64_t n1, int R, V* Y, const uin
     }
 }
 
-// Lanes per hit of the sampled-MTTKRP row pass: group_lanes, doubled (at
-// most 32) when the autotuner chose the wider variant.
+// Lanes per run of the sampled-MTTKRP row pass: those that cover R columns, or
+// twice as many (fewer runs, half of their lanes idle) when the autotuner chose
+// that.
 template <typename V>
 int scan_lanes(int R) {
-    int G = group_lanes<V>(R);
-    if (tune_value(sizeof(V) == 8 ? kTuneScanF64 : kTuneScanF32) == 1 && G < 32) G *= 2;
-    return G;
+    const int G = (R + group_vw<V>() - 1) / group_vw<V>();
+    return tune_value(sizeof(V) == 8 ? kTuneScanF64 : kTuneScanF32) == 1 && 2 * G <= 64 ? 2 * G : G;
 }
 
 // Per-workgroup counter partials of a pass over `blocks` workgroups (null
@@ -2480,12 +2733,9 @@ void sampled_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const uint64_t*
                            L.filt.as<uint32_t>(), fsel, Y, ny);
         const dim3 scan_grid(grid_for(nch, kScanThreads / 64, num_cus(s)));   // one workgroup per CU (LDS)
         unsigned long long* part = count_parts(L, counts, scan_grid.x);
-        with_group(scan_lanes<V>(R), [&](auto gc) {
-            hipLaunchKernelGGL((row_scan_reduce<V, false, decltype(gc)::value>), scan_grid, dim3(kScanThreads), 0, s,
-                               L.rrow.as<uint32_t>(), L.rfib.as<uint32_t>(), vals, L.nnz, nch,
-                               L.cmap.as<uint64_t>(), L.filt.as<uint32_t>(), design, ExactSrc<V>{}, R, Y, vec, flag,
-                               key, part);
-        });
+        hipLaunchKernelGGL(row_scan_reduce<V>, scan_grid, dim3(kScanThreads), 0, s, L.rrow.as<uint32_t>(),
+                           L.rfib.as<uint32_t>(), vals, L.nnz, nch, L.cmap.as<uint64_t>(), L.filt.as<uint32_t>(), design,
+                           R, scan_lanes<V>(R), Y, vec, flag, key, part);
         carry_reduce<V>(s, tmp, 2 * nch, R, Y);
         hipLaunchKernelGGL(clear_fibers, dim3(grid_for(Ju, kThreads, 16384) + (counts ? 1 : 0)), dim3(kThreads), 0, s,
                            fsel, Ju, Ju_dev, L.filt.as<uint32_t>(), L.cmap.as<uint64_t>(), part, (int)scan_grid.x,
@@ -2513,13 +2763,10 @@ void exact_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const V* const* U
         V* vec;
         uint32_t *flag, *key;
         carry_views(tmp[2], 2 * nch, R, vec, flag, key);
-        const dim3 scan_grid(grid_for(nch, kScanThreads / 64, num_cus(s)));   // one workgroup per CU (LDS)
+        const dim3 scan_grid(grid_for(nch, kExactThreads / 64, 4 * num_cus(s)));   // four workgroups per CU (registers)
         unsigned long long* part = count_parts(L, counts, scan_grid.x);
-        with_group(group_lanes<V>(R), [&](auto gc) {
-            hipLaunchKernelGGL((row_scan_reduce<V, true, decltype(gc)::value>), scan_grid, dim3(kScanThreads), 0, s,
-                               L.rrow.as<uint32_t>(), L.rfib.as<uint32_t>(), vals, L.nnz, nch, nullptr, nullptr,
-                               nullptr, ex, R, Y, vec, flag, key, part);
-        });
+        hipLaunchKernelGGL(exact_rows<V>, scan_grid, dim3(kExactThreads), 0, s, L.rrow.as<uint32_t>(),
+                           L.rfib.as<uint32_t>(), vals, L.nnz, nch, ex, R, Y, vec, flag, key, part);
         if (counts) hipLaunchKernelGGL(sum_counts, dim3(1), dim3(kThreads), 0, s, part, (int)scan_grid.x, counts);
         carry_reduce<V>(s, tmp, 2 * nch, R, Y);
     }
