@@ -213,10 +213,10 @@ __global__ __launch_bounds__(kThreads) void leaf_gram_bf16(const float* __restri
 
 // Inverse of a symmetric positive semidefinite R x R matrix (upper triangle
 // of M read); pivots at or below tol_rel * (largest diagonal entry) dropped.
-// With pinv_on_drop (1024 threads, R <= 32 only), a dropped pivot makes the
+// With pinv_on_drop (R <= 32 only), a dropped pivot makes the
 // same workgroup write the Moore-Penrose pseudo-inverse instead.
-template <int RPT, int T = kSpdThreads>
-__global__ __launch_bounds__(T) void spd_inverse_kernel(const double* __restrict__ M, int R, double tol_rel,
+template <int RPT>
+__global__ __launch_bounds__(1024) void spd_inverse_kernel(const double* __restrict__ M, int R, double tol_rel,
                                                                   double* __restrict__ out, int* __restrict__ dropped,
                                                                   int pinv_on_drop) {
     __shared__ SpdShared sh;
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(T) void spd_inverse_kernel(const double* __restrict
     const double dmax = spd_max_diag<RPT>(sh, L, a, R);
     const int nd = spd_inverse_regs<RPT>(sh, L, a, R, tol_rel * dmax);
     if (dropped && threadIdx.x == 0) *dropped = nd;
-    if constexpr (T == 1024) {
+    if constexpr (RPT == 1) {
         if (pinv_on_drop && nd > 0) {   // nd is the same in every thread
             psd_pinv_chol_block(M, R, tol_rel, out, sh.full, sh.full + 1024, sh.full + 2048, perm);
             return;
@@ -257,8 +257,8 @@ __global__ __launch_bounds__(T) void spd_inverse_kernel(const double* __restrict
 // the Gauss-Jordan inverse itself (the same arithmetic, so the same values)
 // and keeps its slot's product of the later Grams in registers.  Every thread
 // reads and writes only its own elements of each slot.
-template <int RPT, int T = kSpdThreads>
-__global__ __launch_bounds__(T) void sts_compute_m_mixed(int N, int j, int R,
+template <int RPT>
+__global__ __launch_bounds__(1024) void sts_compute_m_mixed(int N, int j, int R,
                                                                    const double* __restrict__ grams,
                                                                    double* __restrict__ M) {
     __shared__ SpdShared sh;
@@ -475,21 +475,21 @@ void tree_build_f32(hipStream_t s, const float* U, const TreeGeom& g, int R, flo
 }
 
 // rows per thread: 256 / R row groups cover R rows
-#define RM_DISPATCH_GRID(R, KERNEL, GRID, STREAM, ...)                                                      \
-    do {                                                                                                    \
-        if ((R) <= 16) hipLaunchKernelGGL((KERNEL<1>), GRID, dim3(kSpdThreads), 0, STREAM, __VA_ARGS__);     \
-        else if ((R) <= 35) hipLaunchKernelGGL((KERNEL<5>), GRID, dim3(kSpdThreads), 0, STREAM, __VA_ARGS__); \
-        else hipLaunchKernelGGL((KERNEL<16>), GRID, dim3(kSpdThreads), 0, STREAM, __VA_ARGS__);             \
+// One element per thread of 1024 up to R = 32, two to four rows a thread above
+// (256 threads with sixteen rows each hid less of a pivot's latency: R = 64, inverse
+// 386 -> 154 us, the factorisations of computeM 346 -> 125 us).
+#define SPD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                     \
+    do {                                                                                               \
+        const int rpt = ((R) + 1024 / (R) - 1) / (1024 / (R));                                         \
+        if (rpt == 1) hipLaunchKernelGGL((KERNEL<1>), GRID, dim3(1024), 0, STREAM, __VA_ARGS__);       \
+        else if (rpt == 2) hipLaunchKernelGGL((KERNEL<2>), GRID, dim3(1024), 0, STREAM, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((KERNEL<4>), GRID, dim3(1024), 0, STREAM, __VA_ARGS__);                \
     } while (0)
-#define RM_DISPATCH(R, KERNEL, STREAM, ...) RM_DISPATCH_GRID(R, KERNEL, dim3(1), STREAM, __VA_ARGS__)
 
-// R <= 32: one element per thread (1024 threads), else the 256-thread tiling.
+// (the pivoted-Cholesky pseudo-inverse of the same workgroup holds R <= 32)
 static void spd_inverse_launch(hipStream_t s, const double* M, int R, double tol_rel, double* out, int* dropped,
                                int pinv_on_drop) {
-    if (R <= 32)
-        hipLaunchKernelGGL((spd_inverse_kernel<1, 1024>), dim3(1), dim3(1024), 0, s, M, R, tol_rel, out, dropped,
-                           pinv_on_drop);
-    else RM_DISPATCH(R, spd_inverse_kernel, s, M, R, tol_rel, out, dropped, 0);
+    SPD_DISPATCH(R, spd_inverse_kernel, dim3(1), s, M, R, tol_rel, out, dropped, R <= 32 ? pinv_on_drop : 0);
     EX_HIP(hipGetLastError());
 }
 
@@ -505,13 +505,10 @@ void spd_pinv(hipStream_t s, const double* M, int R, double tol_rel, double* out
 }
 
 void sts_compute_m_mixed_launch(hipStream_t s, int N, int j, int R, const double* grams, double* M) {
-    // R <= 32: one element per thread (1024 threads; faster than 256 threads
-    // with five rows each, and than one wavefront with sixteen)
     // one workgroup per factorisation: slot N and every slot k in 1 .. N-1, k != j
     int jobs = 1;
     for (int k = 1; k < N; k++) jobs += k != j ? 1 : 0;
-    if (R <= 32) hipLaunchKernelGGL((sts_compute_m_mixed<1, 1024>), dim3(jobs), dim3(1024), 0, s, N, j, R, grams, M);
-    else RM_DISPATCH_GRID(R, sts_compute_m_mixed, dim3(jobs), s, N, j, R, grams, M);
+    SPD_DISPATCH(R, sts_compute_m_mixed, dim3(jobs), s, N, j, R, grams, M);
     EX_HIP(hipGetLastError());
 }
 

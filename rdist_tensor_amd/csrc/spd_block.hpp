@@ -98,12 +98,11 @@ __device__ void psd_pinv_chol_block(const double* __restrict__ M, int R, double 
 }
 
 // ---------------------------------------------------------------- FP64 SPD solves
-// One workgroup of T threads (256, or 1024 for R <= 32) holds an R x R
+// One workgroup of T = 1024 threads holds an R x R
 // matrix in registers: thread t owns column j = t % R and rows g, g + GR,
 // g + 2 GR, ... (g = t / R, GR = T / R row groups, at most RPT rows).  Each elimination step
 // publishes one column (and row) through LDS; the buffers alternate between
 // steps, so one barrier per step suffices.
-constexpr int kSpdThreads = 256;
 
 struct SpdShared {
     double col[2][kMaxRank];
@@ -160,28 +159,23 @@ __device__ int spd_inverse_regs(SpdShared& sh, const SpdLayout& L, double (&a)[R
         const bool skip = !(piv > tol);
         dropped += skip ? 1 : 0;
         const double inv = skip ? 0.0 : 1.0 / piv;
-        if (L.on) {
-            const double rk = sh.row[b][L.j];
-            const int j = L.j;
+        if (!L.on) continue;
+        const int j = L.j;
+        if (skip) {   // the same for the whole workgroup
 #pragma unroll
-            for (int m = 0; m < RPT; m++) {
-                const int i = L.row(m);
-                if (i >= R) continue;
-                const double ci = sh.col[b][i];
-                double v = a[m];
-                if (skip) {
-                    if (i == k || j == k) v = 0.0;
-                } else if (i == k && j == k) {
-                    v = inv;
-                } else if (i == k) {
-                    v = rk * inv;
-                } else if (j == k) {
-                    v = -ci * inv;
-                } else {
-                    v = v - ci * (rk * inv);
-                }
-                a[m] = v;
-            }
+            for (int m = 0; m < RPT; m++)
+                if (L.row(m) == k || j == k) a[m] = 0.0;
+            continue;
+        }
+        // a_ij - a_ik t with t = a_kj / piv; in column k a_ij is taken as zero and
+        // a_kj as one, and row k becomes t
+        const double rk = sh.row[b][j], t = j == k ? inv : rk * inv;
+#pragma unroll
+        for (int m = 0; m < RPT; m++) {
+            const int i = L.row(m);
+            const double ci = sh.col[b][i < R ? i : 0], v0 = j == k ? 0.0 : a[m];
+            const double v = v0 - ci * t;
+            a[m] = i == k ? t : v;
         }
     }
     // mirror the upper triangle
