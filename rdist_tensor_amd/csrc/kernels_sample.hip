@@ -36,17 +36,33 @@ __device__ __forceinline__ void tri_ab_direct(int R, int e, int& a, int& b) {
 
 // ---------------------------------------------------------------- row trees
 // Leaf Grams: one wavefront per leaf; the leaf's F = R rows are staged in LDS
-// and each lane produces its packed-upper elements, summing the rows' products
-// in row order without fused multiply-adds (the oracle's sums exactly, so
-// that every node of the tree, and the factor Gram at its root, is bitwise
-// the oracle's).
-template <int WPB>
+// and each lane produces TS x TS tiles of the upper triangle, summing the rows'
+// products in row order without fused multiply-adds (the oracle's sums exactly,
+// so that every node of the tree, and the factor Gram at its root, is bitwise
+// the oracle's).  One packed element a lane at a time was bound by its two LDS
+// reads per product; a 4 x 4 tile has half a read.  The packed leaf goes out
+// through LDS, so that it is written in order.  NP tiles a lane: one up to R = 32
+// (36 tiles; 2 x 2 tiles up to R = 20, where 4 x 4 would leave most lanes idle),
+// three above.  Modes of 500000, 300000 and 50000 rows at
+// R = 32: 100 -> 46 us on average; of 30-70 rows at R = 16: 8 -> 5.
+template <int WPB, int TS, int NP>
 __global__ __launch_bounds__(64 * WPB) void leaf_gram_kernel(const double* __restrict__ U, int64_t n, int R,
                                                              TreeGeom g, double* __restrict__ nodes) {
 #pragma clang fp contract(off)
-    __shared__ double blk[WPB][kMaxRank * kMaxRank / WPB];
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double blk[WPB][kMaxRank * kMaxRank / WPB];
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int P = tri_size(R), S = tri_stride(R);
+    const int RS = (R + TS - 1) / TS * TS, nt = RS / TS, tiles = nt * (nt + 1) / 2;   // LDS row stride, tiles
+    int ta[NP], tb[NP];
+#pragma unroll
+    for (int q = 0; q < NP; q++) {
+        const int id = lane + 64 * q < tiles ? lane + 64 * q : 0;
+        int a, b;
+        tri_ab(nt, id, a, b);
+        ta[q] = TS * a;
+        tb[q] = TS * b;
+    }
     const int64_t first_leaf = (int64_t)g.node_count - g.leaf_count;
     for (int64_t i = blockIdx.x * (int64_t)WPB + wave; i < (int64_t)g.leaf_count; i += (int64_t)gridDim.x * WPB) {
         const int64_t c = first_leaf + i;
@@ -54,19 +70,57 @@ __global__ __launch_bounds__(64 * WPB) void leaf_gram_kernel(const double* __res
         const int64_t r0 = idx * g.F;
         const int rows = (int)((n - r0) < g.F ? (n - r0) : g.F);
         double* b = blk[wave];
-        for (int e = lane; e < rows * R; e += 64) b[e] = U[r0 * R + e];
+        if (RS == R) {
+            for (int e = lane; e < rows * R; e += 64) b[e] = U[r0 * R + e];
+        } else {   // (the columns past R are not used)
+            for (int e = lane; e < rows * R; e += 64) {
+                const int r = e / R;
+                b[e + r * (RS - R)] = U[r0 * R + e];
+            }
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (int e = lane; e < S; e += 64) {
-            double acc = 0.0;
-            if (e < P) {
-                int a, bb;
-                tri_ab(R, e, a, bb);
-                for (int r = 0; r < rows; r++) acc += b[r * R + a] * b[r * R + bb];
+        double acc[NP][TS][TS];
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+#pragma unroll
+            for (int x = 0; x < TS; x++)
+#pragma unroll
+                for (int y = 0; y < TS; y++) acc[q][x][y] = 0.0;
+            if (64 * q >= tiles) continue;
+            for (int r = 0; r < rows; r++) {
+                double u[TS], v[TS];
+#pragma unroll
+                for (int x = 0; x < TS; x += 2) {
+                    const d2 p = *reinterpret_cast<const d2*>(b + r * RS + ta[q] + x);
+                    const d2 s = *reinterpret_cast<const d2*>(b + r * RS + tb[q] + x);
+                    u[x] = p[0];
+                    u[x + 1] = p[1];
+                    v[x] = s[0];
+                    v[x + 1] = s[1];
+                }
+#pragma unroll
+                for (int x = 0; x < TS; x++)
+#pragma unroll
+                    for (int y = 0; y < TS; y++) acc[q][x][y] += u[x] * v[y];
             }
-            nodes[c * S + e] = acc;
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int q = 0; q < NP; q++)
+            if (lane + 64 * q < tiles)
+#pragma unroll
+                for (int x = 0; x < TS; x++)
+#pragma unroll
+                    for (int y = 0; y < TS; y++)
+                        if (ta[q] + x <= tb[q] + y && tb[q] + y < R) b[tri_index(R, ta[q] + x, tb[q] + y)] = acc[q][x][y];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int e = lane; e < S; e += 64) nodes[c * S + e] = e < P ? b[e] : 0.0;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1334,12 +1388,15 @@ template void unpack_root<float>(hipStream_t, const float*, int, double*);
 
 void tree_build(hipStream_t s, const double* U, const TreeGeom& g, int R, double* nodes) {
     const int S = tri_stride(R);
-    if (R <= 32) {
-        unsigned nb = grid_for(g.leaf_count, 4, 1 << 16);
-        hipLaunchKernelGGL(leaf_gram_kernel<4>, dim3(nb), dim3(256), 0, s, U, g.n, R, g, nodes);
+    if (R <= 20) {
+        hipLaunchKernelGGL((leaf_gram_kernel<4, 2, 1>), dim3(grid_for(g.leaf_count, 4, 1 << 16)), dim3(256), 0, s, U, g.n,
+                           R, g, nodes);
+    } else if (R <= 32) {
+        hipLaunchKernelGGL((leaf_gram_kernel<4, 4, 1>), dim3(grid_for(g.leaf_count, 4, 1 << 16)), dim3(256), 0, s, U, g.n,
+                           R, g, nodes);
     } else {
-        unsigned nb = grid_for(g.leaf_count, 1, 1 << 16);
-        hipLaunchKernelGGL(leaf_gram_kernel<1>, dim3(nb), dim3(64), 0, s, U, g.n, R, g, nodes);
+        hipLaunchKernelGGL((leaf_gram_kernel<1, 4, 3>), dim3(grid_for(g.leaf_count, 1, 1 << 16)), dim3(64), 0, s, U, g.n,
+                           R, g, nodes);
     }
     EX_HIP(hipGetLastError());
     level_sums<double>(s, g, S, nodes);
