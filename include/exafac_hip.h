@@ -145,7 +145,9 @@ int ex_smttkrp_backward(ex_tensor* t, int mode, int64_t Ju, const uint32_t* samp
  * waiting.  Duplicate samples
  * are not reported by the return code: the outputs come out NaN.  The
  * temporaries live in the tensor (grown on demand, which drains the device
- * once): calls on one tensor must be ordered, e.g. on one stream. */
+ * once): calls on one tensor must be ordered, e.g. on one stream.  The first
+ * backward of a mode also lays out a copy of its nonzeros (12 bytes each)
+ * there, where the device has room and `stream` is not being captured. */
 int ex_smttkrp_forward_async(ex_tensor* t, void* stream, int mode, int64_t Ju, const uint32_t* samples,
                              const double* weights, const double* const* factors, int64_t R, double* Y);
 int ex_smttkrp_backward_async(ex_tensor* t, void* stream, int mode, int64_t Ju, const uint32_t* samples,

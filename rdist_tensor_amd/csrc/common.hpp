@@ -51,18 +51,28 @@ struct DevBuf {
         p = nullptr; bytes = 0;
     }
     void ensure(size_t n) {
-        if (n <= bytes) return;
+        const hipError_t e = grow(n);
+        if (e != hipSuccess)
+            throw Error(5, "hipMalloc(" + std::to_string(n) + " bytes) failed: " + hipGetErrorString(e));
+    }
+    // Whether there is room for n bytes (false: no allocation is held).
+    bool try_ensure(size_t n) { return grow(n) == hipSuccess; }
+    hipError_t grow(size_t n) {
+        if (n <= bytes) return hipSuccess;
         // queued kernels may still read the old allocation: drain the device
         // before freeing it (buffers only grow, so this is rare)
         if (p) (void)hipDeviceSynchronize();
         release();
-        size_t want = n < 256 ? 256 : n;
-        hipError_t e = hipMalloc(&p, want);
+        const size_t want = n < 256 ? 256 : n;
+        const hipError_t e = hipMalloc(&p, want);
         if (e != hipSuccess) {
             p = nullptr;
-            throw Error(5, "hipMalloc(" + std::to_string(want) + " bytes) failed: " + hipGetErrorString(e));
+            // the failure is reported here, not by the next launch's check
+            (void)hipGetLastError();
+            return e;
         }
         bytes = want;
+        return hipSuccess;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
@@ -137,10 +147,12 @@ struct ModeLookup {
     DevBuf cpos;    // u32[nnz]: design row of the hit at a row-order position (valid where its bit is set)
     DevBuf marks;   // u8, whole 4096-position chunks: 1 at this step's hit positions (zero between steps)
     DevBuf cpart;   // u64 per-workgroup counter partials of the passes
-    // bucketed path and adjoint (built on first use): key-order target row and value of each nonzero
+    // bucketed path and adjoint (built on first use; the adjoint does without
+    // where there is no room): key-order target row and value of each nonzero
     DevBuf krow;    // u32[nnz]
     DevBuf kval;    // f64[nnz]
     DevBuf kval32;  // f32[nnz]
+    bool krow_filled = false, kval_filled = false, kval32_filled = false;
     int64_t maxfib = 0;    // nonzeros in the longest fiber
     int mttkrp_path = 0;   // 0: chosen per step from the sizes, 1: full row pass, 2: hit bitmap, 3: bucketed hits
 };
@@ -290,7 +302,8 @@ void exact_mttkrp(hipStream_t s, ModeLookup& L, const V* vals, const V* const* U
                   V* Y, int64_t I_j, DevBuf* tmp, uint64_t* counts = nullptr);
 // Adjoint of the sampled MTTKRP: dD = per-sample fiber sums of x * G[row]
 // (Ju x R, written), then grads[k] (k != j, non-null) += dD * dDesign/dU_k.
-// work: the units of long fibers; *distinct: the number of distinct keys in kd
+// work: the units of long fibers (without room for them a long fiber is summed
+// by one wavefront); *distinct: the number of distinct keys in kd
 // (the gradients are not formed unless it is Ju).
 void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uint32_t* sd, const double* wd,
                      int64_t Ju, int N, int j, int R, const double* const* U, const double* G,

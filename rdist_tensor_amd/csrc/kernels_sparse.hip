@@ -8,6 +8,7 @@
 #include <type_traits>
 #include "common.hpp"
 #include "device.hpp"
+#include "key_copies.hpp"
 
 namespace exafac {
 
@@ -2251,19 +2252,32 @@ void with_group(int G, F f) {
     }
 }
 
-// Key-order copies of a mode's target rows and values (L.krow, L.kval or
-// L.kval32), built on first use.
 template <typename V>
-void key_order(hipStream_t s, ModeLookup& L, const V* vals) {
+bool key_order_filled(const ModeLookup& L) {
+    return L.krow_filled && (sizeof(V) == 4 ? L.kval32_filled : L.kval_filled);
+}
+
+// Key-order copies of a mode's target rows and values (L.krow, L.kval or
+// L.kval32), built on first use.  false: no room for them.
+template <typename V>
+bool key_order(hipStream_t s, ModeLookup& L, const V* vals) {
     DevBuf& kv = sizeof(V) == 4 ? L.kval32 : L.kval;
-    const bool rows = !L.krow.p;
-    const size_t n = (size_t)(L.nnz > 0 ? L.nnz : 1);
-    if (rows) L.krow.ensure(n * 4);
-    kv.ensure(n * sizeof(V));
-    if (L.nnz == 0) return;
-    hipLaunchKernelGGL(bk_keyorder<V>, dim3(grid_for(L.nnz, kThreads, 16384)), dim3(kThreads), 0, s,
-                       L.kpos.as<uint32_t>(), L.rrow.as<uint32_t>(), vals, L.nnz,
-                       rows ? L.krow.as<uint32_t>() : nullptr, kv.as<V>());
+    return fill_key_copies(L.krow, L.krow_filled, kv, sizeof(V) == 4 ? L.kval32_filled : L.kval_filled,
+                           (size_t)(L.nnz > 0 ? L.nnz : 1), sizeof(V), [&](bool rows) {
+                               if (L.nnz == 0) return;
+                               hipLaunchKernelGGL(bk_keyorder<V>, dim3(grid_for(L.nnz, kThreads, 16384)), dim3(kThreads),
+                                                  0, s, L.kpos.as<uint32_t>(), L.rrow.as<uint32_t>(), vals, L.nnz,
+                                                  rows ? L.krow.as<uint32_t>() : nullptr, kv.as<V>());
+                               EX_HIP(hipGetLastError());
+                           });
+}
+
+// Whether the stream may be given new memory: not while it is being captured.
+bool may_allocate(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
 }
 
 // ---------------------------------------------------------------- adjoint
@@ -2271,7 +2285,9 @@ void key_order(hipStream_t s, ModeLookup& L, const V* vals) {
 // x * G[i]: the transpose of the sampled MTTKRP.  The nonzeros are read in key
 // order (L.krow, L.kval), where a fiber's are contiguous, and the rows of G
 // gathered by GL lanes each, two columns a lane, 64 / GL nonzeros side by side
-// and kAdjBatch of each group in flight.
+// and kAdjBatch of each group in flight.  Those copies are 12 bytes a nonzero;
+// where there is no room for them, or they would have to be made inside a graph
+// capture, the row-order arrays are gathered through kpos instead (the same sums).
 //
 // Leverage samples fall on long fibers (Zipf(1.1), 2e7 nonzeros: 4e4 and more
 // in the longest), and one wavefront walking such a fiber set the time of the
@@ -2284,37 +2300,40 @@ constexpr int kAdjUnit = 512;
 constexpr int kAdjBatch = 4;
 
 struct AdjUnits {
-    unsigned int* count;   // [0] units, [1] cut fibers (zero before and after a call)
+    unsigned int* count;   // [0] units, [1] cut fibers (cleared by each call first)
     uint2* unit;           // (first key-order position, its nonzeros) of each unit
     uint4* cut;            // (sample, first unit, units) of each cut fiber
     double* part;          // units x R
 };
 
-// acc[v] = sum over key-order positions [k0, k1) of kval * G[krow][2 sub + v],
-// complete in every lane group.
-template <int GL>
-__device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ krow, const double* __restrict__ kval,
-                                          uint32_t k0, uint32_t k1, const double* __restrict__ G, int R, bool vec,
-                                          int lane, double (&acc)[2]) {
+// acc[v] = sum over key-order positions [k0, k1) of val * G[row][2 sub + v],
+// complete in every lane group.  row and val are in key order (kKeyed), or in row
+// order with pos[k] the place of the k-th.
+template <int GL, bool kKeyed>
+__device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ row, const double* __restrict__ val,
+                                          const uint32_t* __restrict__ pos, uint32_t k0, uint32_t k1,
+                                          const double* __restrict__ G, int R, bool vec, int lane,
+                                          double (&acc)[2]) {
     constexpr int S = 64 / GL;
     typedef double VT __attribute__((ext_vector_type(2)));
     const int g = lane / GL, col = 2 * (lane % GL);
     const int c0 = col < R ? col : 0, c1 = col + 1 < R ? col + 1 : 0;
     acc[0] = acc[1] = 0.0;
     for (uint32_t k = k0; k < k1; k += kAdjBatch * S) {
-        uint32_t row[kAdjBatch];
+        uint32_t target[kAdjBatch];
         double x[kAdjBatch], d[kAdjBatch][2];
 #pragma unroll
         for (int b = 0; b < kAdjBatch; b++) {
             const uint32_t i = k + b * S + g;
-            const uint32_t at = i < k1 ? i : k1 - 1;
-            row[b] = krow[at];
-            const double v = kval[at];
+            uint32_t at = i < k1 ? i : k1 - 1;
+            if constexpr (!kKeyed) at = pos[at];
+            target[b] = row[at];
+            const double v = val[at];
             x[b] = i < k1 ? v : 0.0;
         }
 #pragma unroll
         for (int b = 0; b < kAdjBatch; b++) {
-            const double* r = G + (int64_t)row[b] * R;
+            const double* r = G + (int64_t)target[b] * R;
             if (vec) {
                 const VT v = *reinterpret_cast<const VT*>(r + c0);
                 d[b][0] = v[0];
@@ -2346,12 +2365,13 @@ __device__ __forceinline__ void adj_store(double* __restrict__ out, int R, int l
     if (lane < GL && col + 1 < R) out[col + 1] = acc[1];
 }
 
-template <int GL>
+template <int GL, bool kKeyed>
 __global__ __launch_bounds__(kThreads) void fiber_adjoint(const uint64_t* __restrict__ kd, int64_t Ju,
                                                           const uint64_t* __restrict__ fkey, int64_t nfib,
                                                           const uint32_t* __restrict__ fptr,
-                                                          const uint32_t* __restrict__ krow,
-                                                          const double* __restrict__ kval,
+                                                          const uint32_t* __restrict__ row,
+                                                          const double* __restrict__ val,
+                                                          const uint32_t* __restrict__ pos,
                                                           const double* __restrict__ G, int R, bool vec,
                                                           double* __restrict__ dD, AdjUnits units,
                                                           const uint64_t* __restrict__ distinct) {
@@ -2379,15 +2399,16 @@ __global__ __launch_bounds__(kThreads) void fiber_adjoint(const uint64_t* __rest
                 }
                 continue;   // fiber_total writes this sample's row
             }
-            fiber_sum<GL>(krow, kval, k0, k1, G, R, vec, lane, acc);
+            fiber_sum<GL, kKeyed>(row, val, pos, k0, k1, G, R, vec, lane, acc);
         }
         adj_store<GL>(dD + c * R, R, lane, acc);
     }
 }
 
-template <int GL>
-__global__ __launch_bounds__(kThreads) void fiber_units(const uint32_t* __restrict__ krow,
-                                                        const double* __restrict__ kval,
+template <int GL, bool kKeyed>
+__global__ __launch_bounds__(kThreads) void fiber_units(const uint32_t* __restrict__ row,
+                                                        const double* __restrict__ val,
+                                                        const uint32_t* __restrict__ pos,
                                                         const double* __restrict__ G, int R, bool vec,
                                                         AdjUnits units) {
     const int lane = threadIdx.x % 64;
@@ -2395,7 +2416,7 @@ __global__ __launch_bounds__(kThreads) void fiber_units(const uint32_t* __restri
     for (uint32_t u = blockIdx.x * (kThreads / 64) + threadIdx.x / 64; u < n; u += gridDim.x * (kThreads / 64)) {
         const uint2 w = units.unit[u];
         double acc[2];
-        fiber_sum<GL>(krow, kval, w.x, w.x + w.y, G, R, vec, lane, acc);
+        fiber_sum<GL, kKeyed>(row, val, pos, w.x, w.x + w.y, G, R, vec, lane, acc);
         adj_store<GL>(units.part + (int64_t)u * R, R, lane, acc);
     }
 }
@@ -2465,7 +2486,10 @@ void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uin
                      int64_t Ju, int N, int j, int R, const double* const* U, const double* G,
                      double* const* grads, double* dD, DevBuf& work, const uint64_t* distinct) {
     if (Ju == 0) return;
-    if (!L.kval.p) key_order<double>(s, L, L.rval.as<double>());
+    const bool keyed = key_order_filled<double>(L) || (may_allocate(s) && key_order<double>(s, L, L.rval.as<double>()));
+    const uint32_t* row = keyed ? L.krow.as<uint32_t>() : L.rrow.as<uint32_t>();
+    const double* val = keyed ? L.kval.as<double>() : L.rval.as<double>();
+    const uint32_t* pos = keyed ? nullptr : L.kpos.as<uint32_t>();
     // units of cut fibers: at most one per kAdjUnit hits and one more per cut
     // fiber, each of which has more than kAdjUnit of the hits
     AdjUnits units{};
@@ -2477,21 +2501,27 @@ void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uin
         auto take = [&](size_t bytes) { size_t r = o; o = (o + bytes + 255) & ~(size_t)255; return r; };
         const size_t o_c = take(8), o_u = take((size_t)nu * 8), o_l = take((size_t)nc * 16),
                      o_p = take((size_t)nu * R * 8);
-        work.ensure(o);
-        char* b = work.as<char>();
-        units = AdjUnits{(unsigned int*)(b + o_c), (uint2*)(b + o_u), (uint4*)(b + o_l), (double*)(b + o_p)};
-        hipLaunchKernelGGL(adj_clear, dim3(1), dim3(64), 0, s, units.count);
+        if (o <= work.bytes || (may_allocate(s) && work.try_ensure(o))) {
+            char* b = work.as<char>();
+            units = AdjUnits{(unsigned int*)(b + o_c), (uint2*)(b + o_u), (uint4*)(b + o_l), (double*)(b + o_p)};
+            hipLaunchKernelGGL(adj_clear, dim3(1), dim3(64), 0, s, units.count);
+        }
     }
     const bool vec = R % 2 == 0 && ((uintptr_t)G % 16) == 0;
     const dim3 block(kThreads);
-    with_group(group_lanes<double>(R), [&](auto gc) {
+    auto sums = [&](auto gc, auto kc) {
         constexpr int GL = decltype(gc)::value;
-        hipLaunchKernelGGL(fiber_adjoint<GL>, dim3(grid_for(Ju, kThreads / 64, 16384)), block, 0, s, kd, Ju,
-                           L.fkey.as<uint64_t>(), L.nfib, L.fptr.as<uint32_t>(), L.krow.as<uint32_t>(),
-                           L.kval.as<double>(), G, R, vec, dD, units, distinct);
+        constexpr bool kKeyed = decltype(kc)::value;
+        hipLaunchKernelGGL((fiber_adjoint<GL, kKeyed>), dim3(grid_for(Ju, kThreads / 64, 16384)), block, 0, s, kd, Ju,
+                           L.fkey.as<uint64_t>(), L.nfib, L.fptr.as<uint32_t>(), row, val, pos, G, R, vec, dD, units,
+                           distinct);
         if (units.count)
-            hipLaunchKernelGGL(fiber_units<GL>, dim3((unsigned)(8 * num_cus(s))), block, 0, s, L.krow.as<uint32_t>(),
-                               L.kval.as<double>(), G, R, vec, units);
+            hipLaunchKernelGGL((fiber_units<GL, kKeyed>), dim3((unsigned)(8 * num_cus(s))), block, 0, s, row, val, pos, G,
+                               R, vec, units);
+    };
+    with_group(group_lanes<double>(R), [&](auto gc) {
+        if (keyed) sums(gc, std::true_type{});
+        else sums(gc, std::false_type{});
     });
     if (units.count) hipLaunchKernelGGL(fiber_total, dim3((unsigned)num_cus(s)), block, 0, s, units, R, dD);
     DesignArgs a;
@@ -2580,7 +2610,7 @@ void sampled_mttkrp_buckets(hipStream_t s, ModeLookup& L, const V* vals, const u
     const int64_t nnz = L.nnz;
     EX_CHECK(nnz < ((int64_t)1 << 31), 4, "the bucketed sampled MTTKRP needs fewer than 2^31 nonzeros");
     DevBuf& kv = sizeof(V) == 4 ? L.kval32 : L.kval;
-    if (!kv.p) key_order<V>(s, L, vals);
+    EX_CHECK(key_order<V>(s, L, vals), 5, "no room for the key-order copies of the bucketed sampled MTTKRP");
     int bsh = 13;
     while (((nnz - 1) >> bsh) + 1 > kBkMaxBuckets) bsh++;
     const int NB = (int)(((nnz - 1) >> bsh) + 1);
