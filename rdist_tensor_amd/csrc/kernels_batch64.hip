@@ -37,6 +37,26 @@ __host__ __device__ inline int gram_live_groups(int R) {
     return g < kChunkRows ? g : kChunkRows;
 }
 __host__ __device__ inline int gram_items(int R) { return gram_live_groups(R) * (R > 16 ? 3 : 1); }
+// Low ranks have up to 256 groups, each of few rows and few sums: up to 32 rows a
+// group, a Gram is summed by one thread per group and entry, else by one
+// wavefront per group and 16 x 16 tile, which loads 16 steps of four rows at least.
+// 256 tensors, J = 500, the design's and the factor's Gram: R = 1 191 + 532 -> 5 +
+// 39 us by threads, R = 4 134 + 225 -> 15 + 35, R = 8 40 + 85 -> 13 + 31.  (At 128
+// rows a group a thread's chain would be eight rounds of loads; the wavefronts take
+// two: R = 8, J = 8192 17 us.)
+__host__ __device__ inline bool gram_by_threads(int R, int64_t rows) {
+    return R <= 16 && rows <= 32 * (int64_t)gram_live_groups(R);
+}
+__host__ __device__ inline int gram_thread_blocks(int R) { return (gram_live_groups(R) * tri_size(R) + kT - 1) / kT; }
+__host__ __device__ inline int gram_wave_blocks(int R) { return (gram_items(R) + kT / 64 - 1) / (kT / 64); }
+// Workgroups for a Gram of exactly `rows` rows, and of at most that many.
+__host__ __device__ inline int gram_blocks(int R, int64_t rows) {
+    return gram_by_threads(R, rows) ? gram_thread_blocks(R) : gram_wave_blocks(R);
+}
+inline int gram_blocks_bound(int R, int64_t rows) {
+    const int t = gram_by_threads(R, 0) ? gram_thread_blocks(R) : 0;
+    return gram_by_threads(R, rows) ? t : std::max(t, gram_wave_blocks(R));
+}
 // Rows of the factor update whose squares one thread of a column adds up, in
 // order: q, q + norm_classes, ...
 __host__ __device__ inline int norm_classes(int R) { return kBT / R; }
@@ -49,16 +69,24 @@ __global__ __launch_bounds__(kT) void b64_draw(const BatchTensor* __restrict__ t
                                                const BatchCtl* __restrict__ ctl) {
     const BatchTensor& T = ts[blockIdx.y];
     const int N = T.N;
+    if (j >= N) return;
+    // the logarithms that every sample shares: a lane each
+    __shared__ double logs[kMaxModes + 1];
+    if (threadIdx.x <= (unsigned)N) {
+        const int k = (int)threadIdx.x;
+        logs[k] = log(k < N ? (k != j ? 0.0 + gl(T.ssum)[k] : 1.0) : (double)J);
+    }
+    __syncthreads();
     const int64_t s = blockIdx.x * (int64_t)kT + threadIdx.x;
-    if (j >= N || s >= J) return;
-    double w = 0.0 - log((double)J);
+    if (s >= J) return;
+    double w = 0.0 - logs[N];
     uint64_t key = 0;
     for (int k = 0; k < N; k++) {
         uint32_t row = 0;
         if (k != j) {
             const BatchMode& M = T.m[k];
             const uint32_t L = gl(T.cnt)[k];
-            const double ls = log(0.0 + gl(T.ssum)[k]);
+            const double ls = logs[k];
             const double u = uniform01(T.seed, stream_id(ctl->sweep, (uint32_t)j, (uint32_t)k, 0), (uint64_t)s);
             double sc = 0.0;
             if (L > 0) {
@@ -198,10 +226,21 @@ __global__ __launch_bounds__(kT) void b64_design(const BatchTensor* __restrict__
     if (rl < rows) {
         const Gp<double> dg = gl(static_cast<double*>(T.dg));
         for (uint32_t c = c0 + rl; c < c1; c += rows) {
+            // every index, then every row entry, then the products in mode order
+            uint32_t at[kMaxModes];
+            double u[kMaxModes];
+#pragma unroll
+            for (int k = 0; k < kMaxModes; k++)
+                if (k < N && k != j) at[k] = gl(T.sd)[(int64_t)c * N + k];
+            const double wd = gl(T.wd)[c];
+#pragma unroll
+            for (int k = 0; k < kMaxModes; k++)
+                if (k < N && k != j) u[k] = gl(static_cast<const double*>(T.m[k].U))[(int64_t)at[k] * R + r];
             double d = 1.0;
-            for (int k = 0; k < N; k++)
-                if (k != j) d *= gl(static_cast<const double*>(T.m[k].U))[(int64_t)gl(T.sd)[(int64_t)c * N + k] * R + r];
-            dg[(int64_t)c * R + r] = d * gl(T.wd)[c];
+#pragma unroll
+            for (int k = 0; k < kMaxModes; k++)
+                if (k < N && k != j) d *= u[k];
+            dg[(int64_t)c * R + r] = d * wd;
         }
     }
     if (threadIdx.x >= kDesignRows) return;       // one wavefront
@@ -328,17 +367,93 @@ __device__ __forceinline__ void gram_item(Gp<const double> A, const double* sig,
     }
 }
 
-// Workgroup x: four items of the design Gram; the last one lists the rows that
+// The same sum for one group and entry (a, b) on one thread, item = group x
+// tri_size(R) + entry: sixteen rows in flight, added in order.
+template <bool kScaled>
+__device__ __forceinline__ void gram_entry(Gp<const double> A, const double* sig, uint32_t rows, int R, int item,
+                                           Gp<double> part) {
+    constexpr int kU = 16;
+    const int P = tri_size(R), groups = gram_groups(R), g = item / P;
+    int b = item - g * P, a = 0;
+    while (b >= R - a) {
+        b -= R - a;
+        a++;
+    }
+    b += a;
+    const double sa = kScaled ? sig[a] : 1.0, sb = kScaled ? sig[b] : 1.0;
+    uint32_t chunk = 0, at = (uint32_t)g;   // the group's next row is chunk + at
+    double acc = 0.0;
+    for (bool more = (uint32_t)g < rows; more;) {
+        double x[kU], y[kU];
+        bool in[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const uint32_t r = chunk + at;
+            in[u] = r < rows;
+            const Gp<const double> q = A + (int64_t)(in[u] ? r : (uint32_t)g) * R;
+            x[u] = q[a];
+            y[u] = q[b];
+            at += (uint32_t)groups;
+            if (at >= (uint32_t)kChunkRows) {
+                at = (uint32_t)g;
+                chunk += kChunkRows;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const double s = fma(kScaled ? x[u] / sa : x[u], kScaled ? y[u] / sb : y[u], acc);
+            acc = in[u] ? s : acc;
+        }
+        more = chunk + at < rows;
+    }
+    part[(int64_t)g * R * R + a * R + b] = acc;
+}
+
+// The workgroup's share (block of gram_blocks) of the group sums of a Gram.
+// kLow: every Gram of the launch is summed by threads, so that the kernel does
+// without the registers of gram_item (two workgroups a CU).
+template <bool kScaled, bool kLow>
+__device__ __forceinline__ void gram_share(Gp<const double> A, const double* sig, uint32_t rows, int R, int block,
+                                           Gp<double> part) {
+    if (kLow || gram_by_threads(R, rows)) {
+        const int item = block * kT + (int)threadIdx.x;
+        if (item < gram_live_groups(R) * tri_size(R)) gram_entry<kScaled>(A, sig, rows, R, item, part);
+        return;
+    }
+    if constexpr (!kLow) {
+        const int item = block * (kT / 64) + (int)(threadIdx.x >> 6);
+        if (item < gram_items(R)) gram_item<kScaled>(A, sig, rows, R, item, part);
+    }
+}
+
+// x[0] + x[stride] + ... (n terms, in order), sixteen loads ahead of the adds.
+template <typename P>
+__device__ __forceinline__ double sum_in_order(P x, int n, int stride) {
+    constexpr int kU = 16;
+    double t = 0.0;
+    for (int q = 0; q < n; q += kU) {
+        double v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; u++) v[u] = x[(int64_t)(q + u < n ? q + u : n - 1) * stride];
+#pragma unroll
+        for (int u = 0; u < kU; u++) {
+            const double s = t + v[u];
+            t = q + u < n ? s : t;
+        }
+    }
+    return t;
+}
+
+// Workgroup x: a share of the design Gram; the last one lists the rows that
 // were stamped this step, ascending.
+template <bool kLow>
 __global__ __launch_bounds__(kT) void b64_gram_list(const BatchTensor* __restrict__ ts, int j,
                                                     const BatchCtl* __restrict__ ctl) {
     const BatchTensor& T = ts[blockIdx.y];
     if (j >= T.N) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (blockIdx.x + 1 < gridDim.x) {
-        const int item = (int)blockIdx.x * (kT / 64) + wave;
-        if (item < gram_items(T.R))
-            gram_item<false>(gl(static_cast<const double*>(T.dg)), nullptr, *T.ju, T.R, item, gl(T.gpart));
+        gram_share<false, kLow>(gl(static_cast<const double*>(T.dg)), nullptr, *gl(T.ju), T.R, (int)blockIdx.x, gl(T.gpart));
         return;
     }
     __shared__ uint32_t ws[2][kT / 64];
@@ -453,9 +568,7 @@ __global__ __launch_bounds__(kT) void b64_solve(const BatchTensor* __restrict__ 
     for (int o = threadIdx.x; o < R * R; o += kT) {
         const int a = o / R, b = o - a * R;
         if (a > b) continue;
-        double sum = 0.0;
-        for (int q = 0; q < groups; q++) sum += gl(T.gpart)[(int64_t)q * R * R + o];
-        sh.A[tri_index(R, a, b)] = sum;
+        sh.A[tri_index(R, a, b)] = sum_in_order(gl((const double*)T.gpart) + o, groups, R * R);
     }
     __syncthreads();
     jacobi_block<kBatchMaxRank>(sh.A, sh.A2, sh.V, R, sh.j);
@@ -490,31 +603,29 @@ __global__ __launch_bounds__(kT) void b64_update(const BatchTensor* __restrict__
 }
 
 // sigma_c = the column norms; Gram of U_j = Uc diag(1 / sigma) over the listed
-// rows (the others are zero): four items a workgroup; the workgroups past
-// gram_blocks write the rows of U_j.
-__global__ __launch_bounds__(kT) void b64_scale_gram(const BatchTensor* __restrict__ ts, int j, int gram_blocks) {
+// rows (the others are zero) by the first gblocks workgroups, a share each; the
+// workgroups past them write the rows of U_j.
+template <bool kLow>
+__global__ __launch_bounds__(kT) void b64_scale_gram(const BatchTensor* __restrict__ ts, int j, int gblocks) {
     const BatchTensor& T = ts[blockIdx.y];
     if (j >= T.N) return;
     __shared__ double sig[kBatchMaxRank], sums[kBatchNormPart];
     const int R = T.R;
     const uint32_t L = gl(T.cnt)[j];
     const int rows = kT / R, rl = threadIdx.x / R, r = threadIdx.x - rl * R;
-    const int block = (int)blockIdx.x - gram_blocks, nblocks = (int)gridDim.x - gram_blocks;
-    if (block < 0 && (int)blockIdx.x * (kT / 64) >= gram_items(R)) return;
+    const int block = (int)blockIdx.x - gblocks, nblocks = (int)gridDim.x - gblocks;
+    if (block < 0 && (int)blockIdx.x >= gram_blocks(R, L)) return;
     if (block > 0 && (uint32_t)block * rows >= L) return;
     for (int o = threadIdx.x; o < norm_classes(R) * R; o += kT) sums[o] = gl(T.npart)[o];
     __syncthreads();
     if (threadIdx.x < R) {
-        double t = 0.0;
-        for (int g = 0; g < norm_classes(R); g++) t += sums[g * R + threadIdx.x];
-        const double sg = sqrt(t);
+        const double sg = sqrt(sum_in_order((const double*)sums + threadIdx.x, norm_classes(R), R));
         if (block == 0) T.sigma[threadIdx.x] = sg;
         sig[threadIdx.x] = sg;
     }
     __syncthreads();
     if (block < 0) {
-        const int item = (int)blockIdx.x * (kT / 64) + (int)(threadIdx.x >> 6);
-        if (item < gram_items(R)) gram_item<true>(gl((const double*)T.Uc), sig, L, R, item, gl(T.gpart));
+        gram_share<true, kLow>(gl((const double*)T.Uc), sig, L, R, (int)blockIdx.x, gl(T.gpart));
         return;
     }
     const Gp<double> U = gl(static_cast<double*>(T.m[j].U));
@@ -602,12 +713,15 @@ namespace k {
 void batch_sweep64(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, const BatchShape& shape) {
     EX_CHECK(J >= 1 && J <= kBatchMaxJ, 1, "batched sweep: J out of range");
     EX_CHECK(shape.R_max >= 1 && shape.R_max <= kBatchMaxRank && shape.R_min >= 1, 1, "batched sweep: rank out of range");
-    int items = 1, norms = 1;
+    int design_blocks = 1, factor_blocks = 1, norms = 1;   // (a Gram of the design's J rows, of a factor's)
+    bool design_low = true, factor_low = true;
     for (int R = shape.R_min; R <= shape.R_max; R++) {
-        items = std::max(items, gram_items(R));
+        design_blocks = std::max(design_blocks, gram_blocks_bound(R, J));
+        factor_blocks = std::max(factor_blocks, gram_blocks_bound(R, shape.I_max));
+        design_low = design_low && gram_by_threads(R, J);
+        factor_low = factor_low && gram_by_threads(R, shape.I_max);
         norms = std::max(norms, (norm_classes(R) + kT / R - 1) / (kT / R));
     }
-    const unsigned gb = (unsigned)((items + kT / 64 - 1) / (kT / 64));
     // Workgroups of the row-wise phases: two rows a thread group for the longest
     // mode, up to 64 a tensor (a grid-stride loop takes the rest), and about 2048
     // in all: most tensors list few rows, and a workgroup that finds none still
@@ -621,10 +735,12 @@ void batch_sweep64(hipStream_t s, const BatchTensor* ts, int n, int64_t J, Batch
             hipLaunchKernelGGL(b64_draw, dim3(grid_for(J, kT), ny), dim3(kT), 0, s, t, j, J, ctl);
             hipLaunchKernelGGL(b64_dedup, dim3(ny), dim3(kBT), 0, s, t, j, J);
             hipLaunchKernelGGL(b64_design, dim3(db, ny), dim3(kT), 0, s, t, j, ctl);
-            hipLaunchKernelGGL(b64_gram_list, dim3(gb + 1, ny), dim3(kT), 0, s, t, j, ctl);
+            hipLaunchKernelGGL(design_low ? b64_gram_list<true> : b64_gram_list<false>,
+                               dim3((unsigned)design_blocks + 1, ny), dim3(kT), 0, s, t, j, ctl);
             hipLaunchKernelGGL(b64_solve, dim3(1 + rb, ny), dim3(kT), 0, s, t, j, ctl);
             hipLaunchKernelGGL(b64_update, dim3((unsigned)norms, ny), dim3(kT), 0, s, t, j);
-            hipLaunchKernelGGL(b64_scale_gram, dim3(gb + rb, ny), dim3(kT), 0, s, t, j, (int)gb);
+            hipLaunchKernelGGL(factor_low ? b64_scale_gram<true> : b64_scale_gram<false>,
+                               dim3((unsigned)factor_blocks + rb, ny), dim3(kT), 0, s, t, j, factor_blocks);
             hipLaunchKernelGGL(b64_solve, dim3(1, ny), dim3(kT), 0, s, t, j, ctl);
             hipLaunchKernelGGL(b64_scores, dim3(rb, ny), dim3(kT), 0, s, t, j);
             hipLaunchKernelGGL(b64_cdf, dim3(ny), dim3(kBT), 0, s, t, j);
