@@ -284,7 +284,9 @@ int ex_batch_destroy(ex_batch* b);
  * optimizers only; on == 0 drops the graph. */
 int ex_als_use_graph(ex_als* a, int on);
 /* ALS_Optimizer::compute_exact_fit -- als_optimizer.hpp:208-211,
- * sparse_tensor.hpp:288-356 */
+ * sparse_tensor.hpp:288-356: 1 - |X - Xh| / |X|, by |X|^2 + |Xh|^2 - 2 <X, Xh>.
+ * Where that is negative by no more than rounding (the model reproduces X) the
+ * fit is 1; more negative (X repeats coordinates), it is NaN. */
 int ex_als_fit(ex_als* a, double* fit);
 /* ALS_Optimizer::get_statistics_json -- als_optimizer.hpp:126-128.
  * Writes at most *len bytes (NUL-terminated) and sets *len to the full

@@ -12,6 +12,7 @@
 #include <thread>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <sstream>
@@ -1005,17 +1006,23 @@ double als_fit_impl(ex_als* a) {
     for (int k2 = 0; k2 < N; k2++)
         k::gram(st, f->U[k2].as<double>(), f->dims[k2], R, a->fit_grams.as<double>() + (int64_t)k2 * R * R, a->part);
     double* d = a->scal.as<double>();
-    k::chain_had_norm(st, a->fit_grams.as<double>(), N, R, f->sigma.as<double>(), d);
+    k::chain_had_norm(st, a->fit_grams.as<double>(), N, R, f->sigma.as<double>(), d, d + 2);
     // in the row order of mode 0 the last mode's rows are the scattered ones,
     // in the last mode's order the one before it: the smaller factor of the two
     const int by = t->dims[N - 1] <= t->dims[N - 2] ? 0 : N - 1;
     k::fit_dot(st, t->lk[by], f->ptrs, t->dims, f->sigma.as<double>(), R, d + 1, a->fit_part);
-    double h[2];
+    double h[3];
     d2h(st, h, d, sizeof(h));
-    // where the model reproduces X this is rounding noise of either sign, and
-    // a negative one counts as zero (NaN stays)
-    const double res2 = t->norm2 + h[0] - 2.0 * h[1];
-    return 1.0 - std::sqrt(res2 < 0.0 ? 0.0 : res2) / t->norm;
+    // Where the model reproduces X, res2 is rounding noise of either sign, and a
+    // negative one counts as zero.  The terms of each of the three sums have
+    // absolute sums of at most (|X| + S)^2, S = sum_r |sigma_r| prod_k |u_kr|, and no
+    // sum adds more than `chain` values one after another; a res2 below that noise
+    // comes from sums that do not belong together (coordinates that X repeats) and
+    // the fit is NaN.
+    const double res2 = t->norm2 + h[0] - 2.0 * h[1], size = t->norm + h[2];
+    const double chain = 4096.0 + (double)(t->nnz + *std::max_element(t->dims, t->dims + N)) / 1024.0;
+    const bool noise = res2 < 0.0 && -res2 <= chain * std::numeric_limits<double>::epsilon() * size * size;
+    return 1.0 - std::sqrt(noise ? 0.0 : res2) / t->norm;
 }
 
 // Keys of device sample tuples for `mode`, checked distinct (the sampled

@@ -187,7 +187,8 @@ void dsymm(hipStream_t s, const double* G, const double* Y, int64_t m, int R, do
 // sigma_c = the column norms of U, U /= sigma
 void normalize_cols(hipStream_t s, double* U, int64_t m, int R, double* sigma, DevBuf& part);
 void cos_init(hipStream_t s, double* U, int64_t m, int R);
-void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out);
+// *out = |Xh|^2, *size = sum_r |sigma_r| prod_k |u_kr|
+void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out, double* size);
 // out = elementwise product of grams[k] (k != exclude), k ascending
 void chain_had(hipStream_t s, const double* grams, int N, int exclude, int R, double* out);
 // preprocessing / norms

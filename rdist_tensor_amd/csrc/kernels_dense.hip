@@ -540,9 +540,15 @@ __global__ __launch_bounds__(kThreads) void cos_init_kernel(double* __restrict__
 // sum_ab (prod_k G_k)[a][b] sigma_a sigma_b  (chain_had_prod over all modes).
 __global__ __launch_bounds__(kThreads) void chain_had_norm_kernel(const double* __restrict__ grams, int N, int R,
                                                                   const double* __restrict__ sigma,
-                                                                  double* __restrict__ out) {
-    __shared__ double red[kThreads];
+                                                                  double* __restrict__ out,
+                                                                  double* __restrict__ size) {
+    __shared__ double red[kThreads], part[kMaxRank];
     const int R2 = R * R;
+    if (threadIdx.x < R) {
+        double p = fabs(sigma[threadIdx.x]);
+        for (int k = 0; k < N; k++) p *= sqrt(grams[(int64_t)k * R2 + threadIdx.x * (R + 1)]);
+        part[threadIdx.x] = p;
+    }
     double acc = 0.0;
     for (int o = threadIdx.x; o < R2; o += blockDim.x) {
         double p = 1.0;
@@ -555,6 +561,9 @@ __global__ __launch_bounds__(kThreads) void chain_had_norm_kernel(const double* 
         double s = 0.0;
         for (int t = 0; t < kThreads; t++) s += red[t];
         *out = s;
+        double z = 0.0;
+        for (int r = 0; r < R; r++) z += part[r];
+        *size = z;
     }
 }
 
@@ -757,8 +766,8 @@ void cos_init(hipStream_t s, double* U, int64_t m, int R) {
     EX_HIP(hipGetLastError());
 }
 
-void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out) {
-    hipLaunchKernelGGL(chain_had_norm_kernel, dim3(1), dim3(kThreads), 0, s, grams, N, R, sigma, out);
+void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out, double* size) {
+    hipLaunchKernelGGL(chain_had_norm_kernel, dim3(1), dim3(kThreads), 0, s, grams, N, R, sigma, out, size);
     EX_HIP(hipGetLastError());
 }
 
