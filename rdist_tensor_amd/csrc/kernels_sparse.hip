@@ -2296,6 +2296,11 @@ bool may_allocate(hipStream_t s) {
 // (one wavefront a unit) and fiber_total adds in order, so the result does not
 // depend on the order in which the units were listed.  J = 65536, R = 32: 35.2
 // ms in one launch before, 0.24 ms in these (0.155 + 0.075 + 0.01).
+//
+// Where every fiber has one or two nonzeros the search and the instructions
+// around it are the time: one nonzero takes a column a lane and no exchange, up to
+// 64 / GL take one of each group.  1e5 samples of one nonzero, R = 32: 43 us (62 by
+// the batched sums); of two on average 46 (one after the other: 55).
 constexpr int kAdjUnit = 512;
 constexpr int kAdjBatch = 4;
 
@@ -2306,9 +2311,9 @@ struct AdjUnits {
     double* part;          // units x R
 };
 
-// acc[v] = sum over key-order positions [k0, k1) of val * G[row][2 sub + v],
-// complete in every lane group.  row and val are in key order (kKeyed), or in row
-// order with pos[k] the place of the k-th.
+// acc[v] = sum over key-order positions [k0, k1) of val * G[row][2 sub + v] in the
+// first lane group.  row and val are in key order (kKeyed), or in row order with
+// pos[k] the place of the k-th.
 template <int GL, bool kKeyed>
 __device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ row, const double* __restrict__ val,
                                           const uint32_t* __restrict__ pos, uint32_t k0, uint32_t k1,
@@ -2319,38 +2324,45 @@ __device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ row, cons
     const int g = lane / GL, col = 2 * (lane % GL);
     const int c0 = col < R ? col : 0, c1 = col + 1 < R ? col + 1 : 0;
     acc[0] = acc[1] = 0.0;
-    for (uint32_t k = k0; k < k1; k += kAdjBatch * S) {
-        uint32_t target[kAdjBatch];
-        double x[kAdjBatch], d[kAdjBatch][2];
+    auto sum = [&](auto batch) {
+        constexpr int B = decltype(batch)::value;
+        for (uint32_t k = k0; k < k1; k += B * S) {
+            uint32_t target[B];
+            double x[B], d[B][2];
 #pragma unroll
-        for (int b = 0; b < kAdjBatch; b++) {
-            const uint32_t i = k + b * S + g;
-            uint32_t at = i < k1 ? i : k1 - 1;
-            if constexpr (!kKeyed) at = pos[at];
-            target[b] = row[at];
-            const double v = val[at];
-            x[b] = i < k1 ? v : 0.0;
-        }
+            for (int b = 0; b < B; b++) {
+                const uint32_t i = k + b * S + g;
+                uint32_t at = i < k1 ? i : k1 - 1;
+                if constexpr (!kKeyed) at = pos[at];
+                target[b] = row[at];
+                const double v = val[at];
+                x[b] = i < k1 ? v : 0.0;
+            }
 #pragma unroll
-        for (int b = 0; b < kAdjBatch; b++) {
-            const double* r = G + (int64_t)target[b] * R;
-            if (vec) {
-                const VT v = *reinterpret_cast<const VT*>(r + c0);
-                d[b][0] = v[0];
-                d[b][1] = v[1];
-            } else {
-                d[b][0] = r[c0];
-                d[b][1] = r[c1];
+            for (int b = 0; b < B; b++) {
+                const double* r = G + (int64_t)target[b] * R;
+                if (vec) {
+                    const VT v = *reinterpret_cast<const VT*>(r + c0);
+                    d[b][0] = v[0];
+                    d[b][1] = v[1];
+                } else {
+                    d[b][0] = r[c0];
+                    d[b][1] = r[c1];
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                // (a position past the end adds nothing, whatever the row holds)
+                const bool in = k + b * S + g < k1;
+                acc[0] += in ? x[b] * d[b][0] : 0.0;
+                acc[1] += in ? x[b] * d[b][1] : 0.0;
             }
         }
-#pragma unroll
-        for (int b = 0; b < kAdjBatch; b++) {
-            // (a position past the end adds nothing, whatever the row holds)
-            const bool in = k + b * S + g < k1;
-            acc[0] += in ? x[b] * d[b][0] : 0.0;
-            acc[1] += in ? x[b] * d[b][1] : 0.0;
-        }
-    }
+    };
+    // at most one nonzero a group (the fibers of very sparse tensors): the other
+    // positions of a batch would be loads of the last one again
+    if (k1 - k0 <= S) sum(std::integral_constant<int, 1>{});
+    else sum(std::integral_constant<int, kAdjBatch>{});
 #pragma unroll
     for (int o = GL; o < 64; o <<= 1) {
         acc[0] += __shfl_xor(acc[0], o, 64);
@@ -2361,8 +2373,14 @@ __device__ __forceinline__ void fiber_sum(const uint32_t* __restrict__ row, cons
 template <int GL>
 __device__ __forceinline__ void adj_store(double* __restrict__ out, int R, int lane, const double (&acc)[2]) {
     const int col = 2 * lane;
-    if (lane < GL && col < R) out[col] = acc[0];
-    if (lane < GL && col + 1 < R) out[col + 1] = acc[1];
+    if (lane >= GL || col >= R) return;
+    if (R % 2 == 0) {   // (the rows start 16-byte aligned)
+        typedef double VT __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<VT*>(out + col) = VT{acc[0], acc[1]};
+        return;
+    }
+    out[col] = acc[0];
+    if (col + 1 < R) out[col + 1] = acc[1];
 }
 
 template <int GL, bool kKeyed>
@@ -2375,16 +2393,24 @@ __global__ __launch_bounds__(kThreads) void fiber_adjoint(const uint64_t* __rest
                                                           const double* __restrict__ G, int R, bool vec,
                                                           double* __restrict__ dD, AdjUnits units,
                                                           const uint64_t* __restrict__ distinct) {
-    // repeated samples: the caller's outputs become NaN, and kd holds fewer
-    // than Ju keys (the unit lists are sized for distinct fibers)
-    if ((int64_t)*distinct != Ju) return;
+    const bool whole = (int64_t)*distinct == Ju;
     const int lane = threadIdx.x % 64;
     for (int64_t c = blockIdx.x * (int64_t)(kThreads / 64) + threadIdx.x / 64; c < Ju;
          c += (int64_t)gridDim.x * (kThreads / 64)) {
         const int64_t f = wave_find_key(fkey, nfib, kd[c], lane);
+        // repeated samples: the caller's outputs become NaN, and kd holds fewer than
+        // Ju keys (the unit lists are sized for distinct fibers); tested here, where
+        // the count has arrived beside the search
+        if (!whole) return;
         double acc[2] = {0.0, 0.0};
         if (f >= 0) {
             const uint32_t k0 = fptr[f], k1 = fptr[f + 1];
+            if (k1 - k0 == 1) {   // most fibers of a very sparse tensor: a column a lane
+                const uint32_t p = kKeyed ? k0 : pos[k0];
+                const double x = val[p], *g = G + (int64_t)row[p] * R;
+                if (lane < R) dD[c * R + lane] = 0.0 + x * g[lane];
+                continue;
+            }
             if (units.count && k1 - k0 > kAdjUnit) {
                 const uint32_t n = (k1 - k0 + kAdjUnit - 1) / kAdjUnit;
                 uint32_t u0 = 0;
