@@ -43,7 +43,9 @@ __device__ __forceinline__ void tri_ab_direct(int R, int e, int& a, int& b) {
 // reads per product; a 4 x 4 tile has half a read.  The packed leaf goes out
 // through LDS, so that it is written in order.  NP tiles a lane: one up to R = 32
 // (36 tiles; 2 x 2 tiles up to R = 20, where 4 x 4 would leave most lanes idle),
-// three above.  Modes of 500000, 300000 and 50000 rows at
+// three above.  Up to R = 10 a lane holds one packed element and writes it itself:
+// a leaf's few elements are less than the way through LDS (500000 rows, R = 1 158
+// -> 108 us, 4 64 -> 51, 8 40 -> 36; 12 by tiles 41, so 56).  Modes of 500000, 300000 and 50000 rows at
 // R = 32: 100 -> 46 us on average; of 30-70 rows at R = 16: 8 -> 5.
 template <int WPB, int TS, int NP>
 __global__ __launch_bounds__(64 * WPB) void leaf_gram_kernel(const double* __restrict__ U, int64_t n, int R,
@@ -81,6 +83,17 @@ __global__ __launch_bounds__(64 * WPB) void leaf_gram_kernel(const double* __res
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (TS == 1) {   // (tile = packed element)
+            static_assert(NP == 1, "an element a lane");
+            double acc = 0.0;
+            const int mine = lane < P ? rows : 0;
+            for (int r = 0; r < mine; r++) acc += b[r * R + ta[0]] * b[r * R + tb[0]];
+            if (lane < S) nodes[c * S + lane] = lane < P ? acc : 0.0;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            continue;
+        }
         double acc[NP][TS][TS];
 #pragma unroll
         for (int q = 0; q < NP; q++) {
@@ -92,7 +105,7 @@ __global__ __launch_bounds__(64 * WPB) void leaf_gram_kernel(const double* __res
             for (int r = 0; r < rows; r++) {
                 double u[TS], v[TS];
 #pragma unroll
-                for (int x = 0; x < TS; x += 2) {
+                for (int x = 0; x + 1 < TS; x += 2) {
                     const d2 p = *reinterpret_cast<const d2*>(b + r * RS + ta[q] + x);
                     const d2 s = *reinterpret_cast<const d2*>(b + r * RS + tb[q] + x);
                     u[x] = p[0];
@@ -1388,7 +1401,10 @@ template void unpack_root<float>(hipStream_t, const float*, int, double*);
 
 void tree_build(hipStream_t s, const double* U, const TreeGeom& g, int R, double* nodes) {
     const int S = tri_stride(R);
-    if (R <= 20) {
+    if (R <= 10) {   // (at most 55 elements, a stride of at most 64)
+        hipLaunchKernelGGL((leaf_gram_kernel<4, 1, 1>), dim3(grid_for(g.leaf_count, 4, 1 << 16)), dim3(256), 0, s, U, g.n,
+                           R, g, nodes);
+    } else if (R <= 20) {
         hipLaunchKernelGGL((leaf_gram_kernel<4, 2, 1>), dim3(grid_for(g.leaf_count, 4, 1 << 16)), dim3(256), 0, s, U, g.n,
                            R, g, nodes);
     } else if (R <= 32) {
