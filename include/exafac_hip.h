@@ -313,8 +313,10 @@ int ex_tns_read(const char* path, int64_t nnz, int nmodes, uint64_t* coords, dou
  * writes tuning.txt beside the library.  The first ex_ctx_create of a
  * process loads that file ($EXAFAC_TUNING names another file; "off" keeps
  * the defaults).  Every variant computes the same draws and sums up to
- * rounding (FP64 draws stay index-exact).  Knobs are numbered 0..n-1;
- * variant 0 is the built-in default.  A file line is "name value" ('#'
+ * rounding (FP64 draws stay index-exact).  Knobs are numbered 0..n-1; a
+ * variant's number keeps its meaning from build to build, so that a file
+ * written earlier selects what it measured.  A knob that nothing has set holds
+ * its built-in default.  A file line is "name value" ('#'
  * starts a comment); an unknown name or an out-of-range value is an error. */
 int ex_tuning_count(int* n);
 int ex_tuning_info(int knob, char* name, size_t len, int* variants, int* value);

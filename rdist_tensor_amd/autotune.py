@@ -11,8 +11,8 @@ with Zipf(1.1) coordinates at R = 32 (and R = 16 for the r16 knobs), and the
 four-mode 1e7 x 1e6 x 1e4 x 1e2 tensor at R = 64 for sts_draw.fp32.r64, at
 `scale` of their nonzeros (the draws' cost depends on the mode sizes, which
 stay full).  Every variant starts from the same factors and seed.  The
-fastest mean launch wins; a variant must beat the default by 1% to replace
-it.  The result is written as tuning.txt ("knob value" lines, the measured
+fastest mean launch wins; a variant must beat the built-in default by 1% to
+replace it.  The result is written as tuning.txt ("knob value" lines, the measured
 times in comments), which the first ex_ctx_create of a process loads from
 the library's directory.
 """
@@ -100,15 +100,16 @@ def main():
             _, R, precision, span = KNOBS[k]
             U0 = synthetic.factors(cfg["dims"], R, cfg["seed"])
             times = []
+            default = info[k][1]
             for v in range(info[k][0]):
                 abi.tuning_set(k, v)
                 ms = time_variant(abi, ctx, T, cfg, U0, R, precision, span, args.warm, args.sweeps)
                 times.append(ms)
                 log(f"[autotune] {k} variant {v}: {ms:.4f} ms per launch")
-            abi.tuning_set(k, 0)
+            abi.tuning_set(k, default)
             best = min(range(len(times)), key=lambda v: times[v])
-            if times[best] > 0.99 * times[0]:
-                best = 0
+            if times[best] > 0.99 * times[default]:
+                best = default
             results[k] = {"value": best, "ms": times, "workload": wl, "scale": scale, "R": R,
                           "precision": precision, "span": span}
         T.close()

@@ -50,13 +50,14 @@ void lookup_static_scratch(int device) {
 
 thread_local std::string g_last_error;
 
-// Launch variants (common.hpp TuneKnob): names, variant counts, current values.
+// Launch variants (common.hpp TuneKnob): names, variant counts, current values
+// (the initial ones are the built-in defaults).
 const TuneInfo kTuneTable[kTuneKnobs] = {
-    {"sts_draw.fp64.r16", 4}, {"sts_draw.fp64.r32", 6}, {"sts_draw.fp32.r16", 4},
-    {"sts_draw.fp32.r32", 7}, {"sts_draw.fp32.r64", 4}, {"row_scan.fp64", 2},
+    {"sts_draw.fp64.r16", 5}, {"sts_draw.fp64.r32", 7}, {"sts_draw.fp32.r16", 5},
+    {"sts_draw.fp32.r32", 7}, {"sts_draw.fp32.r64", 5}, {"row_scan.fp64", 2},
     {"row_scan.fp32", 2}, {"sts_first.fp32", 2},
 };
-std::atomic<int> g_tune[kTuneKnobs];
+std::atomic<int> g_tune[kTuneKnobs] = {{4}, {6}};
 std::once_flag g_tune_once;
 
 int tune_index(const std::string& name) {

@@ -363,8 +363,8 @@ size_t exclusive_scan_u64(hipStream_t s, void* temp, size_t temp_bytes, const ui
 // ---------------------------------------------------------------- launch variants
 // Compiled alternatives an offline autotuner chooses between
 // (rdist_tensor_amd/autotune.py measures them and writes tuning.txt beside
-// the library, which the first context loads).  Value 0 is the built-in
-// default; every variant computes the same quantities.
+// the library, which the first context loads).  Every variant computes the same
+// quantities.  A number keeps its meaning: tuning files name it.
 enum TuneKnob {
     kTuneDrawF64R16,   // STS-CP draw, FP64 nodes, R <= 16: (lanes per sample, vectors per lane, threads)
     kTuneDrawF64R32,   // FP64, 16 < R <= 32

@@ -1452,16 +1452,18 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     // flight together).
     bool deep = false;   // a tree of 2^7 leaves or more
     for (int k = 0; k < N; k++) deep = deep || (k != j && modes[k].g.lfill_level >= 7);
-    // Variant 0 of each rank class is the default; the others are the
-    // alternatives the autotuner measures (tune_value).
+    // The variants of each rank class that the autotuner measures (tune_value).  A
+    // number keeps its shape: tuning files name it.  The last ones choose the shape
+    // by rank, samples and trees.
     if (node_bytes == 8) {
         // NV: no more vectors than the triangle fills (R = 25: 6, not 9)
         if (R <= 16) {
             switch (tune_value(kTuneDrawF64R16)) {
+                case 0: DRAW_LAUNCH(double, 16, 5, 1024); break;
                 case 1: DRAW_LAUNCH(double, 8, 9, 1024); break;
                 case 2: DRAW_LAUNCH(double, 32, 3, 1024); break;
                 case 3: DRAW_LAUNCH(double, 8, 9, 512); break;
-                default:
+                default:   // 4
                     // few samples: more lanes each, and small workgroups to
                     // reach every CU (R = 16, J = 4096: 43 -> 22 us; J = 16384:
                     // 45 against 57 the other way)
@@ -1471,12 +1473,13 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
             }
         } else if (R <= 32) {
             switch (tune_value(kTuneDrawF64R32)) {
+                case 0: DRAW_LAUNCH(double, 32, 9, 1024); break;
                 case 1: DRAW_LAUNCH(double, 16, 17, 1024); break;
                 case 2: DRAW_LAUNCH(double, 64, 5, 1024); break;
-                case 3: DRAW_LAUNCH(double, 32, 9, 1024); break;
+                case 3: DRAW_LAUNCH(double, 32, 9, 256); break;
                 case 4: DRAW_LAUNCH(double, 16, 17, 512); break;
                 case 5: DRAW_LAUNCH(double, 64, 5, 256); break;
-                default:
+                default:   // 6
                     if (R <= 24) DRAW_LAUNCH(double, 32, 5, 256);
                     else if (R <= 27) DRAW_LAUNCH(double, 32, 6, 256);
                     else if (R <= 29) DRAW_LAUNCH(double, 32, 7, 256);
@@ -1497,12 +1500,13 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     } else {
         if (R <= 16) {
             switch (tune_value(kTuneDrawF32R16)) {
-                case 1:
+                case 1: DRAW_LAUNCH(float, 8, 5, 1024); break;
+                case 2: DRAW_LAUNCH(float, 32, 2, 1024); break;
+                case 3: DRAW_LAUNCH(float, 8, 5, 512); break;
+                case 4:
                     if (J < 8192) DRAW_LAUNCH(float, 8, 5, 256);
                     else DRAW_LAUNCH(float, 8, 5, 1024);
                     break;
-                case 2: DRAW_LAUNCH(float, 32, 2, 1024); break;
-                case 3: DRAW_LAUNCH(float, 8, 5, 512); break;
                 default: DRAW_LAUNCH(float, 16, 3, 1024); break;
             }
         } else if (R <= 32) {
@@ -1521,7 +1525,10 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
             DRAW_LAUNCH(float, 32, 9, 256);
         } else {
             switch (tune_value(kTuneDrawF32R64)) {
-                case 1:
+                case 1: DRAW_LAUNCH(float, 32, 17, 1024); break;
+                case 2: DRAW_LAUNCH(float, 32, 17, 512); break;
+                case 3: DRAW_LAUNCH(float, 64, 9, 256); break;
+                case 4:
                     // deep trees read most levels from L2 and beyond, where three
                     // small workgroups per CU wait less than a large one; shallow
                     // ones live on the levels that a large one stages (R = 64,
@@ -1530,8 +1537,6 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                     if (deep || J < 8192) DRAW_LAUNCH(float, 32, 17, 256);
                     else DRAW_LAUNCH(float, 32, 17, 1024);
                     break;
-                case 2: DRAW_LAUNCH(float, 32, 17, 512); break;
-                case 3: DRAW_LAUNCH(float, 64, 9, 256); break;
                 default: DRAW_LAUNCH(float, 64, 9, 1024); break;
             }
         }
