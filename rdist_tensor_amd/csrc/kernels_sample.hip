@@ -1307,13 +1307,15 @@ static int64_t first_tables(const StsModeArgs& m, int R) {
     return VT * KB * 512 + 2 * kMaxRank + (int64_t)R * m.g.node_count;
 }
 
-// The tables cost three launches and one pass over the tree, the descents a node
-// per level and sample.  Measured (two modes of 3e5 rows, a draw with descents
-// only against one with the first mode tabulated): R = 32, J = 65536 648 -> 476
-// us, 16384 182 -> 168, 4096 65 -> 83; R = 64 3190 -> 1941, 785 -> 614, 202 ->
-// 257; R = 16, J = 65536 182 -> 151.
+// The tables cost three launches (about 11 us) and one pass over the tree, the
+// descents a node per level and sample.  Measured, us by descents / with tables, on
+// modes of 300, 20000 and 500000 rows: R = 16, J = 28000 41 / 43, 51 / 54, 75 / 74;
+// 40000 52 / 53, 65 / 64, 95 / 86; 65536 80 / 73, 95 / 87, 141 / 116 (R = 1 to 12 cross
+// in the same places); R = 17, J = 16000 75 / 79, 94 / 90, 126 / 119; 65536 293 / 264,
+// 351 / 292, 480 / 368; R = 64, J = 16000 355 / 331, 464 / 392, 649 / 516.
 bool sts_first_pays(const StsModeArgs& m, int R, int64_t J) {
-    return J >= (R <= 16 ? 24576 : 16384) && J * (int64_t)(m.g.lfill_level + 1) >= 4 * (int64_t)m.g.node_count;
+    const int64_t from = R > 16 ? 16384 : m.g.lfill_level >= 11 ? 28672 : 40960;
+    return J >= from && J * (int64_t)(m.g.lfill_level + 1) >= 4 * (int64_t)m.g.node_count;
 }
 
 size_t sts_first_bytes(const StsModeArgs& m, int R, int64_t J) {
@@ -1418,6 +1420,14 @@ void tree_build(hipStream_t s, const double* U, const TreeGeom& g, int R, double
     level_sums<double>(s, g, S, nodes);
 }
 
+// Whether workgroups of 1024 threads draw J samples of G lanes in less time than of
+// 256: whole rounds x cost of the large ones, one a CU, against rounds of the small
+// ones, three a CU, whose last one is half as long as it is empty.
+static bool wide_draw(int64_t J, int G, double cost) {
+    const int64_t narrow = 256 * 3 * (256 / G), wide = 256 * (1024 / G);   // samples a round
+    return cost * (double)((J + wide - 1) / wide) < 0.5 * ((double)((J + narrow - 1) / narrow) + (double)J / narrow);
+}
+
 void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* modes, const double* pinv_packed,
               uint64_t seed, uint64_t sweep, const double* draws_row, const double* draws_eig, uint32_t* samples,
               double* weights, int node_bytes, const uint64_t* sweep_dev, unsigned long long* dropped,
@@ -1439,6 +1449,11 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     a.vec_leaf = R % vw == 0;
     for (int k = 0; k < N; k++)
         if (k != j && ((uintptr_t)modes[k].rows % (size_t)(vw * node_bytes)) != 0) a.vec_leaf = 0;
+#define DRAW_BY_ROUNDS(TN, G, NV, COST)                      \
+    do {                                                     \
+        if (wide_draw(J, G, COST)) DRAW_LAUNCH(TN, G, NV, 1024); \
+        else DRAW_LAUNCH(TN, G, NV, 256);                    \
+    } while (0)
 #define DRAW_LAUNCH(TN, G, NV, NT)                                                                     \
     do {                                                                                               \
         static_assert(draw_rmax(G, NV, Vec<TN>::W) >= 16, "variant below the smallest rank class");   \
@@ -1450,8 +1465,18 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
     // NT threads per workgroup (1024: more samples share each staged copy of
     // the top levels; 512: registers for every node load of a level in
     // flight together).
-    bool deep = false;   // a tree of 2^7 leaves or more
-    for (int k = 0; k < N; k++) deep = deep || (k != j && modes[k].g.lfill_level >= 7);
+    // DRAW_BY_ROUNDS: workgroups of 256 or of 1024 threads, whichever ends first.
+    // Registers and LDS leave a CU three small workgroups or a large one, so a round
+    // of the chip's 256 CUs takes 3/4 as many samples in small ones; a large one
+    // stages more levels but waits longer, and its round takes `cost` times a small
+    // one's (measured at 500 to 131072 samples on modes of 30 to 500000 rows; deep
+    // trees read more levels past the staged ones).  FP64, R = 16 / 25 / 41 on 100-300
+    // rows, us: J = 8000 23 / 49 / 138 (by the other shape 24 / 65 / 152), 12000 26 / 77 /
+    // 201 (39 / 92 / 215); FP32, R = 45: J = 8000 70 (86), 12000 102 (127).
+    uint32_t levels = 0;   // of the deepest tree
+    for (int k = 0; k < N; k++)
+        if (k != j) levels = std::max(levels, modes[k].g.lfill_level);
+    const bool deep = levels >= 7;
     // The variants of each rank class that the autotuner measures (tune_value).  A
     // number keeps its shape: tuning files name it.  The last ones choose the shape
     // by rank, samples and trees.
@@ -1463,12 +1488,10 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                 case 1: DRAW_LAUNCH(double, 8, 9, 1024); break;
                 case 2: DRAW_LAUNCH(double, 32, 3, 1024); break;
                 case 3: DRAW_LAUNCH(double, 8, 9, 512); break;
-                default:   // 4
-                    // few samples: more lanes each, and small workgroups to
-                    // reach every CU (R = 16, J = 4096: 43 -> 22 us; J = 16384:
-                    // 45 against 57 the other way)
-                    if (J < 8192) DRAW_LAUNCH(double, 32, 3, 256);
-                    else DRAW_LAUNCH(double, 8, 9, 1024);
+                default:   // 4: lanes a sample as long as one round holds J
+                    if (J <= 6144) DRAW_LAUNCH(double, 32, 3, 256);
+                    else if (J <= 12288) DRAW_LAUNCH(double, 16, 5, 256);
+                    else DRAW_BY_ROUNDS(double, 8, 9, deep ? 1.5 : 1.3);
                     break;
             }
         } else if (R <= 32) {
@@ -1480,18 +1503,18 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                 case 4: DRAW_LAUNCH(double, 16, 17, 512); break;
                 case 5: DRAW_LAUNCH(double, 64, 5, 256); break;
                 default:   // 6
-                    if (R <= 24) DRAW_LAUNCH(double, 32, 5, 256);
-                    else if (R <= 27) DRAW_LAUNCH(double, 32, 6, 256);
-                    else if (R <= 29) DRAW_LAUNCH(double, 32, 7, 256);
-                    else DRAW_LAUNCH(double, 32, 9, 256);
+                    if (R <= 24) DRAW_BY_ROUNDS(double, 32, 5, 1.3);
+                    else if (R <= 27) DRAW_BY_ROUNDS(double, 32, 6, deep ? 1.5 : 1.3);
+                    else if (R <= 29) DRAW_BY_ROUNDS(double, 32, 7, deep ? 1.5 : 1.3);
+                    else DRAW_BY_ROUNDS(double, 32, 9, deep ? 1.5 : 1.3);
                     break;
             }
         } else if (R <= 35) {
-            DRAW_LAUNCH(double, 64, 5, 256);
+            DRAW_BY_ROUNDS(double, 64, 5, deep ? 1.5 : 1.3);
         } else if (R <= 41) {
-            DRAW_LAUNCH(double, 64, 7, 256);
+            DRAW_BY_ROUNDS(double, 64, 7, deep ? 1.5 : 1.3);
         } else if (R <= 45) {
-            DRAW_LAUNCH(double, 64, 9, 256);
+            DRAW_BY_ROUNDS(double, 64, 9, deep ? 1.5 : 1.3);
         } else if (R <= 54) {
             DRAW_LAUNCH(double, 64, 12, 256);
         } else {
@@ -1503,10 +1526,7 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                 case 1: DRAW_LAUNCH(float, 8, 5, 1024); break;
                 case 2: DRAW_LAUNCH(float, 32, 2, 1024); break;
                 case 3: DRAW_LAUNCH(float, 8, 5, 512); break;
-                case 4:
-                    if (J < 8192) DRAW_LAUNCH(float, 8, 5, 256);
-                    else DRAW_LAUNCH(float, 8, 5, 1024);
-                    break;
+                case 4: DRAW_BY_ROUNDS(float, 8, 5, 1.5); break;
                 default: DRAW_LAUNCH(float, 16, 3, 1024); break;
             }
         } else if (R <= 32) {
@@ -1520,9 +1540,7 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                 default: DRAW_LAUNCH(float, 8, 17, 1024); break;
             }
         } else if (R <= 45) {
-            // (256 threads against 1024, R = 40, J = 65536: 514 against 678 us at
-            // 3e5 rows, 337 against 333 at 300)
-            DRAW_LAUNCH(float, 32, 9, 256);
+            DRAW_BY_ROUNDS(float, 32, 9, levels >= 11 ? 2.0 : 1.6);
         } else {
             switch (tune_value(kTuneDrawF32R64)) {
                 case 1: DRAW_LAUNCH(float, 32, 17, 1024); break;
@@ -1532,9 +1550,10 @@ void sts_draw(hipStream_t s, int N, int j, int R, int64_t J, const StsModeArgs* 
                     // deep trees read most levels from L2 and beyond, where three
                     // small workgroups per CU wait less than a large one; shallow
                     // ones live on the levels that a large one stages (R = 64,
-                    // J = 65536: 975 against 1186 us at 3e5 rows, 622 against 529
-                    // at 300; J = 4096: 144 against 215)
-                    if (deep || J < 8192) DRAW_LAUNCH(float, 32, 17, 256);
+                    // J = 65536: 763 against 981 us at 3e5 rows, 528 against 422
+                    // at 300), but for one round of small ones (J = 4000: 40
+                    // against 67)
+                    if (deep || J <= 6144) DRAW_LAUNCH(float, 32, 17, 256);
                     else DRAW_LAUNCH(float, 32, 17, 1024);
                     break;
                 default: DRAW_LAUNCH(float, 64, 9, 1024); break;
