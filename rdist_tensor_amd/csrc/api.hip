@@ -15,6 +15,7 @@
 #include <limits>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -1001,7 +1002,7 @@ double als_fit_impl(ex_als* a) {
     ex_tensor* t = a->t;
     hipStream_t st = a->ctx->c.stream;
     const int N = f->N, R = f->R;
-    a->scal.ensure(64);
+    a->scal.ensure((size_t)(2 + kMaxRank) * 8);
     a->fit_grams.ensure((size_t)N * R * R * 8);
     f->sync64_all();
     for (int k2 = 0; k2 < N; k2++)
@@ -1011,16 +1012,17 @@ double als_fit_impl(ex_als* a) {
     // in the row order of mode 0 the last mode's rows are the scattered ones,
     // in the last mode's order the one before it: the smaller factor of the two
     const int by = t->dims[N - 1] <= t->dims[N - 2] ? 0 : N - 1;
-    k::fit_dot(st, t->lk[by], f->ptrs, t->dims, f->sigma.as<double>(), R, d + 1, a->fit_part);
-    double h[3];
-    d2h(st, h, d, sizeof(h));
+    k::fit_dot(st, t->lk[by], t->coords.as<uint32_t>(), t->vals.as<double>(), f->ptrs, t->dims, f->sigma.as<double>(),
+               R, d + 1, a->fit_part);
+    double h[2 + kMaxRank];
+    d2h(st, h, d, (size_t)(2 + R) * 8);
     // Where the model reproduces X, res2 is rounding noise of either sign, and a
     // negative one counts as zero.  The terms of each of the three sums have
     // absolute sums of at most (|X| + S)^2, S = sum_r |sigma_r| prod_k |u_kr|, and no
     // sum adds more than `chain` values one after another; a res2 below that noise
     // comes from sums that do not belong together (coordinates that X repeats) and
     // the fit is NaN.
-    const double res2 = t->norm2 + h[0] - 2.0 * h[1], size = t->norm + h[2];
+    const double res2 = t->norm2 + h[0] - 2.0 * h[1], size = std::accumulate(h + 2, h + 2 + R, t->norm);
     const double chain = 4096.0 + (double)(t->nnz + *std::max_element(t->dims, t->dims + N)) / 1024.0;
     const bool noise = res2 < 0.0 && -res2 <= chain * std::numeric_limits<double>::epsilon() * size * size;
     return 1.0 - std::sqrt(noise ? 0.0 : res2) / t->norm;

@@ -187,7 +187,7 @@ void dsymm(hipStream_t s, const double* G, const double* Y, int64_t m, int R, do
 // sigma_c = the column norms of U, U /= sigma
 void normalize_cols(hipStream_t s, double* U, int64_t m, int R, double* sigma, DevBuf& part);
 void cos_init(hipStream_t s, double* U, int64_t m, int R);
-// *out = |Xh|^2, *size = sum_r |sigma_r| prod_k |u_kr|
+// *out = |Xh|^2, size[r] = |sigma_r| prod_k |u_kr|
 void chain_had_norm(hipStream_t s, const double* grams, int N, int R, const double* sigma, double* out, double* size);
 // out = elementwise product of grams[k] (k != exclude), k ascending
 void chain_had(hipStream_t s, const double* grams, int N, int exclude, int R, double* out);
@@ -312,9 +312,10 @@ void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uin
 // out[0..n) = NaN unless *count == want: a device-side argument check whose
 // failure the caller sees in the output, with nothing waited for.
 void poison_unless(hipStream_t s, const uint64_t* count, int64_t want, double* out, int64_t n);
-// *out = <X, Xh> over the lookup's nonzeros (FP64 factors).
-void fit_dot(hipStream_t s, const ModeLookup& L, const double* const* U, const int64_t* dims, const double* sigma,
-             int R, double* out, DevBuf& part);
+// *out = <X, Xh> (FP64 factors) over the nonzeros: of the lookup, or (coords, vals)
+// in input order.
+void fit_dot(hipStream_t s, const ModeLookup& L, const uint32_t* coords, const double* vals, const double* const* U,
+             const int64_t* dims, const double* sigma, int R, double* out, DevBuf& part);
 // final stages shared with the mixed-precision kernels
 void gram_final_launch(hipStream_t s, const double* part, int nb, int R, double* G);
 void col_sumsq_final_launch(hipStream_t s, const double* part, int nb, int R, double* sigma);

@@ -542,13 +542,8 @@ __global__ __launch_bounds__(kThreads) void chain_had_norm_kernel(const double* 
                                                                   const double* __restrict__ sigma,
                                                                   double* __restrict__ out,
                                                                   double* __restrict__ size) {
-    __shared__ double red[kThreads], part[kMaxRank];
+    __shared__ double red[kThreads];
     const int R2 = R * R;
-    if (threadIdx.x < R) {
-        double p = fabs(sigma[threadIdx.x]);
-        for (int k = 0; k < N; k++) p *= sqrt(grams[(int64_t)k * R2 + threadIdx.x * (R + 1)]);
-        part[threadIdx.x] = p;
-    }
     double acc = 0.0;
     for (int o = threadIdx.x; o < R2; o += blockDim.x) {
         double p = 1.0;
@@ -561,9 +556,12 @@ __global__ __launch_bounds__(kThreads) void chain_had_norm_kernel(const double* 
         double s = 0.0;
         for (int t = 0; t < kThreads; t++) s += red[t];
         *out = s;
-        double z = 0.0;
-        for (int r = 0; r < R; r++) z += part[r];
-        *size = z;
+    }
+    if (threadIdx.x >= 64 && threadIdx.x < 64 + R) {   // (beside the sum, on another wavefront)
+        const int r = threadIdx.x - 64;
+        double p = fabs(sigma[r]);
+        for (int k = 0; k < N; k++) p *= sqrt(grams[(int64_t)k * R2 + r * (R + 1)]);
+        size[r] = p;
     }
 }
 

@@ -2005,6 +2005,36 @@ __global__ __launch_bounds__(kThreads) void fit_kernel(const uint32_t* __restric
     }
 }
 
+// The same for R <= 2, a thread per nonzero in input order: a row is one load, and
+// the row order's fiber keys (a gather more for each nonzero) are what the pass
+// above waits for.  1.5e6 nonzeros, three modes of 5e4-5e5 rows, R = 1 42 us by the
+// pass above, 2 48; at R = 3 it is the faster one (54 against 62).
+__global__ __launch_bounds__(kThreads) void fit_input_order(const uint32_t* __restrict__ coords,
+                                                            const double* __restrict__ vals, int64_t nnz,
+                                                            const double* __restrict__ sigma, FitArgs a,
+                                                            double* __restrict__ part) {
+    __shared__ double red[kThreads / 64];
+    double acc = 0.0;
+    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < nnz; i += (int64_t)gridDim.x * kThreads) {
+        const uint32_t* c = coords + i * a.N;
+        double v = 0.0;
+        for (int r = 0; r < a.R; r++) {
+            double p = sigma[r];
+            for (int k = 0; k < a.N; k++) p *= a.U[k][(int64_t)c[k] * a.R + r];
+            v += p;
+        }
+        acc += vals[i] * v;
+    }
+    const double t = wave_sum(acc);
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int q = 0; q < kThreads / 64; q++) s += red[q];
+        part[blockIdx.x] = s;
+    }
+}
+
 __global__ void fit_final(const double* __restrict__ part, int n, double* __restrict__ out) {
     const int lane = threadIdx.x;
     double s = 0.0;
@@ -2854,8 +2884,8 @@ void zero_bytes(hipStream_t s, void* p, size_t bytes) {
     EX_HIP(hipGetLastError());
 }
 
-void fit_dot(hipStream_t s, const ModeLookup& L, const double* const* U, const int64_t* dims, const double* sigma,
-             int R, double* out, DevBuf& part) {
+void fit_dot(hipStream_t s, const ModeLookup& L, const uint32_t* coords, const double* vals, const double* const* U,
+             const int64_t* dims, const double* sigma, int R, double* out, DevBuf& part) {
     FitArgs a;
     a.N = L.kl.N;
     a.mode = L.mode;
@@ -2871,11 +2901,16 @@ void fit_dot(hipStream_t s, const ModeLookup& L, const double* const* U, const i
     // eight wavefronts per SIMD)
     const int nb = (int)grid_for((L.nnz + kFitChunk - 1) / kFitChunk, kThreads / 64, 8 * num_cus(s));
     part.ensure((size_t)nb * sizeof(double));
-    with_group(group_lanes<double>(R), [&](auto gc) {
-        hipLaunchKernelGGL(fit_kernel<decltype(gc)::value>, dim3(nb), dim3(kThreads), 0, s, L.rrow.as<uint32_t>(),
-                           L.rfib.as<uint32_t>(), L.rval.as<double>(), L.fkey.as<uint64_t>(), L.nnz, sigma, a,
+    if (R <= 2) {
+        hipLaunchKernelGGL(fit_input_order, dim3(nb), dim3(kThreads), 0, s, coords, vals, L.nnz, sigma, a,
                            part.as<double>());
-    });
+    } else {
+        with_group(group_lanes<double>(R), [&](auto gc) {
+            hipLaunchKernelGGL(fit_kernel<decltype(gc)::value>, dim3(nb), dim3(kThreads), 0, s, L.rrow.as<uint32_t>(),
+                               L.rfib.as<uint32_t>(), L.rval.as<double>(), L.fkey.as<uint64_t>(), L.nnz, sigma, a,
+                               part.as<double>());
+        });
+    }
     hipLaunchKernelGGL(fit_final, dim3(1), dim3(64), 0, s, part.as<double>(), nb, out);
     EX_HIP(hipGetLastError());
 }
