@@ -58,8 +58,10 @@ struct Lds {
 // Draws (cp_arls_lev.hpp:36-163 with the row CDFs of the other modes):
 // sample s takes row lower_bound(cdf_k, u) of every mode k != j, u from the
 // generator at (sweep, j, k); weight = prod_k (sum_k / score_k) / J.
-// Thread t holds samples [t Q, t Q + Q).
-__device__ void draw_phase(const BatchTensor& T, int j, int64_t J, uint64_t sweep) {
+// Thread t holds samples [t Q, t Q + Q).  Not inlined: the sweep kernel has
+// no registers to spare for it (spilled words a lane 60 -> 154; 256 tensors of R = 16, J =
+// 8192 740 -> 935 us a sweep).
+__device__ __attribute__((noinline)) void draw_phase(const BatchTensor& T, int j, int64_t J, uint64_t sweep) {
     const int N = T.N;
     const int Q = (int)((J + kBT - 1) / kBT);
     const int64_t s0 = (int64_t)threadIdx.x * Q;
