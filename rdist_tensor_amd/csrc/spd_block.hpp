@@ -159,7 +159,7 @@ __device__ int spd_inverse_regs(SpdShared& sh, const SpdLayout& L, double (&a)[R
         const bool skip = !(piv > tol);
         dropped += skip ? 1 : 0;
         const double inv = skip ? 0.0 : 1.0 / piv;
-        if (!L.on) continue;
+        if (!L.on || L.row(0) >= R) continue;   // (most wavefronts at small orders)
         const int j = L.j;
         if (skip) {   // the same for the whole workgroup
 #pragma unroll
