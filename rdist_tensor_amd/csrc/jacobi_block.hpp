@@ -1,7 +1,6 @@
 // Cyclic Jacobi eigensolver and the Jacobi pseudo-inverse of an R x R
-// symmetric matrix on one workgroup (kJacobiThreads threads do the work; a
-// larger workgroup's other threads only take part in the barriers), shared by
-// the dense kernels and the batched sweep.
+// symmetric matrix on one workgroup of kJacobiThreads threads, shared by the dense
+// kernels and the FP64 batched sweep.
 #pragma once
 #include "common.hpp"
 
@@ -101,9 +100,8 @@ __device__ __forceinline__ double rot_row(bool rot, double c, double s, int i, d
 // one chosen, so that the wavefront does not diverge.  Up to order 32 the
 // wavefronts that have no blocks rotate V, the last one also the pairs' own
 // elements; above, every wavefront does both.  The convergence flag of each
-// sweep is published by thread 0 in LDS; threads past kJacobiThreads only meet
-// the barriers.  Afterwards A holds the result and sh.rank[v] is the ascending
-// position of A[v][v] (ties by index).
+// sweep is published by thread 0 in LDS.  Afterwards A holds the result and
+// sh.rank[v] is the ascending position of A[v][v] (ties by index).
 // By index, with packed-triangle indices computed in each round and every
 // wavefront doing blocks and rows: 146 / 344 / 2358 us for an eigendecomposition
 // of order 16 / 32 / 64 (a random Gram with a repeated column); so: 102 / 234 / 971.
@@ -116,12 +114,11 @@ __device__ __forceinline__ void jacobi_block(double* A, double* A2, double* V, i
     constexpr int NBL = kSplit ? 1 : 2;          // 496 blocks at most
     constexpr int NV = kSplit ? 4 : 8;           // rows of V a lane slot rotates
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-    const bool act = tid < kJacobiThreads;       // wavefront-uniform
     const int n = R, ne = n + (n & 1), npair = ne / 2, m = ne - 1;
     const int noff = npair * (npair - 1) / 2, diag = 4 * noff;
     const int bwaves = kSplit ? (noff + 63) / 64 : kWaves;
-    const bool has_blocks = act && wave < bwaves;
-    const bool has_diag = act && wave == kWaves - 1 && lane < npair;
+    const bool has_blocks = wave < bwaves;
+    const bool has_diag = wave == kWaves - 1 && lane < npair;
     // blocks: positions (P, ne-1-P) x (Q, ne-1-Q), and where each element goes
     int bP[NBL], bQ[NBL], bi[NBL], to[NBL][4];
 #pragma unroll
@@ -145,10 +142,10 @@ __device__ __forceinline__ void jacobi_block(double* A, double* A2, double* V, i
     // rows of V: lane slots of npair lanes on the wavefronts that rotate V
     const int vslots = 64 / npair, vwaves = kSplit ? kWaves - bwaves : kWaves, vwave = kSplit ? wave - bwaves : wave;
     const int vstride = vwaves * vslots;
-    const bool has_v = act && vwave >= 0;
+    const bool has_v = vwave >= 0;
     const int vrow = has_v && lane < vslots * npair ? vwave * vslots + lane / npair : n;
     // into the layout of round 0, where the index at a position is the position
-    for (int e = tid; act && e < ne * ne; e += kJacobiThreads) {
+    for (int e = tid; e < ne * ne; e += kJacobiThreads) {
         const int a = e / ne, b = e - a * ne;
         if (a <= b) A2[rr_place(npair, a, b)] = b < n ? A[tri_index(R, a, b)] : 0.0;
         if (a < n) V[e] = a == b ? 1.0 : 0.0;
@@ -159,81 +156,79 @@ __device__ __forceinline__ void jacobi_block(double* A, double* A2, double* V, i
     bool any = false;
     int sweep = 0, round = 0;
     for (;;) {
-        if (act) {
-            // every read of the round first
-            const double aff = cur[diag + pair], afg = cur[diag + npair + pair], agg = cur[diag + 2 * npair + pair];
-            double x[NBL][2][2];
+        // every read of the round first
+        const double aff = cur[diag + pair], afg = cur[diag + npair + pair], agg = cur[diag + 2 * npair + pair];
+        double x[NBL][2][2];
 #pragma unroll
-            for (int b = 0; b < NBL; b++)
+        for (int b = 0; b < NBL; b++)
 #pragma unroll
-                for (int u = 0; u < 4; u++) x[b][u >> 1][u & 1] = has_blocks ? cur[u * noff + (bi[b] < 0 ? 0 : bi[b])] : 0.0;
-            double vf[NV], vg[NV];
+            for (int u = 0; u < 4; u++) x[b][u >> 1][u & 1] = has_blocks ? cur[u * noff + (bi[b] < 0 ? 0 : bi[b])] : 0.0;
+        double vf[NV], vg[NV];
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+            const int kk = vrow + vstride * u < n ? vrow + vstride * u : 0;   // (row 0: not used)
+            vf[u] = has_v ? V[kk * ne + fpos] : 0.0;
+            vg[u] = has_v ? V[kk * ne + gpos] : 0.0;
+        }
+        const int fi = rr_index(m, round, fpos), gi = rr_index(m, round, gpos);
+        const JacobiRot mine = jacobi_rot(aff, agg, afg, fi < n && gi < n, fi > gi);
+        const bool rot = mine.c > 0.0;
+        const bool rotates = __ballot(rot) != 0;   // the same on every wavefront
+        any |= rotates;
+        if (has_blocks) {
+#pragma unroll
+            for (int b = 0; b < NBL; b++) {
+                double off[2][2];
+#pragma unroll
+                for (int u = 0; u < 4; u++) off[u >> 1][u & 1] = x[b][u >> 1][u & 1];
+                if (rotates) {
+                    const int P = bP[b], Q = bQ[b];
+                    const double cP = __shfl(mine.c, P, 64), sP = __shfl(mine.s, P, 64);
+                    const double cQ = __shfl(mine.c, Q, 64), sQ = __shfl(mine.s, Q, 64);
+                    const bool rP = cP > 0.0, rQ = cQ > 0.0;
+                    // fa: rows by P's rotation, then columns by Q's (P's index
+                    // the smaller); fb: rows by Q's, then columns by P's
+                    double ra_[2][2], fa[2][2], rb_[2][2], fb[2][2];
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                        ra_[0][k] = rot_row(rP, cP, sP, 0, x[b][0][k], x[b][1][k]);
+                        ra_[1][k] = rot_row(rP, cP, sP, 1, x[b][0][k], x[b][1][k]);
+                        rb_[0][k] = rot_row(rQ, cQ, sQ, 0, x[b][k][0], x[b][k][1]);
+                        rb_[1][k] = rot_row(rQ, cQ, sQ, 1, x[b][k][0], x[b][k][1]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        fa[i][0] = rot_row(rQ, cQ, sQ, 0, ra_[i][0], ra_[i][1]);
+                        fa[i][1] = rot_row(rQ, cQ, sQ, 1, ra_[i][0], ra_[i][1]);
+                        fb[i][0] = rot_row(rP, cP, sP, 0, rb_[i][0], rb_[i][1]);
+                        fb[i][1] = rot_row(rP, cP, sP, 1, rb_[i][0], rb_[i][1]);
+                    }
+                    const int ri[2] = {rr_index(m, round, P), rr_index(m, round, m - P)};
+                    const int ci[2] = {rr_index(m, round, Q), rr_index(m, round, m - Q)};
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const int i = u >> 1, k = u & 1;
+                        off[i][k] = ri[i] < ci[k] ? fa[i][k] : fb[k][i];
+                    }
+                }
+                if (bi[b] >= 0)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) nxt[to[b][u]] = off[u >> 1][u & 1];
+            }
+        }
+        if (has_diag) {   // the exact 2x2 result
+            nxt[toff] = rot ? aff - mine.t * afg : aff;
+            nxt[togg] = rot ? agg + mine.t * afg : agg;
+            nxt[tofg] = rot ? 0.0 : afg;
+        }
+        if (has_v) {
+            // a row's lanes are in one wavefront: every read of it is above
 #pragma unroll
             for (int u = 0; u < NV; u++) {
-                const int kk = vrow + vstride * u < n ? vrow + vstride * u : 0;   // (row 0: not used)
-                vf[u] = has_v ? V[kk * ne + fpos] : 0.0;
-                vg[u] = has_v ? V[kk * ne + gpos] : 0.0;
-            }
-            const int fi = rr_index(m, round, fpos), gi = rr_index(m, round, gpos);
-            const JacobiRot mine = jacobi_rot(aff, agg, afg, fi < n && gi < n, fi > gi);
-            const bool rot = mine.c > 0.0;
-            const bool rotates = __ballot(rot) != 0;   // the same on every wavefront
-            any |= rotates;
-            if (has_blocks) {
-#pragma unroll
-                for (int b = 0; b < NBL; b++) {
-                    double off[2][2];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) off[u >> 1][u & 1] = x[b][u >> 1][u & 1];
-                    if (rotates) {
-                        const int P = bP[b], Q = bQ[b];
-                        const double cP = __shfl(mine.c, P, 64), sP = __shfl(mine.s, P, 64);
-                        const double cQ = __shfl(mine.c, Q, 64), sQ = __shfl(mine.s, Q, 64);
-                        const bool rP = cP > 0.0, rQ = cQ > 0.0;
-                        // fa: rows by P's rotation, then columns by Q's (P's index
-                        // the smaller); fb: rows by Q's, then columns by P's
-                        double ra_[2][2], fa[2][2], rb_[2][2], fb[2][2];
-#pragma unroll
-                        for (int k = 0; k < 2; k++) {
-                            ra_[0][k] = rot_row(rP, cP, sP, 0, x[b][0][k], x[b][1][k]);
-                            ra_[1][k] = rot_row(rP, cP, sP, 1, x[b][0][k], x[b][1][k]);
-                            rb_[0][k] = rot_row(rQ, cQ, sQ, 0, x[b][k][0], x[b][k][1]);
-                            rb_[1][k] = rot_row(rQ, cQ, sQ, 1, x[b][k][0], x[b][k][1]);
-                        }
-#pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            fa[i][0] = rot_row(rQ, cQ, sQ, 0, ra_[i][0], ra_[i][1]);
-                            fa[i][1] = rot_row(rQ, cQ, sQ, 1, ra_[i][0], ra_[i][1]);
-                            fb[i][0] = rot_row(rP, cP, sP, 0, rb_[i][0], rb_[i][1]);
-                            fb[i][1] = rot_row(rP, cP, sP, 1, rb_[i][0], rb_[i][1]);
-                        }
-                        const int ri[2] = {rr_index(m, round, P), rr_index(m, round, m - P)};
-                        const int ci[2] = {rr_index(m, round, Q), rr_index(m, round, m - Q)};
-#pragma unroll
-                        for (int u = 0; u < 4; u++) {
-                            const int i = u >> 1, k = u & 1;
-                            off[i][k] = ri[i] < ci[k] ? fa[i][k] : fb[k][i];
-                        }
-                    }
-                    if (bi[b] >= 0)
-#pragma unroll
-                        for (int u = 0; u < 4; u++) nxt[to[b][u]] = off[u >> 1][u & 1];
-                }
-            }
-            if (has_diag) {   // the exact 2x2 result
-                nxt[toff] = rot ? aff - mine.t * afg : aff;
-                nxt[togg] = rot ? agg + mine.t * afg : agg;
-                nxt[tofg] = rot ? 0.0 : afg;
-            }
-            if (has_v) {
-                // a row's lanes are in one wavefront: every read of it is above
-#pragma unroll
-                for (int u = 0; u < NV; u++) {
-                    const int kk = vrow + vstride * u;
-                    if (kk < n) {
-                        V[kk * ne + fnext] = rot ? mine.c * vf[u] - mine.s * vg[u] : vf[u];
-                        V[kk * ne + gnext] = rot ? mine.s * vf[u] + mine.c * vg[u] : vg[u];
-                    }
+                const int kk = vrow + vstride * u;
+                if (kk < n) {
+                    V[kk * ne + fnext] = rot ? mine.c * vf[u] - mine.s * vg[u] : vf[u];
+                    V[kk * ne + gnext] = rot ? mine.s * vf[u] + mine.c * vg[u] : vg[u];
                 }
             }
         }
@@ -257,7 +252,7 @@ __device__ __forceinline__ void jacobi_block(double* A, double* A2, double* V, i
 #pragma unroll
     for (int q = 0; q < kHold; q++) {
         const int e = tid + q * kJacobiThreads;
-        if (!act || e >= n * n) continue;
+        if (e >= n * n) continue;
         const int a = e / n, b = e - a * n;
         ha[q] = cur[rr_place(npair, a, b)];
         hv[q] = V[a * ne + b];
@@ -266,7 +261,7 @@ __device__ __forceinline__ void jacobi_block(double* A, double* A2, double* V, i
 #pragma unroll
     for (int q = 0; q < kHold; q++) {
         const int e = tid + q * kJacobiThreads;
-        if (!act || e >= n * n) continue;
+        if (e >= n * n) continue;
         const int a = e / n, b = e - a * n;
         if (a <= b) A[tri_index(R, a, b)] = ha[q];
         V[e] = hv[q];

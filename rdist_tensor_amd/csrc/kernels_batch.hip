@@ -48,7 +48,7 @@ struct Lds {
     unsigned char* big;
     double* G;      // R x R: design Gram, then the sampler's Gram
     double* Gi;     // R x R: pseudo-inverses
-    double* M;      // R x R: Gi diag(1 / sigma), rounded to V
+    double* M;      // R x R: Gi diag(1 / sigma), rounded to FP32
     double* sig;    // R
     uint32_t* wsu;  // kWaves
     double* wsd;    // kWaves
@@ -185,24 +185,23 @@ __device__ uint32_t dedup_phase(const BatchTensor& T, int j, int64_t J, const Ld
 }
 
 // KRP gather (accumulator_stationary.hpp:210-249): dg = prod_{k != j}
-// U_k[s_k] sqrt(w), dm = dg sqrt(w), in V arithmetic.  A thread takes kLane
+// U_k[s_k] sqrt(w), dm = dg sqrt(w), in FP32.  A thread takes kLane
 // rows at a time so that their index loads, then their factor-row loads,
 // are in flight together.
-template <typename V>
 __device__ void design_phase(const BatchTensor& T, int j, uint32_t Ju) {
     const int N = T.N, R = T.R;
     const int rows = kBT / R, rl = threadIdx.x / R, r = threadIdx.x - rl * R;
-    V* dg = static_cast<V*>(T.dg);
-    V* dm = static_cast<V*>(T.dm);
+    float* dg = static_cast<float*>(T.dg);
+    float* dm = static_cast<float*>(T.dm);
     if (rl < rows)
         for (uint32_t c0 = rl; c0 < Ju; c0 += (uint32_t)rows * kLane) {
-            V d[kLane];
+            float d[kLane];
             uint32_t idx[kLane];
 #pragma unroll
-            for (int b = 0; b < kLane; b++) d[b] = (V)1;
+            for (int b = 0; b < kLane; b++) d[b] = 1.0f;
             for (int k = 0; k < N; k++) {
                 if (k == j) continue;
-                const V* U = static_cast<const V*>(T.m[k].U);
+                const float* U = static_cast<const float*>(T.m[k].U);
 #pragma unroll
                 for (int b = 0; b < kLane; b++) {
                     const uint32_t c = c0 + (uint32_t)b * rows;
@@ -215,8 +214,8 @@ __device__ void design_phase(const BatchTensor& T, int j, uint32_t Ju) {
             for (int b = 0; b < kLane; b++) {
                 const uint32_t c = c0 + (uint32_t)b * rows;
                 if (c >= Ju) continue;
-                const V sw = (V)sqrt(T.wd[c]);
-                const V v = d[b] * sw;
+                const float sw = (float)sqrt(T.wd[c]);
+                const float v = d[b] * sw;
                 dg[(int64_t)c * R + r] = v;
                 dm[(int64_t)c * R + r] = v * sw;
             }
@@ -233,8 +232,7 @@ __device__ void design_phase(const BatchTensor& T, int j, uint32_t Ju) {
 // last chunk is done, are added in group order.  Entries (a, b) and (b, a)
 // are the same products summed in the same order, so G is exactly symmetric.
 // The solver's scratch overlaps the staging area: it is dead once G is formed.
-template <typename V>
-__device__ void block_gram(const V* __restrict__ A, const uint32_t* __restrict__ idx, uint32_t rows, int R,
+__device__ void block_gram(const float* __restrict__ A, const uint32_t* __restrict__ idx, uint32_t rows, int R,
                            double* G, const Lds& s) {
     double* stage = reinterpret_cast<double*>(s.big + kOffStage);
     const int H = (R + 1) / 2, HH = H * H, groups = kBT / HH;
@@ -334,14 +332,13 @@ __device__ uint64_t hits_phase(const BatchTensor& T, int j, uint32_t Ju, uint32_
 }
 
 // Clears factor j's previously listed rows.
-template <typename V>
 __device__ void clear_rows_phase(const BatchTensor& T, int j) {
     const int R = T.R;
     const int rows = kBT / R, rl = threadIdx.x / R, r = threadIdx.x - rl * R;
     const uint32_t L = T.cnt[j];
-    V* U = static_cast<V*>(T.m[j].U);
+    float* U = static_cast<float*>(T.m[j].U);
     if (rl < rows)
-        for (uint32_t q = rl; q < L; q += rows) U[(int64_t)T.m[j].list[q] * R + r] = (V)0;
+        for (uint32_t q = rl; q < L; q += rows) U[(int64_t)T.m[j].list[q] * R + r] = 0.0f;
     __syncthreads();
 }
 
@@ -382,16 +379,15 @@ __device__ __forceinline__ int row_lanes(int R) {
 // = sum over its stamped positions, in row order, of x * dm[design row].  The
 // row's lanes test G positions at a time (one coalesced load of stamps); the
 // hits among them, found by a ballot, are added in ascending position.
-template <typename V>
 __device__ void y_phase(const BatchTensor& T, int j, uint32_t L, uint32_t stamp) {
     const int R = T.R, G = row_lanes(R);
     const int rows = kBT / G, rl = threadIdx.x / G, r = threadIdx.x - rl * G;
     const int gbase = (threadIdx.x & 63) - r;
     const uint64_t gmask = G >= 64 ? ~0ull : ((1ull << G) - 1ull);
     const BatchMode& M = T.m[j];
-    const V* val = static_cast<const V*>(M.rval);
-    const V* dm = static_cast<const V*>(T.dm);
-    V* Y = static_cast<V*>(T.Yc);
+    const float* val = static_cast<const float*>(M.rval);
+    const float* dm = static_cast<const float*>(T.dm);
+    float* Y = static_cast<float*>(T.Yc);
     for (uint32_t q0 = 0; q0 < L; q0 += rows) {
         const uint32_t q = q0 + rl;
         uint32_t p0 = 0, p1 = 0;
@@ -400,7 +396,7 @@ __device__ void y_phase(const BatchTensor& T, int j, uint32_t L, uint32_t stamp)
             p0 = M.rowptr[row];
             p1 = M.rowptr[row + 1];
         }
-        V acc = (V)0;
+        float acc = 0.0f;
         for (uint32_t p = p0; p < p1; p += G) {
             const uint32_t pp = p + r;
             const bool hit = pp < p1 && T.hstamp[pp] == stamp;
@@ -410,7 +406,7 @@ __device__ void y_phase(const BatchTensor& T, int j, uint32_t L, uint32_t stamp)
                 m &= m - 1;
                 const uint32_t ph = p + (uint32_t)b;
                 const uint32_t u = T.hu[ph];
-                const V x = val[ph];
+                const float x = val[ph];
                 if (r < R) acc += x * dm[(int64_t)u * R + r];
             }
         }
@@ -420,11 +416,10 @@ __device__ void y_phase(const BatchTensor& T, int j, uint32_t L, uint32_t stamp)
 }
 
 // Factor update on the mixed path (accumulator_stationary.hpp:280-289):
-// sigma_c = sqrt((Gi Y^T Y Gi)_cc), M = Gi diag(1 / sigma) rounded to V,
+// sigma_c = sqrt((Gi Y^T Y Gi)_cc), M = Gi diag(1 / sigma) rounded to FP32,
 // U_j rows = Y M on the listed rows (one pass over Y); then the sampler's
 // Gram U_j^T U_j = M^T (Y^T Y) M into s.G (upper triangle computed,
 // mirrored).
-template <typename V>
 __device__ void update_phase(const BatchTensor& T, int j, uint32_t L, const Lds& s) {
     const int R = T.R, R2 = R * R;
     const double* GY = reinterpret_cast<const double*>(s.big + kOffGY);
@@ -446,16 +441,16 @@ __device__ void update_phase(const BatchTensor& T, int j, uint32_t L, const Lds&
         s.sig[c] = sg;
     }
     __syncthreads();
-    for (int o = threadIdx.x; o < R2; o += kBT) s.M[o] = (double)(V)(gi[o] / s.sig[o % R]);
+    for (int o = threadIdx.x; o < R2; o += kBT) s.M[o] = (double)(float)(gi[o] / s.sig[o % R]);
     __syncthreads();
     // U_j rows, and tmp = (Y^T Y) M
     const int rows = kBT / R, rl = threadIdx.x / R, r = threadIdx.x - rl * R;
-    const V* Y = static_cast<const V*>(T.Yc);
-    V* U = static_cast<V*>(T.m[j].U);
+    const float* Y = static_cast<const float*>(T.Yc);
+    float* U = static_cast<float*>(T.m[j].U);
     if (rl < rows)
         for (uint32_t q = rl; q < L; q += rows) {
-            V acc = (V)0;
-            for (int b = 0; b < R; b++) acc += Y[(int64_t)q * R + b] * (V)s.M[b * R + r];
+            float acc = 0.0f;
+            for (int b = 0; b < R; b++) acc += Y[(int64_t)q * R + b] * (float)s.M[b * R + r];
             U[(int64_t)T.m[j].list[q] * R + r] = acc;
         }
     for (int o = threadIdx.x; o < R2; o += kBT) {
@@ -477,17 +472,16 @@ __device__ void update_phase(const BatchTensor& T, int j, uint32_t L, const Lds&
 }
 
 // Sampler update (cp_arls_lev.hpp:25-34): Gp = pinv(U_j^T U_j) (in s.Gi),
-// score of each listed row u^T Gp u (FP64 from V rows; the row's lanes hold
+// score of each listed row u^T Gp u (FP64 from FP32 rows; the row's lanes hold
 // one entry each, t_c = sum_b u_b Gp[b][c] over broadcasts, then a butterfly
 // sum of u_c t_c), their sum and the CDF of score / sum over the listed rows
 // in ascending order (last entry 1).
-template <typename V>
 __device__ void scores_phase(const BatchTensor& T, int j, uint32_t L, const Lds& s) {
     const int R = T.R, G = row_lanes(R);
     const int rows = kBT / G, rl = threadIdx.x / G, r = threadIdx.x - rl * G;
     const int gbase = (threadIdx.x & 63) - r;
     const BatchMode& M = T.m[j];
-    const V* U = static_cast<const V*>(M.U);
+    const float* U = static_cast<const float*>(M.U);
     const double* g = s.Gi;
     const int rc = r < R ? r : 0;
     for (uint32_t q0 = 0; q0 < L; q0 += rows) {
@@ -529,22 +523,21 @@ __device__ void scores_phase(const BatchTensor& T, int j, uint32_t L, const Lds&
     __syncthreads();
 }
 
-template <typename V>
 __device__ void mode_step(const BatchTensor& T, int j, int64_t J, uint64_t sweep, uint32_t stamp, const Lds& s) {
     const int R = T.R;
     draw_phase(T, j, J, sweep);
     const uint32_t Ju = dedup_phase(T, j, J, s);
-    design_phase<V>(T, j, Ju);
-    block_gram<V>(static_cast<const V*>(T.dg), nullptr, Ju, R, s.G, s);
+    design_phase(T, j, Ju);
+    block_gram(static_cast<const float*>(T.dg), nullptr, Ju, R, s.G, s);
     block_spd_pinv(s.G, R, 1e-11, s.Gi, s);
     const uint64_t hits = hits_phase(T, j, Ju, stamp);
-    clear_rows_phase<V>(T, j);
+    clear_rows_phase(T, j);
     const uint32_t L = list_phase(T, j, stamp, s);
-    y_phase<V>(T, j, L, stamp);
-    block_gram<V>(static_cast<const V*>(T.Yc), nullptr, L, R, reinterpret_cast<double*>(s.big + kOffGY), s);
-    update_phase<V>(T, j, L, s);
+    y_phase(T, j, L, stamp);
+    block_gram(static_cast<const float*>(T.Yc), nullptr, L, R, reinterpret_cast<double*>(s.big + kOffGY), s);
+    update_phase(T, j, L, s);
     block_spd_pinv(s.G, R, 1e-11, s.Gi, s);
-    scores_phase<V>(T, j, L, s);
+    scores_phase(T, j, L, s);
     const double h = block_sum_f64((double)hits, s.wsd);
     if (threadIdx.x == 0) {
         atomicAdd(&T.stats[0], (unsigned long long)h);
@@ -553,7 +546,6 @@ __device__ void mode_step(const BatchTensor& T, int j, int64_t J, uint64_t sweep
     }
 }
 
-template <typename V>
 __global__ __launch_bounds__(kBT) void batch_sweep_kernel(const BatchTensor* __restrict__ ts, int n, int64_t J,
                                                           BatchCtl* ctl) {
     __shared__ __align__(16) unsigned char big[kBigBytes];
@@ -572,7 +564,7 @@ __global__ __launch_bounds__(kBT) void batch_sweep_kernel(const BatchTensor* __r
         if (t >= (uint32_t)n) break;
         const BatchTensor& T = ts[t];
         const int N = T.N;
-        for (int j = 0; j < N; j++) mode_step<V>(T, j, J, sweep, epoch * (uint32_t)N + (uint32_t)j + 1u, s);
+        for (int j = 0; j < N; j++) mode_step(T, j, J, sweep, epoch * (uint32_t)N + (uint32_t)j + 1u, s);
     }
     if (threadIdx.x == 0) {
         __threadfence();
@@ -618,7 +610,7 @@ void batch_init(hipStream_t s, const BatchTensor* ts, int n) {
 void batch_sweep32(hipStream_t s, const BatchTensor* ts, int n, int64_t J, BatchCtl* ctl, int grid) {
     EX_CHECK(J >= 1 && J <= kBatchMaxJ, 1, "batched sweep: J out of range");
     EX_CHECK(grid >= 1, 1, "batched sweep: empty grid");
-    hipLaunchKernelGGL(batch_sweep_kernel<float>, dim3((unsigned)grid), dim3(kBT), 0, s, ts, n, J, ctl);
+    hipLaunchKernelGGL(batch_sweep_kernel, dim3((unsigned)grid), dim3(kBT), 0, s, ts, n, J, ctl);
     EX_HIP(hipGetLastError());
 }
 
