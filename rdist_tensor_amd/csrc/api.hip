@@ -565,10 +565,10 @@ void sampler_draw_impl(ex_sampler* s, int64_t J, int j, uint64_t sweep, const do
             k::sts_first_cdf(st, m[k0], R, s->first_cdf.as<double>());
             first_cdf = s->first_cdf.as<double>();
         }
-        // FP64: its draws from tabulated masses where that is faster
+        // FP64: its draws from tabulated masses where that is faster and there is
+        // room for the tables (the same draws by descents)
         const k::StsFirstDraw* first_draw = nullptr;
-        if (!mixed && k::sts_first_pays(m[k0], R, J)) {
-            s->first_cdf.ensure(k::sts_first_bytes(m[k0], R, J));
+        if (!mixed && k::sts_first_pays(m[k0], R, J) && room_for(st, s->first_cdf, k::sts_first_bytes(m[k0], R, J))) {
             const k::StsFirstArgs fa{m[k0].g, m[k0].ge, j, k0, J, s->seed, sweep, s->sweep_dev, draws_row_dev,
                                      draws_eig_dev};
             first_draw = k::sts_first_draw(st, m[k0], R, fa, s->first_cdf.p);

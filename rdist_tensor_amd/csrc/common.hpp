@@ -77,6 +77,19 @@ struct DevBuf {
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Whether the stream may be given new memory: not while it is being captured.
+inline bool may_allocate(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
+// Whether b holds n bytes of scratch that a call on s can do without.
+inline bool room_for(hipStream_t s, DevBuf& b, size_t n) {
+    return n <= b.bytes || (may_allocate(s) && b.try_ensure(n));
+}
+
 // Packed upper triangle of an R x R symmetric matrix, row-major over the
 // upper triangle: (a, b), a <= b, at a*R - a*(a-1)/2 + (b - a).
 __host__ __device__ inline int tri_size(int R) { return R * (R + 1) / 2; }

@@ -2302,14 +2302,6 @@ bool key_order(hipStream_t s, ModeLookup& L, const V* vals) {
                            });
 }
 
-// Whether the stream may be given new memory: not while it is being captured.
-bool may_allocate(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
-    (void)hipGetLastError();
-    return false;
-}
-
 // ---------------------------------------------------------------- adjoint
 // dD[c] = sum over the nonzeros (row i, value x) of sample c's fiber of
 // x * G[i]: the transpose of the sampled MTTKRP.  The nonzeros are read in key
@@ -2557,7 +2549,7 @@ void smttkrp_adjoint(hipStream_t s, ModeLookup& L, const uint64_t* kd, const uin
         auto take = [&](size_t bytes) { size_t r = o; o = (o + bytes + 255) & ~(size_t)255; return r; };
         const size_t o_c = take(8), o_u = take((size_t)nu * 8), o_l = take((size_t)nc * 16),
                      o_p = take((size_t)nu * R * 8);
-        if (o <= work.bytes || (may_allocate(s) && work.try_ensure(o))) {
+        if (room_for(s, work, o)) {
             char* b = work.as<char>();
             units = AdjUnits{(unsigned int*)(b + o_c), (uint2*)(b + o_u), (uint4*)(b + o_l), (double*)(b + o_p)};
             hipLaunchKernelGGL(adj_clear, dim3(1), dim3(64), 0, s, units.count);
