@@ -24,7 +24,7 @@ ARCH = "gfx950"
 HIP_SOURCES = ["api.hip", "kernels_dense.hip", "kernels_sample.hip", "kernels_sparse.hip", "kernels_mixed.hip",
                "kernels_batch.hip", "kernels_batch64.hip", "sort.hip", "tensor_io.hip"]
 HEADERS = ["common.hpp", "device.hpp", "dsymm.hpp", "spd_block.hpp", "jacobi_block.hpp", "wave_psd.hpp",
-           "batch_block.hpp", "key_copies.hpp"]
+           "batch_block.hpp", "key_copies.hpp", "group_probe.hpp"]
 
 HIP_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

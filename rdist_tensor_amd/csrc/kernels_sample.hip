@@ -8,6 +8,7 @@
 // discrete_distribution (random.tcc:2655-2712).
 #include "common.hpp"
 #include "device.hpp"
+#include "group_probe.hpp"
 #include "wave_psd.hpp"
 
 namespace exafac {
@@ -501,18 +502,13 @@ __device__ __forceinline__ int leaf_pick(const double* q2, int F, double frac, i
 template <int G>
 __device__ __forceinline__ int64_t group_upper(const double* __restrict__ cum, int64_t n, double t, int l, int grp) {
     const uint64_t gmask = G == 64 ? ~0ull : ((1ull << G) - 1);
-    int64_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const int64_t step = (hi - lo + G - 1) / G;
-        int64_t idx = lo + (int64_t)(l + 1) * step - 1;
-        if (idx > hi - 1) idx = hi - 1;
-        const uint64_t bits = (__ballot(cum[idx] > t) >> (grp * G)) & gmask;
-        const int first = bits ? __ffsll((unsigned long long)bits) - 1 : G - 1;
-        const int64_t nhi = lo + (int64_t)(first + 1) * step;
-        lo += (int64_t)first * step;
-        hi = nhi < hi ? nhi : hi;
+    ProbeRange r{0, n};
+    while (r.hi - r.lo > 1) {
+        const int64_t step = probe_step(r, G);
+        const uint64_t bits = (__ballot(cum[probe_at(r, step, l)] > t) >> (grp * G)) & gmask;
+        r = probe_narrow(r, step, bits ? __ffsll((unsigned long long)bits) - 1 : -1);
     }
-    return lo;
+    return r.lo;
 }
 
 // x^T G x of node c of a tree whose first nst nodes are staged in LDS
