@@ -239,22 +239,25 @@ int ex_als_run(ex_als* a, int64_t rounds, int64_t J, int64_t epoch);
 int ex_als_run_batch(ex_als* const* als, int n, int64_t rounds, int64_t J, double* seconds);
 
 /* (no counterpart: the reference runs decompositions one after another)
- * Many CP-ARLS-LEV decompositions advanced by ONE kernel launch per sweep:
- * a workgroup of 1024 threads takes whole tensors from a queue and runs
+ * Many CP-ARLS-LEV decompositions advanced together.  EX_MIXED: ONE kernel launch
+ * per sweep, a workgroup of 1024 threads takes whole tensors from a queue.  EX_FP64:
+ * a chain of launches per mode step, each one phase of every tensor.  Both run
  * every mode step of AccumulatorStationary::execute_ALS_step
  * (accumulator_stationary.hpp:139-295) with the CP-ARLS-LEV sampler
- * (cp_arls_lev.hpp:25-163) as workgroup-level phases.  Each optimizer keeps
- * its own tensor, factors, sampler and seed; all share one device and one
- * precision, R <= 32 and 1 <= J <= 8192; no two share a LowRankTensor.
+ * (cp_arls_lev.hpp:25-163).  Each optimizer keeps its own tensor, factors,
+ * sampler and seed; all share one device and one precision, R <= 32 and
+ * 1 <= J <= 8192; no two share a LowRankTensor.
  * The batch keeps each mode's leverage scores over the rows where the factor
  * is nonzero (after a step, the rows a sampled fiber's nonzero reached) and
  * draws from the CDF over them: the row picked for a uniform draw is the one
  * the full-length CDF picks.  Arithmetic as the optimizers' precision
  * (EX_MIXED: FP32 factors, values, design and MTTKRP rows; FP64 Grams,
  * products and sums of FP32 rows, R x R pseudo-inverses -- pivoted Cholesky
- * when singular -- scores and CDFs; EX_FP64: all FP64).  The factor update
- * forms U_j = Y Gi diag(1/sigma) and the sampler's Gram as
- * M^T (Y^T Y) M, so results agree with ex_als_run's to rounding, not bitwise.
+ * when singular -- scores and CDFs; EX_FP64: all FP64).  The mixed factor update
+ * forms U_j = Y Gi diag(1/sigma) and the sampler's Gram as M^T (Y^T Y) M; the FP64
+ * one solves with the two-sided Jacobi where ex_als_run takes Gauss-Jordan if the
+ * Gram is well posed.  So results agree with ex_als_run's to rounding, not bitwise,
+ * and a sweep on factors of a few rows magnifies rounding without bound.
  * ex_batch_create rebuilds every optimizer's sampler state and copies it;
  * ex_batch_run runs `rounds` sweeps (draws keyed by sweeps 1..rounds, as
  * ex_als_run keys them), each one launch (EX_MIXED) or a chain of launches that

@@ -474,10 +474,10 @@ void tree_build_f32(hipStream_t s, const float* U, const TreeGeom& g, int R, flo
     level_sums(s, g, S, nodes);
 }
 
-// rows per thread: 256 / R row groups cover R rows
-// One element per thread of 1024 up to R = 32, two to four rows a thread above
-// (256 threads with sixteen rows each hid less of a pivot's latency: R = 64, inverse
-// 386 -> 154 us, the factorisations of computeM 346 -> 125 us).
+// Rows per thread: the 1024 / R row groups of a workgroup cover R rows, one element
+// a thread up to R = 32, two to four rows above (256 threads with sixteen rows each
+// hid less of a pivot's latency: R = 64, inverse 386 -> 154 us, the factorisations of
+// computeM 346 -> 125 us).
 #define SPD_DISPATCH(R, KERNEL, GRID, STREAM, ...)                                                     \
     do {                                                                                               \
         const int rpt = ((R) + 1024 / (R) - 1) / (1024 / (R));                                         \
