@@ -2224,11 +2224,12 @@ int64_t dedup_hash(hipStream_t s, const uint32_t* samples, const double* weights
     int tbits = 10;
     while (((int64_t)1 << tbits) < 2 * J) tbits++;
     const int64_t T = (int64_t)1 << tbits;
-    const void* before = table.p;
+    const size_t before = table.bytes;
     table.ensure((size_t)T * 16);
     // a new table starts empty (a fill kernel, not a memset: this runs beside
-    // graph captures); every call leaves the slots it used empty
-    if (table.p != before)
+    // graph captures); every call leaves the slots it used empty.  A larger table can
+    // come back at the address of the one freed for it, so its size tells
+    if (table.bytes != before)
         hipLaunchKernelGGL(zero_fill<uint32_t>, dim3(grid_for((int64_t)(table.bytes / 4), kThreads, 8192)),
                            dim3(kThreads), 0, s, table.as<uint32_t>(), (int64_t)(table.bytes / 4));
     unsigned long long* hkey = table.as<unsigned long long>();
